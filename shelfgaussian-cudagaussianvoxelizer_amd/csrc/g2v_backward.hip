@@ -1150,24 +1150,32 @@ __global__ void __launch_bounds__(kBtThreads, 1) k_bwd_tile(
 // ------------------------------------------------------------------------------------------
 // Phase A for short lists (1 .. smax <= kBsMax Gaussians).  k_bwd_tile holds one tile per CU (its LDS is
 // sized for 256-Gaussian passes), so a short list leaves that tile's chain of loads and barriers
-// bare; here a 4-wave workgroup with about 17 KB of LDS takes the tile and many run per CU.  The
-// per-pair results are those of k_bwd_tile up to float32 rounding: U = G F^T from float32 products
-// of gF and the split features' hi + lo (the matrix-core path leaves out lo x lo), t_v from U,
-// the same e (the same helper operations) and so the same split weights, and the moments summed
-// over the voxels in another order.  Which kernel takes a tile depends on its list length alone.
-// Thread = (voxel row lane, Gaussian slots wave + 4 i): the slots are dealt round robin over the waves.
+// bare; here a 4-wave workgroup with 17 KB of LDS takes the tile and many run per CU.
+//
+// U = G F^T on the float32 matrix cores (16x16x4), straight from the caller's rows: wave w owns the
+// 16 voxels x = x0 + w of the tile (A operand: lane l % 16 = voxel, B operand: lane l % 16 = list entry
+// 16 b + l % 16), and lane group q = l / 16 loads channels 16 s + 4 q .. + 3 of its row as one 16-byte
+// piece, whose four components feed four MFMAs (the order of the channels in the sum is free).  No
+// value goes through LDS and the loop over the channels has no barrier: what bounds such a tile is
+// the latency of its loads, so every load of a group of steps is issued before the first product of
+// the group before it.  The result lies with one list entry per lane column and the four voxels z
+// of (x0 + w, y0 + q) in the lane: t_v is a sum over 16 lanes, a pair's moments a sum over the four lane
+// groups and the four waves.  Products and sums are float32 of the caller's values (the matrix-core
+// path's split leaves about 2^-17 of each).  The weights come from k_bwd_tile's operations, so they
+// are the same bits.  Which kernel takes a tile depends on its list length alone.
+// Against 32-channel chunks of gF and the features staged in LDS and multiplied by the vector units: 6
+// scenes of 200 x 200 x 16 x 64 with 36,350 tiles of at most 8 entries 0.385 -> 0.274 ms (0.60 GB of gF,
+// 0.11 ms at the copy rate; the rest is the tiles' chain of loads), seven tiles at 768 channels beside
+// 9,993 long ones 0.145 -> 0.036 ms.
 // ------------------------------------------------------------------------------------------
 constexpr int kBsThreads = 256;
 constexpr int kBsMax = 64;     // longest list the kernel can take
-constexpr int kBsKc = 32;      // channels per staged chunk
+constexpr int kBsNb = kBsMax / 16;
 
 struct BsSmem {
-    float g[64][kBsKc + 1];    // gF chunk, voxel-major; rows padded so that lanes (voxels) hit distinct banks
-    float f[kBsKc][4][kBsMax / 4];   // feature chunk: [channel][wave][i] of slot wave + 4 i (a wave reads its slots at once)
     ParamTile<kBsMax> pt;
-    int vlin[64];
-    float gD[64], inv[64], D[64], tv[64];
-    float tpart[kBsThreads / 64][64];
+    int pidx[kBsMax];                        // G->T pair of each entry with this tile (-1: none)
+    float xch[4][kBsMax][kNumGrads];         // moments of each wave's 16 voxels
 };
 
 // e of Gaussian p at voxel (x, y, z) with the operations of lane_geom / lane_exp / lane_e (so the
@@ -1186,15 +1194,51 @@ __device__ __forceinline__ float voxel_e(const Grid& G, const GaussParams& p, in
     return __builtin_amdgcn_exp2f(fmaf(gxy, dz, fxy + fz));
 }
 
-// BF: grad_feats and the features are bfloat16 (the split rows then hold 64-channel chunks of the
-// values).
+// U of the wave's 16 voxels against NB blocks of 16 list entries; arow: the lane's gF row, brow: its
+// entries' feature rows.
+template <int NB, typename T>
+__device__ __forceinline__ void bs_products(const T* __restrict__ arow, const T* const (&brow)[kBsNb], int C, int q,
+                                            f32x4 (&u)[kBsNb]) {
+    constexpr int kU = NB <= 2 ? 2 : 1;   // steps of 16 channels per group of loads
+    f32x4 a[2][kU], b[2][kU][NB];
+    auto load = [&](int s0, int buf) {
+#pragma unroll
+        for (int i = 0; i < kU; ++i) {
+            const int c = (s0 + i) * 16 + 4 * q;
+            a[buf][i] = load4_row(arow, c, C);
+#pragma unroll
+            for (int k = 0; k < NB; ++k) b[buf][i][k] = load4_row(brow[k], c, C);
+        }
+    };
+    auto mult = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < kU; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int k = 0; k < NB; ++k)
+                    u[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[buf][i][e], b[buf][i][k][e], u[k], 0, 0, 0);
+    };
+    const int ns = (C + 15) >> 4;
+    load(0, 0);
+    for (int s = 0; s < ns; s += 2 * kU) {   // steps past the row load zeros
+        if (s + kU < ns) load(s + kU, 1);
+        mult(0);
+        if (s + kU < ns) {
+            if (s + 2 * kU < ns) load(s + 2 * kU, 0);
+            mult(1);
+        }
+    }
+}
+
+// BF: grad_feats and the features are bfloat16.
 template <bool BF>
-__global__ void __launch_bounds__(kBsThreads) k_bwd_tile_short(
-    Grid G, int n, int C, int nchk, const float* __restrict__ gD, const void* __restrict__ gF_,
+__global__ void __launch_bounds__(kBsThreads, 4) k_bwd_tile_short(
+    Grid G, int C, const float* __restrict__ gD, const void* __restrict__ gF_,
     const float* __restrict__ means, const float* __restrict__ opacity, const float* __restrict__ cov_inv,
     const int* __restrict__ lb, const int* __restrict__ ub, const int* __restrict__ g2t_offsets,
     const int* __restrict__ toff, const int* __restrict__ sorted_gauss, int M, const float* __restrict__ density,
-    const __bf16* __restrict__ fsp, float* __restrict__ pair_partials, __bf16* __restrict__ wt, int smax) {
+    const void* __restrict__ features, float* __restrict__ pair_partials, __bf16* __restrict__ wt, int smax) {
     __shared__ BsSmem sm;
     const int T = scene_tiles(G);
     const int tb = uniform(xcd_remap(blockIdx.x, gridDim.x));   // the batch's tile (its list)
@@ -1203,195 +1247,152 @@ __global__ void __launch_bounds__(kBsThreads) k_bwd_tile_short(
     const int Ng = uniform(min(max(toff[tb + 1], j0), M)) - j0;
     if (Ng <= 0 || Ng > smax) return;
     const int scene = uniform(tb / T), tile = tb - scene * T;
-    typedef typename std::conditional<BF, __bf16, float>::type GT;   // element of grad_feats
-    const GT* gF = static_cast<const GT*>(gF_);
-    if (scene > 0) {   // the scene's voxel rows
+    typedef typename std::conditional<BF, __bf16, float>::type FT;   // element of grad_feats and the features
+    const FT* gF = static_cast<const FT*>(gF_);
+    const FT* feats = static_cast<const FT*>(features);
+    {   // the scene's voxel rows
         const int64_t vb = scene * scene_voxels(G);
         gD += vb;
         density += vb;
         gF += vb * C;
     }
     const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
-    int x, y, z;
-    tile_voxel(G, tile, lane, x, y, z);   // voxel row lane of the tile
-
-    // Staging roles.  gF: voxel row sr, channels 8 sq .. 8 sq + 7 of a chunk.  Features: slots fs
-    // and fs + 32 (the zero row past the list), channels 4 fo .. 4 fo + 3.  A chunk's values are loaded into
-    // registers one chunk ahead (the first chunk's loads go out with the tile's own), stored to
-    // LDS at the chunk's start.
-    const int sr = threadIdx.x >> 2, sq = threadIdx.x & 3;
-    const int fs = threadIdx.x >> 3, fo = threadIdx.x & 7;
-    int rx, ry, rz;
-    tile_voxel(G, tile, sr, rx, ry, rz);
-    const bool srok = in_grid(G, rx, ry, rz);
-    const GT* gsrc = gF + (srok ? voxel_index(G, rx, ry, rz) : 0) * C;
-    const bool gvec = (C & 7) == 0 && ((uintptr_t)gF & 15) == 0;   // 16-byte row pieces
-    const int rowlen = nchk * 2 * kBtKc;                              // bf16 per split feature row
-    const __bf16* frow[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-        frow[h] = fsp + (int64_t)(fs + 32 * h < Ng ? sorted_gauss[j0 + fs + 32 * h] : n) * rowlen;
-    float gv[8], fv[2][4];
-    auto load_g = [&](int c0) {
-        const int c = c0 + 8 * sq;
-        if (gvec) {   // whole octets: C % 8 == 0
-            if (c < C) {
-                if constexpr (BF) {
-                    const uint4 h = *reinterpret_cast<const uint4*>(gsrc + c);
-                    const unsigned w[4] = {h.x, h.y, h.z, h.w};
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        gv[2 * i] = __uint_as_float(w[i] << 16);
-                        gv[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-                    }
-                } else {
-                    const float4 q0 = *reinterpret_cast<const float4*>(gsrc + c);
-                    const float4 q1 = *reinterpret_cast<const float4*>(gsrc + c + 4);
-                    gv[0] = q0.x; gv[1] = q0.y; gv[2] = q0.z; gv[3] = q0.w;
-                    gv[4] = q1.x; gv[5] = q1.y; gv[6] = q1.z; gv[7] = q1.w;
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 8; ++i) gv[i] = 0.0f;
-            }
-        } else {      // every element loaded (clamped into the row) before any is masked
-#pragma unroll
-            for (int i = 0; i < 8; ++i) gv[i] = (float)gsrc[min(c + i, C - 1)];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) gv[i] = c + i < C ? gv[i] : 0.0f;
-        }
-    };
-    auto load_f = [&](int c0) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            if constexpr (BF) {   // the values themselves, 64-channel chunks: element c at offset c
-                const uint2 hv = *reinterpret_cast<const uint2*>(frow[h] + c0 + 4 * fo);
-                fv[h][0] = __uint_as_float(hv.x << 16);
-                fv[h][1] = __uint_as_float(hv.x & 0xffff0000u);
-                fv[h][2] = __uint_as_float(hv.y << 16);
-                fv[h][3] = __uint_as_float(hv.y & 0xffff0000u);
-            } else {              // chunk c0 / 32: hi[32] then lo[32]
-                const __bf16* ck = frow[h] + (c0 / kBtKc) * (2 * kBtKc);
-                const uint2 hv = *reinterpret_cast<const uint2*>(ck + 4 * fo);
-                const uint2 lv = *reinterpret_cast<const uint2*>(ck + kBtKc + 4 * fo);
-                fv[h][0] = __uint_as_float(hv.x << 16) + __uint_as_float(lv.x << 16);
-                fv[h][1] = __uint_as_float(hv.x & 0xffff0000u) + __uint_as_float(lv.x & 0xffff0000u);
-                fv[h][2] = __uint_as_float(hv.y << 16) + __uint_as_float(lv.y << 16);
-                fv[h][3] = __uint_as_float(hv.y & 0xffff0000u) + __uint_as_float(lv.y & 0xffff0000u);
-            }
-        }
-    };
-    load_g(0);
-    load_f(0);
-    if (threadIdx.x < 64) {
-        const bool ok = in_grid(G, x, y, z);
-        const int64_t v = ok ? voxel_index(G, x, y, z) : 0;
-        sm.vlin[lane] = ok ? (int)v : -1;
-        sm.gD[lane] = ok ? gD[v] : 0.0f;
-        sm.D[lane] = ok ? density[v] : 0.0f;
-        sm.inv[lane] = ok ? 1.0f / fmaxf(density[v], kEps) : 0.0f;
-    }
-    stage_params(sm.pt, sorted_gauss + j0, Ng, means, cov_inv, opacity, lb, ub);
-
-    // U: thread (voxel lane, slots wave + 4 i) over 32-channel chunks staged in LDS; a wave
-    // multiplies only its slots' quads that hold list entries
-    const int nq = uniform((max(Ng - wave, 0) + 15) / 16);   // quads of 4 slots with an entry
-    float u[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) u[i] = 0.0f;
-    for (int c0 = 0; c0 < C; c0 += kBsKc) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) sm.g[sr][8 * sq + i] = srok ? gv[i] : 0.0f;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int sl = fs + 32 * h;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sm.f[4 * fo + i][sl & 3][sl >> 2] = fv[h][i];
-        }
-        __syncthreads();   // also orders the tile's own values and parameters before their reads
-        if (c0 + kBsKc < C) {   // the next chunk's loads run under this chunk's products
-            load_g(c0 + kBsKc);
-            load_f(c0 + kBsKc);
-        }
-#pragma unroll 4
-        for (int c = 0; c < kBsKc; ++c) {
-            const float a = sm.g[lane][c];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if (q < nq) {   // wave-uniform
-                    const float4 f4 = *reinterpret_cast<const float4*>(&sm.f[c][wave][4 * q]);
-                    u[4 * q] = fmaf(a, f4.x, u[4 * q]);
-                    u[4 * q + 1] = fmaf(a, f4.y, u[4 * q + 1]);
-                    u[4 * q + 2] = fmaf(a, f4.z, u[4 * q + 2]);
-                    u[4 * q + 3] = fmaf(a, f4.w, u[4 * q + 3]);
-                }
-            }
-        }
-        __syncthreads();
-    }
-
-    // split weights of every pair (row lane of the pair's weight row) and t_v from U
-    const bool rowok = sm.vlin[lane] >= 0;
-    const float inv = sm.inv[lane];
-    float tsum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int slot = wave + 4 * i;
-        if (slot >= Ng) break;   // wave-uniform
-        GaussParams p;
-        read_params(sm.pt, slot, p);
-        float dx, dy, dz;
-        bool in;
-        const float e0 = voxel_e(G, p, x, y, z, dx, dy, dz, in);
-        const float e = (rowok && in) ? e0 : 0.0f;
-        const float w = p.o * e;
-        const float wtil = w * inv;
-        __bf16 hs, ls;
-        split_bf16(wtil, hs, ls);
-        __bf16* wrow = wt + (int64_t)(j0 + slot) * kWtRow;
-        wrow[lane] = hs;
-        wrow[64 + lane] = ls;
-        tsum += (w > 0.0f) ? wtil * u[i] : 0.0f;
-    }
-    sm.tpart[wave][lane] = tsum;
-    lds_barrier();   // the weight stores stay in flight (later kernels read them)
-    if (threadIdx.x < 64) {
-        const float s = ((sm.tpart[0][lane] + sm.tpart[1][lane]) + sm.tpart[2][lane]) + sm.tpart[3][lane];
-        // sum_g [w>0] w u / max(D, eps) = sum_c gF F; zero where D < eps (reference .cu:1450)
-        sm.tv[lane] = (rowok && sm.D[lane] >= kEps) ? s : 0.0f;
-    }
-    lds_barrier();
-
-    // r = gw e and its moments over the tile's voxels (d = centre - mu), as k_bwd_tile stores them
-    const float tv = sm.tv[lane], gd = sm.gD[lane];
+    const int j = lane & 15, q = lane >> 4;
     const int tyz = G.tiles[1] * G.tiles[2];
     const int tx = tile / tyz, ty = (tile - tx * tyz) / G.tiles[2], tz = tile % G.tiles[2];
+    const int x = tx * kTile + wave, y0 = ty * kTile, z0 = tz * kTile;
+
+    // operand rows: voxel 16 wave + j (clamped into the grid: a row outside it only reaches results
+    // that are cleared) and list entries 16 b + j (the last entry again past the list: columns that
+    // nothing reads)
+    const FT* arow;
+    {
+        const int xr = min(x, G.dims[0] - 1), yr = min(y0 + (j >> 2), G.dims[1] - 1), zr = min(z0 + (j & 3), G.dims[2] - 1);
+        arow = gF + voxel_index(G, xr, yr, zr) * C;
+    }
+    const FT* brow[kBsNb];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int slot = wave + 4 * i;
-        if (slot >= Ng) break;   // wave-uniform
+    for (int b = 0; b < kBsNb; ++b) brow[b] = feats + (int64_t)sorted_gauss[j0 + min(16 * b + j, Ng - 1)] * C;
+    // the lane's result voxels (x, y0 + q, z0 + i)
+    float gd[4], dv[4];
+    const bool xyok = x < G.dims[0] && y0 + q < G.dims[1];
+    unsigned vok = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const bool ok = xyok && z0 + i < G.dims[2];
+        const int64_t v = ok ? voxel_index(G, x, y0 + q, z0 + i) : 0;
+        gd[i] = gD[v];
+        dv[i] = density[v];
+        vok |= ok ? 1u << i : 0u;
+    }
+    stage_params(sm.pt, sorted_gauss + j0, Ng, means, cov_inv, opacity, lb, ub);
+    for (int k = threadIdx.x; k < Ng; k += kBsThreads) {
+        const int g = sm.pt.gid[k];   // written by this thread
+        const int tx0 = sm.pt.lb[0][k] / kTile, ty0 = sm.pt.lb[1][k] / kTile, tz0 = sm.pt.lb[2][k] / kTile;
+        const int ey = sm.pt.ub[1][k] / kTile - ty0 + 1, ez = sm.pt.ub[2][k] / kTile - tz0 + 1;
+        const int64_t pair = (int64_t)g2t_offsets[g] + ((tx - tx0) * ey + (ty - ty0)) * ez + (tz - tz0);
+        sm.pidx[k] = pair >= 0 && pair < M ? (int)pair : -1;   // malformed CSR: never write outside the buffer
+    }
+
+    const int nb = (Ng + 15) >> 4;
+    f32x4 u[kBsNb];
+#pragma unroll
+    for (int b = 0; b < kBsNb; ++b) u[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    switch (nb) {
+        case 1: bs_products<1, FT>(arow, brow, C, q, u); break;
+        case 2: bs_products<2, FT>(arow, brow, C, q, u); break;
+        case 3: bs_products<3, FT>(arow, brow, C, q, u); break;
+        default: bs_products<4, FT>(arow, brow, C, q, u); break;
+    }
+    __syncthreads();   // the parameters
+
+    // split weights of every pair (voxel row 16 wave + 4 q + i of the pair's weight row) and t_v from U
+    float inv[4], t[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        inv[i] = (vok >> i) & 1u ? 1.0f / fmaxf(dv[i], kEps) : 0.0f;
+        t[i] = 0.0f;
+    }
+    float e[kBsNb][4];
+    unsigned okm = 0;   // bit 4 b + i: the element lies in the grid, the box and the list
+#pragma unroll
+    for (int b = 0; b < kBsNb; ++b) {
+        if (b >= nb) break;   // uniform
+        const int slot = 16 * b + j;
+        const bool live = slot < Ng;
         GaussParams p;
-        read_params(sm.pt, slot, p);
-        float dx, dy, dz;
-        bool in;
-        const float e0 = voxel_e(G, p, x, y, z, dx, dy, dz, in);
-        const float gw = gd + (u[i] - tv) * inv;
-        const float r = (rowok && in) ? gw * e0 : 0.0f;
-        const float m[16] = {r * dx, r * dy, r * dz, r * dx * dx, r * dy * dy, r * dz * dz,
-                             r * dx * dy, r * dx * dz, r * dy * dz, r, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        // lanes 2k and 2k + 1 of each half-wave get the half's sum of m[k]; lane 2k adds the other
-        // half's and stores value k of the pair
-        float t = transpose_sum16(m, lane & 31);
-        t += __shfl_down(t, 32, 64);
-        const int k = lane >> 1;
-        if ((lane & 1) == 0 && k < kNumGrads) {
-            const int g = sm.pt.gid[slot];
-            const int tx0 = p.lb[0] / kTile, ty0 = p.lb[1] / kTile, tz0 = p.lb[2] / kTile;
-            const int ey = p.ub[1] / kTile - ty0 + 1, ez = p.ub[2] / kTile - tz0 + 1;
-            const int64_t pair = (int64_t)g2t_offsets[g] + ((tx - tx0) * ey + (ty - ty0)) * ez + (tz - tz0);
-            if (pair >= 0 && pair < M)   // malformed CSR: never write outside the buffer
-                pair_partials[pair * kNumGrads + k] = k < kNumGrads - 1 ? p.o * t : t;
+        read_params(sm.pt, live ? slot : Ng - 1, p);
+        typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+        bf16x4 hv, lv;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float dx, dy, dz;
+            bool in;
+            const float e0 = voxel_e(G, p, x, y0 + q, z0 + i, dx, dy, dz, in);
+            const bool ok = live && in && ((vok >> i) & 1u);
+            e[b][i] = ok ? e0 : 0.0f;
+            okm |= ok ? 1u << (4 * b + i) : 0u;
+            const float w = p.o * e[b][i];
+            const float wtil = w * inv[i];
+            __bf16 hs, ls;
+            split_bf16(wtil, hs, ls);
+            hv[i] = hs;
+            lv[i] = ls;
+            t[i] += (w > 0.0f) ? wtil * u[b][i] : 0.0f;
         }
+        if (live) {
+            __bf16* wrow = wt + (int64_t)(j0 + slot) * kWtRow + 16 * wave + 4 * q;
+            *reinterpret_cast<bf16x4*>(wrow) = hv;
+            *reinterpret_cast<bf16x4*>(wrow + 64) = lv;
+        }
+    }
+    // sum_g [w>0] w u / max(D, eps) = sum_c gF F over the 16 lanes; zero where D < eps (reference .cu:1450)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float s = t[i];
+        s += xor_shfl<1>(s);
+        s += xor_shfl<2>(s);
+        s += xor_shfl<4>(s);
+        s += xor_shfl<8>(s);
+        t[i] = dv[i] >= kEps ? s : 0.0f;
+    }
+    // r = gw e and its moments over the voxels (d = centre - mu), as k_bwd_tile stores them
+#pragma unroll
+    for (int b = 0; b < kBsNb; ++b) {
+        if (b >= nb) break;   // uniform
+        const int slot = 16 * b + j;
+        const int ps = min(slot, Ng - 1);
+        const float dx = centre(G, 0, x) - sm.pt.mu[0][ps], dy = centre(G, 1, y0 + q) - sm.pt.mu[1][ps];
+        const float muz = sm.pt.mu[2][ps], o = sm.pt.o[ps];
+        float s0 = 0.0f, sz = 0.0f, szz = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float gw = gd[i] + (u[b][i] - t[i]) * inv[i];
+            const float r = (okm >> (4 * b + i)) & 1u ? gw * e[b][i] : 0.0f;   // an element outside adds exact zeros
+            const float dz = centre(G, 2, z0 + i) - muz;
+            s0 += r;
+            sz = fmaf(r, dz, sz);
+            szz = fmaf(r * dz, dz, szz);
+        }
+        float m[kNumGrads] = {o * dx * s0, o * dy * s0, o * sz, o * dx * dx * s0, o * dy * dy * s0, o * szz,
+                              o * dx * dy * s0, o * dx * sz, o * dy * sz, s0};
+#pragma unroll
+        for (int k = 0; k < kNumGrads; ++k) {   // the four lane groups (y)
+            m[k] += xor_shfl<16>(m[k]);
+            m[k] += __shfl_xor(m[k], 32, 64);
+        }
+        if (q == 0 && slot < Ng) {
+#pragma unroll
+            for (int k = 0; k < kNumGrads; ++k) sm.xch[wave][slot][k] = m[k];
+        }
+    }
+    lds_barrier();   // the weight stores stay in flight (later kernels read them)
+    for (int i = threadIdx.x; i < Ng * kNumGrads; i += kBsThreads) {
+        const int slot = i / kNumGrads, k = i - slot * kNumGrads;
+        const int pair = sm.pidx[slot];
+        if (pair >= 0)
+            pair_partials[(int64_t)pair * kNumGrads + k] =
+                ((sm.xch[0][slot][k] + sm.xch[1][slot][k]) + sm.xch[2][slot][k]) + sm.xch[3][slot][k];
     }
 }
 
@@ -2212,13 +2213,13 @@ hipError_t launch_backward_feats(const Grid& G, int n, int C, const float* grad_
         const int lblocks = (int)ceil_div(nlong, 8) * 8;
         if (!cos) {
             if (fdt == kDtBF16)
-                G2V_LAUNCH(k_bwd_tile_short<true>, dim3(blocks), dim3(kBsThreads), 0, s, G, n, C, nchk, grad_density,
-                           grad_feats, means, opacity, cov_inv, lb, ub, g2t_offsets, tile_offsets, sorted_gauss, (int)M,
-                           density, (const __bf16*)b.fsp, b.partials, b.wt, skip_le);
+                G2V_LAUNCH(k_bwd_tile_short<true>, dim3(blocks), dim3(kBsThreads), 0, s, G, C, grad_density, grad_feats,
+                           means, opacity, cov_inv, lb, ub, g2t_offsets, tile_offsets, sorted_gauss, (int)M, density,
+                           features, b.partials, b.wt, skip_le);
             else
-                G2V_LAUNCH(k_bwd_tile_short<false>, dim3(blocks), dim3(kBsThreads), 0, s, G, n, C, nchk, grad_density,
-                           grad_feats, means, opacity, cov_inv, lb, ub, g2t_offsets, tile_offsets, sorted_gauss, (int)M,
-                           density, (const __bf16*)b.fsp, b.partials, b.wt, skip_le);
+                G2V_LAUNCH(k_bwd_tile_short<false>, dim3(blocks), dim3(kBsThreads), 0, s, G, C, grad_density, grad_feats,
+                           means, opacity, cov_inv, lb, ub, g2t_offsets, tile_offsets, sorted_gauss, (int)M, density,
+                           features, b.partials, b.wt, skip_le);
         }
 #define G2V_BT(V, F, FU)                                                                                      \
     G2V_LAUNCH((k_bwd_tile<V, F, FU>), dim3(lblocks), dim3(kBtThreads), 0, s, G, n, C, nchk, grad_density,         \

@@ -377,9 +377,8 @@ int splat_impl(const Grid& G, int n, int feat_dim, const float* means3D, const f
                    num_pairs, b, s, means3D, opacity, cov_inv);
     if (rc != G2V_OK) return rc;
     if (feat_dim > 0)
-        G2V_HIP(launch_forward_feats(G, feat_dim, means3D, opacity, cov_inv, valid_voxel_lb,
-                                     valid_voxel_ub, b.tile_offsets, b.sorted_gauss, (int)num_pairs, n,
-                                     features, feat_dtype, b.fpk, b.drec, density, grid_feats, b.tl, s));
+        G2V_HIP(launch_forward_feats(G, feat_dim, b.tile_offsets, b.sorted_gauss, (int)num_pairs, n, features,
+                                     feat_dtype, b.fpk, b.drec, density, grid_feats, b.tl, s));
     else
         G2V_HIP(launch_forward_density(G, b.drec, b.tile_offsets, b.sorted_gauss, (int)num_pairs, density, s));
     return G2V_OK;

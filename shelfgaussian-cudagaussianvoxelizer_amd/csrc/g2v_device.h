@@ -293,20 +293,47 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-// Load 8 consecutive floats p[0..7] where only the first `valid` (0..8) are in bounds; the
-// rest read as 0.  `vec_ok` says p is 16-byte aligned so two dwordx4 loads can be used.
-__device__ __forceinline__ void load8(const float* __restrict__ p, int valid, bool vec_ok, float (&v)[8]) {
-    if (valid >= 8 && vec_ok) {
-        const float4 a = *reinterpret_cast<const float4*>(p);
-        const float4 b = *reinterpret_cast<const float4*>(p + 4);
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+// Four consecutive elements c .. c + 3 of a row of C elements as floats, 0 past the row.  Rows need
+// only their element's alignment: one load of four elements where they all lie in the row.
+template <typename T>
+__device__ __forceinline__ f32x4 load4_row(const T* __restrict__ row, int c, int C) {
+    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (c + 4 <= C) {
+        if constexpr (sizeof(T) == 4) {
+            typedef float f32x4_e __attribute__((ext_vector_type(4), aligned(4)));
+            v = *reinterpret_cast<const f32x4_e*>(row + c);
+        } else {
+            typedef __bf16 bf16x4_e __attribute__((ext_vector_type(4), aligned(2)));
+            const bf16x4_e h = *reinterpret_cast<const bf16x4_e*>(row + c);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = (float)h[i];
+        }
     } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = (i < valid) ? p[i] : 0.0f;
+        for (int i = 0; i < 4; ++i)
+            if (c + i < C) v[i] = (float)row[c + i];
     }
+    return v;
 }
 
+// The matching streaming store of v to elements c .. c + 3 (those that lie in the row).
+template <typename T>
+__device__ __forceinline__ void store4_row(T* __restrict__ row, int c, int C, f32x4 v) {
+    if (c + 4 <= C) {
+        if constexpr (sizeof(T) == 4) {
+            typedef float f32x4_e __attribute__((ext_vector_type(4), aligned(4)));
+            __builtin_nontemporal_store((f32x4_e)v, reinterpret_cast<f32x4_e*>(row + c));
+        } else {
+            typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+            typedef __bf16 bf16x4_e __attribute__((ext_vector_type(4), aligned(2)));
+            *reinterpret_cast<bf16x4_e*>(row + c) = (bf16x4_e)__builtin_convertvector(v, bf16x4);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (c + i < C) row[c + i] = (T)v[i];
+    }
+}
 
 // Feature element e of a row of type T, as float.
 template <typename T>

@@ -434,32 +434,29 @@ __device__ __forceinline__ void fwd_zero_tile(const Grid& G, int tile, int C, fl
 
 // ------------------------------------------------------------------------------------------
 // Tiles whose list holds at most smax <= kFsMax Gaussians, empty ones included.  k_fwd_feats keeps two
-// tiles per CU (its LDS holds a 224-Gaussian K chunk), so a short list leaves that tile's chain of
-// loads and barriers bare; here a 4-wave workgroup with about 10 KB of LDS takes the tile and many
-// run per CU.  The weights are those of fwd_build_w (the same operations), the density their sum
-// (in another order), the features float32 sums of max(w, 0) f over the list in its order, read
-// straight from the caller's features.  Which kernel takes a tile depends on its list length
-// alone.
+// tiles per CU (its LDS holds a 256-Gaussian K chunk), so a short list leaves that tile's chain of
+// loads and barriers bare; here a 4-wave workgroup without LDS takes the tile and many run per CU.
+// S = W F on the float32 matrix cores (16x16x4): wave w owns the 16 voxels x = x0 + w, lane l % 16 = voxel,
+// and the lane group q = l / 16 evaluates the weights of the list entries 4 s + q, which are then the A
+// operand of step s as they are (no weight is evaluated twice, none goes through memory).  A lane
+// loads one 16-byte piece of entry 4 s + q's feature row, four channels for the four MFMAs of a
+// 64-channel block, straight from the caller's features; a result row lies in 16 lanes as 64
+// consecutive channels.  Rows whose channels do not make whole 16-byte pieces take single channels, 16
+// consecutive ones per MFMA, so that loads and stores stay in runs of 64 bytes.
+// The weights are those of fwd_build_w (the same operations), the density their sum (in another
+// order), the features float32 sums of max(w, 0) f.  Which kernel takes a tile depends on its list
+// length alone.
 // ------------------------------------------------------------------------------------------
 constexpr int kFsThreads = 256;
 constexpr int kFsMax = 64;          // longest list the kernel can take
-constexpr int kFsStride = kFsMax + 4;   // weight row of a voxel: 16-byte aligned, few bank conflicts
+constexpr int kFsSteps = kFsMax / 4;
 
-struct FsSmem {
-    alignas(16) float w[64][kFsStride];   // feature weights max(w, 0): [voxel row][slot]
-    float dpart[kFsThreads / 64][64];
-    float inv[64];
-    int vlin[64];
-    int gid[kFsMax];
-};
-
-template <bool OBF16>
-__global__ void __launch_bounds__(kFsThreads) k_fwd_short(
-    Grid G, int C, const float* __restrict__ means, const float* __restrict__ opacity,
-    const float* __restrict__ cov_inv, const int* __restrict__ lb, const int* __restrict__ ub,
-    const int* __restrict__ toff, const int* __restrict__ sorted_gauss, int M, const void* __restrict__ features,
-    float* __restrict__ density, void* __restrict__ grid_feats_out, int smax) {
-    __shared__ FsSmem sm;
+// VEC: rows of features and grid_feats are whole aligned groups of four channels.
+template <bool OBF16, bool VEC>
+__global__ void __launch_bounds__(kFsThreads, 4) k_fwd_short(
+    Grid G, int C, const DenParams* __restrict__ drec, const int* __restrict__ toff,
+    const int* __restrict__ sorted_gauss, int M, const void* __restrict__ features, float* __restrict__ density,
+    void* __restrict__ grid_feats_out, int smax) {
     const int T = scene_tiles(G);
     const int tb = uniform(xcd_remap(blockIdx.x, gridDim.x));   // the batch's tile (its list)
     if (tb >= T * G.scenes) return;
@@ -478,91 +475,106 @@ __global__ void __launch_bounds__(kFsThreads) k_fwd_short(
     }
     typedef typename std::conditional<OBF16, __bf16, float>::type FT;   // element of the features
     const FT* feats = static_cast<const FT*>(features);
+    FT* out = static_cast<FT*>(grid_feats_out);
     const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
+    const int j = lane & 15, q = lane >> 4;
     int x, y, z;
-    tile_voxel(G, tile, lane, x, y, z);   // voxel row lane of the tile
+    tile_voxel(G, tile, 16 * wave + j, x, y, z);   // the lane's voxel
     const float cx = centre(G, 0, x), cy = centre(G, 1, y), cz = centre(G, 2, z);
+    const int ns = (Ng + 3) >> 2;
 
-    // weights of voxel row lane against slots wave + 4 i (fwd_build_w's operations); every slot's
-    // weight is written, 0 past the list
-    float dsum = 0.0f;
-#pragma unroll 1
-    for (int i = 0; i < kFsMax / 4; ++i) {
-        const int slot = wave + 4 * i;
-        float wf = 0.0f;
-        if (slot < Ng) {   // wave-uniform
-            const int g = uniform(sorted_gauss[j0 + slot]);
-            float A[9];
+    // the Gaussians of the lane group's entries 4 s + q (the last entry again past the list)
+    const FT* frow[kFsSteps];
+    float w[kFsSteps];
+    float D = 0.0f;
 #pragma unroll
-            for (int k = 0; k < 9; ++k) A[k] = cov_inv[g * 9 + k];
-            const float a00 = kq * A[0], a01 = kq * (A[1] + A[3]), a11 = kq * A[4];
-            const float a02 = kq * (A[2] + A[6]), a12 = kq * (A[5] + A[7]), a22 = kq * A[8];
-            const bool inxy = x >= lb[g * 3] && x <= ub[g * 3] && y >= lb[g * 3 + 1] && y <= ub[g * 3 + 1];
-            const bool inz = z >= lb[g * 3 + 2] && z <= ub[g * 3 + 2];
-            const float dx = cx - means[g * 3], dy = cy - means[g * 3 + 1], dz = cz - means[g * 3 + 2];
-            const float fz = inz ? a22 * dz * dz : -__builtin_inff();
-            float F = fmaf(fmaf(a00, dx, a01 * dy), dx, a11 * dy * dy);
+    for (int s = 0; s < kFsSteps; ++s) {
+        if (s < ns) {   // uniform
+            const int slot = 4 * s + q;
+            const int g = sorted_gauss[j0 + min(slot, Ng - 1)];
+            frow[s] = feats + (int64_t)g * C;
+            const DenParams p = drec[g];
+            // fwd_column_weights' operations
+            const bool inxy = x >= p.lbx && x <= p.ubx && y >= p.lby && y <= p.uby;
+            const bool inz = z >= p.lbz && z <= p.ubz;
+            const float dx = cx - p.mux, dy = cy - p.muy, dz = cz - p.muz;
+            const float fz = inz ? p.a22 * dz * dz : -__builtin_inff();
+            float F = fmaf(fmaf(p.a00, dx, p.a01 * dy), dx, p.a11 * dy * dy);
             F = inxy ? F : -__builtin_inff();
-            const float Gxy = fmaf(a02, dx, a12 * dy);
-            const float w = opacity[g] * __builtin_amdgcn_exp2f(fmaf(Gxy, dz, F) + fz);
-            dsum += w;
-            wf = fmaxf(w, 0.0f);   // feature gate of the reference (.cu:936)
-            if (lane == 0) sm.gid[slot] = g;
+            const float Gxy = fmaf(p.a02, dx, p.a12 * dy);
+            const float wv = slot < Ng ? p.o * __builtin_amdgcn_exp2f(fmaf(Gxy, dz, F) + fz) : 0.0f;
+            D += wv;
+            w[s] = fmaxf(wv, 0.0f);   // feature gate of the reference (.cu:936)
+        } else {
+            frow[s] = feats;
+            w[s] = 0.0f;
         }
-        sm.w[lane][slot] = wf;
     }
-    sm.dpart[wave][lane] = dsum;
-    __syncthreads();
-    if (wave == 0) {
-        const float D = ((sm.dpart[0][lane] + sm.dpart[1][lane]) + sm.dpart[2][lane]) + sm.dpart[3][lane];
-        const bool ok = in_grid(G, x, y, z);
-        const int v = ok ? (int)voxel_index(G, x, y, z) : -1;
-        sm.inv[lane] = 1.0f / fmaxf(D, kEps);
-        sm.vlin[lane] = v;
-        if (ok) density[v] = D;
+    D += xor_shfl<16>(D);   // the four lane groups' entries
+    D += __shfl_xor(D, 32, 64);
+    const bool ok = in_grid(G, x, y, z);
+    const int v = ok ? (int)voxel_index(G, x, y, z) : -1;
+    if (ok && q == 0) density[v] = D;
+    const float inv = 1.0f / fmaxf(D, kEps);
+    float rinv[4];   // of the lane's result rows, voxels 4 q + i of the wave
+    int rv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        rinv[i] = __shfl(inv, 4 * q + i, 64);
+        rv[i] = __shfl(v, 4 * q + i, 64);
     }
-    __syncthreads();
 
-    // features: wave w owns voxel rows 16 w .. 16 w + 15, lane = channel of a 64-channel block;
-    // the list is taken 8 slots at a time (slots past it have weight 0 and read as 0)
+    const bool tail = 4 * (ns - 1) + q >= Ng;   // the lane's entry of the last step lies past the list
     for (int cb = 0; cb < C; cb += 64) {
-        const int c = cb + lane;
-        const int cc = min(c, C - 1);
-        float acc[16];
+        f32x4 acc[4];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-        for (int s0 = 0; s0 < Ng; s0 += 8) {
-            float f[8];
+        for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        // component i of a lane's four channels: cb + 4 j + i (VEC) or cb + 16 i + j
+        const int c0 = VEC ? min(cb + 4 * j, C - 4) : cb + j;
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {   // every load issued before the first product
-                const int sl = s0 + k;
-                const int g = uniform(sm.gid[min(sl, Ng - 1)]);   // a uniform row base: one offset register for all
-                f[k] = sl < Ng ? (float)feats[(int64_t)g * C + cc] : 0.0f;
+        for (int s0 = 0; s0 < kFsSteps; s0 += 4) {
+            if (s0 >= ns) break;   // uniform
+            f32x4 f[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {   // the loads of four steps before their products
+                const int s = s0 + k;
+                if constexpr (VEC) {
+                    f[k] = load4_row(frow[s], c0, C);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) f[k][i] = (float)frow[s][min(c0 + 16 * i, C - 1)];
+                }
             }
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float* wr = &sm.w[16 * wave + r][s0];
-                const float4 wa = *reinterpret_cast<const float4*>(wr);
-                const float4 wb = *reinterpret_cast<const float4*>(wr + 4);
-                acc[r] = fmaf(wa.x, f[0], acc[r]);
-                acc[r] = fmaf(wa.y, f[1], acc[r]);
-                acc[r] = fmaf(wa.z, f[2], acc[r]);
-                acc[r] = fmaf(wa.w, f[3], acc[r]);
-                acc[r] = fmaf(wb.x, f[4], acc[r]);
-                acc[r] = fmaf(wb.y, f[5], acc[r]);
-                acc[r] = fmaf(wb.z, f[6], acc[r]);
-                acc[r] = fmaf(wb.w, f[7], acc[r]);
+            for (int k = 0; k < 4; ++k) {
+                const int s = s0 + k;
+                if (s >= ns) break;   // uniform
+                const bool past = tail && s == ns - 1;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)   // an entry past the list reads as zeros
+                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[s], past ? 0.0f : f[k][i], acc[i], 0, 0, 0);
             }
         }
-        if (c < C) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = 16 * wave + r;
-                const int v = sm.vlin[row];
-                if (v < 0) continue;
-                const float o = acc[r] * sm.inv[row];
-                if constexpr (OBF16) static_cast<__bf16*>(grid_feats_out)[(int64_t)v * C + c] = (__bf16)o;
-                else __builtin_nontemporal_store(o, static_cast<float*>(grid_feats_out) + (int64_t)v * C + c);
+        for (int r = 0; r < 4; ++r) {
+            if (rv[r] < 0) continue;
+            FT* row = out + (int64_t)rv[r] * C;
+            if constexpr (VEC) {
+                if (cb + 4 * j < C) {
+                    const f32x4 o = {acc[0][r] * rinv[r], acc[1][r] * rinv[r], acc[2][r] * rinv[r], acc[3][r] * rinv[r]};
+                    if constexpr (OBF16) {
+                        typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+                        *reinterpret_cast<bf16x4*>(row + cb + 4 * j) = __builtin_convertvector(o, bf16x4);
+                    } else {
+                        __builtin_nontemporal_store(o, reinterpret_cast<f32x4*>(row + cb + 4 * j));
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int c = cb + 16 * i + j;
+                    if (c < C) row[c] = (FT)(acc[i][r] * rinv[r]);
+                }
             }
         }
     }
@@ -813,9 +825,7 @@ hipError_t launch_split_pack(int n, int C, const void* features, int fdt, uint32
     return hipGetLastError();
 }
 
-hipError_t launch_forward_feats(const Grid& G, int C, const float* means, const float* opacity,
-                                const float* cov_inv, const int* lb, const int* ub,
-                                const int* tile_offsets, const int* sorted_gauss, int M, int n,
+hipError_t launch_forward_feats(const Grid& G, int C, const int* tile_offsets, const int* sorted_gauss, int M, int n,
                                 const void* features, int fdt, const uint32_t* fpk, const DenParams* drec,
                                 float* density, void* grid_feats, int* tl_ws, hipStream_t s) {
     const int T = scene_tiles(G) * G.scenes;
@@ -840,19 +850,26 @@ hipError_t launch_forward_feats(const Grid& G, int C, const float* means, const 
         tlist = tl_ws + 1;
     }
     const int lblocks = (int)ceil_div(nlong, 8) * 8;
+    // whole aligned groups of four channels (float: 16 bytes, bfloat16: 8)
+    const uintptr_t am = fdt == kDtBF16 ? 7 : 15;
+    const bool vec = (C & 3) == 0 && ((uintptr_t)features & am) == 0 && ((uintptr_t)grid_feats & am) == 0;
+#define G2V_FS(F, V)                                                                                               \
+    G2V_LAUNCH((k_fwd_short<F, V>), dim3(blocks), dim3(kFsThreads), 0, s, G, C, drec, tile_offsets, sorted_gauss, M, \
+               features, density, grid_feats, smax)
     if (fdt == kDtBF16) {
-        G2V_LAUNCH(k_fwd_short<true>, dim3(blocks), dim3(kFsThreads), 0, s, G, C, means, opacity, cov_inv, lb, ub,
-                   tile_offsets, sorted_gauss, M, features, density, grid_feats, smax);
+        if (vec) G2V_FS(true, true);
+        else G2V_FS(true, false);
         if (nlong > 0)
             G2V_LAUNCH(k_fwd_feats<true>, dim3(lblocks), dim3(kFwdThreads), 0, s, G, C, drec, tile_offsets,
                        sorted_gauss, M, n, Cp, (const uint32_t*)fpk, density, grid_feats, smax, tlist, tcount);
     } else {
-        G2V_LAUNCH(k_fwd_short<false>, dim3(blocks), dim3(kFsThreads), 0, s, G, C, means, opacity, cov_inv, lb, ub,
-                   tile_offsets, sorted_gauss, M, features, density, grid_feats, smax);
+        if (vec) G2V_FS(false, true);
+        else G2V_FS(false, false);
         if (nlong > 0)
             G2V_LAUNCH(k_fwd_feats<false>, dim3(lblocks), dim3(kFwdThreads), 0, s, G, C, drec, tile_offsets,
                        sorted_gauss, M, n, Cp, (const uint32_t*)fpk, density, grid_feats, smax, tlist, tcount);
     }
+#undef G2V_FS
     return hipGetLastError();
 }
 

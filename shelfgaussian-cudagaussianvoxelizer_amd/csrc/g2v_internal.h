@@ -122,9 +122,7 @@ hipError_t launch_forward_density(const Grid& G, const DenParams* drec, const in
 // row, plus a zero row); it depends on the features alone.
 hipError_t launch_split_pack(int n, int C, const void* features, int fdt, uint32_t* fpk, hipStream_t s);
 // fpk: launch_split_pack's output for these features, queued before on s.
-hipError_t launch_forward_feats(const Grid& G, int C, const float* means, const float* opacity,
-                                const float* cov_inv, const int* lb, const int* ub,
-                                const int* tile_offsets, const int* sorted_gauss, int M, int n,
+hipError_t launch_forward_feats(const Grid& G, int C, const int* tile_offsets, const int* sorted_gauss, int M, int n,
                                 const void* features, int fdt, const uint32_t* fpk, const DenParams* drec,
                                 float* density, void* grid_feats, int* tl_ws, hipStream_t s);
 // ints of the long-tile list workspace (tl_ws) of a forward or backward with features.
