@@ -412,7 +412,7 @@ __device__ __forceinline__ void fwd_zero_tile(const Grid& G, int tile, int C, fl
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int x, y, z;
     tile_voxel(G, tile, lane, x, y, z);
-    if (threadIdx.x < 64 && in_grid(G, x, y, z)) density[voxel_index(G, x, y, z)] = 0.0f;
+    if (wave == 0 && in_grid(G, x, y, z)) density[voxel_index(G, x, y, z)] = 0.0f;
     const int x0 = x & ~(kTile - 1), y0 = y & ~(kTile - 1), z0 = z & ~(kTile - 1);
     constexpr int kEs = OBF16 ? 2 : 4;
     const int64_t run = (int64_t)min(kTile, G.dims[2] - z0) * C * kEs;   // bytes of a column
@@ -420,14 +420,14 @@ __device__ __forceinline__ void fwd_zero_tile(const Grid& G, int tile, int C, fl
         const int xc = x0 + (c >> 2), yc = y0 + (c & 3);
         if (xc >= G.dims[0] || yc >= G.dims[1]) continue;   // wave-uniform
         char* dst = static_cast<char*>(grid_feats_out) + voxel_index(G, xc, yc, z0) * C * kEs;
-        if (((uintptr_t)dst & 15) == 0 && (run & 15) == 0) {
-            for (int64_t b = (int64_t)lane * 16; b < run; b += 64 * 16)
-                __builtin_nontemporal_store(f32x4{0.0f, 0.0f, 0.0f, 0.0f}, reinterpret_cast<f32x4*>(dst + b));
-        } else {
-            for (int64_t b = (int64_t)lane * kEs; b < run; b += 64 * kEs) {
-                if constexpr (OBF16) *reinterpret_cast<unsigned short*>(dst + b) = 0;
-                else *reinterpret_cast<float*>(dst + b) = 0.0f;
-            }
+        typedef float f32x4_e __attribute__((ext_vector_type(4), aligned(2)));   // an element's alignment is enough
+        const int64_t whole = run & ~(int64_t)15;
+        for (int64_t b = (int64_t)lane * 16; b < whole; b += 64 * 16)
+            __builtin_nontemporal_store(f32x4_e{0.0f, 0.0f, 0.0f, 0.0f}, reinterpret_cast<f32x4_e*>(dst + b));
+        const int64_t b = whole + (int64_t)lane * kEs;   // the last bytes
+        if (b < run) {
+            if constexpr (OBF16) *reinterpret_cast<unsigned short*>(dst + b) = 0;
+            else *reinterpret_cast<float*>(dst + b) = 0.0f;
         }
     }
 }
@@ -435,6 +435,7 @@ __device__ __forceinline__ void fwd_zero_tile(const Grid& G, int tile, int C, fl
 // ------------------------------------------------------------------------------------------
 // Tiles whose list holds at most smax <= kFsMax Gaussians, empty ones included.  k_fwd_feats keeps two
 // tiles per CU (its LDS holds a 256-Gaussian K chunk), so a short list leaves that tile's chain of
+<<<<<<< Updated upstream
 // loads and barriers bare; here a 4-wave workgroup without LDS takes the tile and many run per CU.
 // S = W F on the float32 matrix cores (16x16x4): wave w owns the 16 voxels x = x0 + w, lane l % 16 = voxel,
 // and the lane group q = l / 16 evaluates the weights of the list entries 4 s + q, which are then the A
@@ -457,6 +458,41 @@ __global__ void __launch_bounds__(kFsThreads, 4) k_fwd_short(
     Grid G, int C, const DenParams* __restrict__ drec, const int* __restrict__ toff,
     const int* __restrict__ sorted_gauss, int M, const void* __restrict__ features, float* __restrict__ density,
     void* __restrict__ grid_feats_out, int smax) {
+=======
+// loads and barriers bare; here a 4-wave workgroup with 17 KB of LDS takes the tile and several
+// run per CU.
+// S = W F on the float32 matrix cores (16x16x4): wave w owns the 16 voxels x = x0 + w, lane l % 16 = voxel,
+// and the lane group q = l / 16 evaluates the weights of the list entries 4 s + q, which are then the A
+// operand of step s as they are (no weight is evaluated twice; they wait in LDS, each read by the lane that
+// wrote it).  A lane
+// loads one 16-byte piece of entry 4 s + q's feature row, four channels for the four MFMAs of a
+// 64-channel block, straight from the caller's features; a result row lies in 16 lanes as 64
+// consecutive channels, in runs of 256 bytes whatever the rows' alignment (single channels in runs of
+// 64 bytes took 0.21 instead of 0.17 ms on 4 scenes of 64 x 191 x 11 x 891).
+// The weights are those of fwd_build_w (the same operations), the density their sum (in another
+// order), the features float32 sums of max(w, 0) f.  Which kernel takes a tile depends on its list
+// length alone.
+// Against weights in LDS and vector products: seven tiles at 768 channels beside 9,993 long ones 0.088 ->
+// 0.040 ms (their chain of dependent loads and stores), 4 scenes of 64 x 191 x 11 x 891 0.178 -> 0.151 ms,
+// 6 sparse scenes of 200 x 200 x 16 x 64 0.163 -> 0.155 ms (0.98 GB written, 0.14 ms at the fill rate).
+// ------------------------------------------------------------------------------------------
+constexpr int kFsThreads = 256;
+constexpr int kFsMax = 64;          // longest list the kernel can take
+constexpr int kFsGrp = 2;           // steps whose pieces are loaded together
+
+// Of each wave: the weight of every step and lane, and the feature row's byte offset of every entry.
+struct FsSmem {
+    float w[kFsThreads / 64][kFsMax / 4][64];
+    uint32_t off[kFsThreads / 64][kFsMax];
+};
+
+template <bool OBF16>
+__global__ void __launch_bounds__(kFsThreads, 6) k_fwd_short(
+    Grid G, int C, const DenParams* __restrict__ drec, const int* __restrict__ toff,
+    const int* __restrict__ sorted_gauss, int M, const void* __restrict__ features, float* __restrict__ density,
+    void* __restrict__ grid_feats_out, int smax) {
+    __shared__ FsSmem sm;
+>>>>>>> Stashed changes
     const int T = scene_tiles(G);
     const int tb = uniform(xcd_remap(blockIdx.x, gridDim.x));   // the batch's tile (its list)
     if (tb >= T * G.scenes) return;
@@ -464,6 +500,7 @@ __global__ void __launch_bounds__(kFsThreads, 4) k_fwd_short(
     const int Ng = uniform(min(max(toff[tb + 1], j0), M)) - j0;
     if (Ng > smax) return;   // k_fwd_feats takes the tile
     const int scene = uniform(tb / T), tile = tb - scene * T;
+    const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
     {
         const int64_t vb = scene * scene_voxels(G);
         density += vb;
@@ -474,6 +511,7 @@ __global__ void __launch_bounds__(kFsThreads, 4) k_fwd_short(
         return;
     }
     typedef typename std::conditional<OBF16, __bf16, float>::type FT;   // element of the features
+<<<<<<< Updated upstream
     const FT* feats = static_cast<const FT*>(features);
     FT* out = static_cast<FT*>(grid_feats_out);
     const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
@@ -494,6 +532,28 @@ __global__ void __launch_bounds__(kFsThreads, 4) k_fwd_short(
             const int g = sorted_gauss[j0 + min(slot, Ng - 1)];
             frow[s] = feats + (int64_t)g * C;
             const DenParams p = drec[g];
+=======
+    const char* fbase = static_cast<const char*>(features);
+    const int j = lane & 15, q = lane >> 4;
+    const int ns = (Ng + 3) >> 2;
+    int x, y, z;
+    tile_voxel(G, tile, 16 * wave + j, x, y, z);   // the lane's voxel
+    float* wl = &sm.w[wave][0][lane];                // the lane's weight of step s: wl[64 s]
+    uint32_t* offs = &sm.off[wave][q];               // its entry's row of step s: offs[4 s]
+
+    // weights of the lane group's entries 4 s + q and their feature rows (past the list: weight 0, and the
+    // last entry's row again)
+    float D = 0.0f;
+    {
+        const float cx = centre(G, 0, x), cy = centre(G, 1, y), cz = centre(G, 2, z);
+        const int* list = sorted_gauss + j0;
+        int g = list[min(q, Ng - 1)];
+        for (int s = 0; s < ns; ++s) {
+            const DenParams p = drec[g];
+            // the byte offset of the row (the packed rows' 32-bit bound covers it)
+            const uint32_t off = (uint32_t)g * ((uint32_t)C * (uint32_t)sizeof(FT));
+            g = list[min(4 * s + 4 + q, Ng - 1)];   // the next step's entry
+>>>>>>> Stashed changes
             // fwd_column_weights' operations
             const bool inxy = x >= p.lbx && x <= p.ubx && y >= p.lby && y <= p.uby;
             const bool inz = z >= p.lbz && z <= p.ubz;
@@ -502,16 +562,25 @@ __global__ void __launch_bounds__(kFsThreads, 4) k_fwd_short(
             float F = fmaf(fmaf(p.a00, dx, p.a01 * dy), dx, p.a11 * dy * dy);
             F = inxy ? F : -__builtin_inff();
             const float Gxy = fmaf(p.a02, dx, p.a12 * dy);
+<<<<<<< Updated upstream
             const float wv = slot < Ng ? p.o * __builtin_amdgcn_exp2f(fmaf(Gxy, dz, F) + fz) : 0.0f;
             D += wv;
             w[s] = fmaxf(wv, 0.0f);   // feature gate of the reference (.cu:936)
         } else {
             frow[s] = feats;
             w[s] = 0.0f;
+=======
+            const float w = 4 * s + q < Ng ? p.o * __builtin_amdgcn_exp2f(fmaf(Gxy, dz, F) + fz) : 0.0f;
+            D += w;
+            // feature gate of the reference (.cu:936)
+            wl[64 * s] = fmaxf(w, 0.0f);
+            if (j == 0) offs[4 * s] = off;
+>>>>>>> Stashed changes
         }
     }
     D += xor_shfl<16>(D);   // the four lane groups' entries
     D += __shfl_xor(D, 32, 64);
+<<<<<<< Updated upstream
     const bool ok = in_grid(G, x, y, z);
     const int v = ok ? (int)voxel_index(G, x, y, z) : -1;
     if (ok && q == 0) density[v] = D;
@@ -575,8 +644,74 @@ __global__ void __launch_bounds__(kFsThreads, 4) k_fwd_short(
                     const int c = cb + 16 * i + j;
                     if (c < C) row[c] = (FT)(acc[i][r] * rinv[r]);
                 }
-            }
+=======
+    if (q == 0 && in_grid(G, x, y, z)) density[voxel_index(G, x, y, z)] = D;
+    // the lane's result rows: voxels 4 q + i of the slab, i.e. (x, y of the tile + q, z of the tile + i)
+    const int yr = (y & ~(kTile - 1)) + q, zr = z & ~(kTile - 1);
+    const int nz = x < G.dims[0] && yr < G.dims[1] ? min(G.dims[2] - zr, kTile) : 0;   // rows to store
+    FT* orow = static_cast<FT*>(grid_feats_out) + (nz > 0 ? voxel_index(G, x, yr, zr) : 0) * C;
+    float rinv[4];
+    {
+        const float inv = 1.0f / fmaxf(D, kEps);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rinv[i] = __shfl(inv, 4 * q + i, 64);
+    }
+
+    wave_lds_sync();
+
+    // Steps run through the channel blocks in one sequence: the pieces of the next kGrp steps are loaded
+    // before the products of the current ones, across the end of a block too, so that its stores (one
+    // in-order counter with the loads) are not waited for.
+    const bool tail = 4 * (ns - 1) + q >= Ng;   // the lane's entry of the last step lies past the list
+    const int ngr = (ns + kFsGrp - 1) / kFsGrp, nit = ngr * ((C + 63) >> 6);
+    f32x4 f[kFsGrp], fn[kFsGrp];
+    float w[kFsGrp], wn[kFsGrp];
+    auto load = [&](int gr, int cb) {
+#pragma unroll
+        for (int k = 0; k < kFsGrp; ++k) {
+            const int s = gr * kFsGrp + k;
+            wn[k] = wl[64 * min(s, ns - 1)];
+            fn[k] = load4_row(reinterpret_cast<const FT*>(fbase + offs[4 * min(s, ns - 1)]), cb + 4 * j, C);
         }
+    };
+    f32x4 acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    int gr = 0, cb = 0, gn = 0, cn = 0;
+    load(0, 0);
+    for (int it = 0; it < nit; ++it) {
+#pragma unroll
+        for (int k = 0; k < kFsGrp; ++k) {
+            f[k] = fn[k];
+            w[k] = wn[k];
+        }
+        if (++gn == ngr) {
+            gn = 0;
+            cn += 64;
+        }
+        if (it + 1 < nit) load(gn, cn);
+#pragma unroll
+        for (int k = 0; k < kFsGrp; ++k) {
+            const int s = gr * kFsGrp + k;
+            if (s >= ns) break;   // uniform
+            const bool past = tail && s == ns - 1;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)   // an entry past the list reads as zeros
+                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[k], past ? 0.0f : f[k][i], acc[i], 0, 0, 0);
+        }
+        if (gr == ngr - 1) {   // the block's last steps
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (r >= nz) break;
+                const f32x4 o = {acc[0][r] * rinv[r], acc[1][r] * rinv[r], acc[2][r] * rinv[r], acc[3][r] * rinv[r]};
+                store4_row(orow + (int64_t)r * C, cb + 4 * j, C, o);
+>>>>>>> Stashed changes
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        gr = gn;
+        cb = cn;
     }
 }
 
@@ -857,14 +992,24 @@ hipError_t launch_forward_feats(const Grid& G, int C, const int* tile_offsets, c
     G2V_LAUNCH((k_fwd_short<F, V>), dim3(blocks), dim3(kFsThreads), 0, s, G, C, drec, tile_offsets, sorted_gauss, M, \
                features, density, grid_feats, smax)
     if (fdt == kDtBF16) {
+<<<<<<< Updated upstream
         if (vec) G2V_FS(true, true);
         else G2V_FS(true, false);
+=======
+        G2V_LAUNCH(k_fwd_short<true>, dim3(blocks), dim3(kFsThreads), 0, s, G, C, drec, tile_offsets, sorted_gauss, M,
+                   features, density, grid_feats, smax);
+>>>>>>> Stashed changes
         if (nlong > 0)
             G2V_LAUNCH(k_fwd_feats<true>, dim3(lblocks), dim3(kFwdThreads), 0, s, G, C, drec, tile_offsets,
                        sorted_gauss, M, n, Cp, (const uint32_t*)fpk, density, grid_feats, smax, tlist, tcount);
     } else {
+<<<<<<< Updated upstream
         if (vec) G2V_FS(false, true);
         else G2V_FS(false, false);
+=======
+        G2V_LAUNCH(k_fwd_short<false>, dim3(blocks), dim3(kFsThreads), 0, s, G, C, drec, tile_offsets, sorted_gauss, M,
+                   features, density, grid_feats, smax);
+>>>>>>> Stashed changes
         if (nlong > 0)
             G2V_LAUNCH(k_fwd_feats<false>, dim3(lblocks), dim3(kFwdThreads), 0, s, G, C, drec, tile_offsets,
                        sorted_gauss, M, n, Cp, (const uint32_t*)fpk, density, grid_feats, smax, tlist, tcount);
