@@ -435,30 +435,6 @@ __device__ __forceinline__ void fwd_zero_tile(const Grid& G, int tile, int C, fl
 // ------------------------------------------------------------------------------------------
 // Tiles whose list holds at most smax <= kFsMax Gaussians, empty ones included.  k_fwd_feats keeps two
 // tiles per CU (its LDS holds a 256-Gaussian K chunk), so a short list leaves that tile's chain of
-<<<<<<< Updated upstream
-// loads and barriers bare; here a 4-wave workgroup without LDS takes the tile and many run per CU.
-// S = W F on the float32 matrix cores (16x16x4): wave w owns the 16 voxels x = x0 + w, lane l % 16 = voxel,
-// and the lane group q = l / 16 evaluates the weights of the list entries 4 s + q, which are then the A
-// operand of step s as they are (no weight is evaluated twice, none goes through memory).  A lane
-// loads one 16-byte piece of entry 4 s + q's feature row, four channels for the four MFMAs of a
-// 64-channel block, straight from the caller's features; a result row lies in 16 lanes as 64
-// consecutive channels.  Rows whose channels do not make whole 16-byte pieces take single channels, 16
-// consecutive ones per MFMA, so that loads and stores stay in runs of 64 bytes.
-// The weights are those of fwd_build_w (the same operations), the density their sum (in another
-// order), the features float32 sums of max(w, 0) f.  Which kernel takes a tile depends on its list
-// length alone.
-// ------------------------------------------------------------------------------------------
-constexpr int kFsThreads = 256;
-constexpr int kFsMax = 64;          // longest list the kernel can take
-constexpr int kFsSteps = kFsMax / 4;
-
-// VEC: rows of features and grid_feats are whole aligned groups of four channels.
-template <bool OBF16, bool VEC>
-__global__ void __launch_bounds__(kFsThreads, 4) k_fwd_short(
-    Grid G, int C, const DenParams* __restrict__ drec, const int* __restrict__ toff,
-    const int* __restrict__ sorted_gauss, int M, const void* __restrict__ features, float* __restrict__ density,
-    void* __restrict__ grid_feats_out, int smax) {
-=======
 // loads and barriers bare; here a 4-wave workgroup with 17 KB of LDS takes the tile and several
 // run per CU.
 // S = W F on the float32 matrix cores (16x16x4): wave w owns the 16 voxels x = x0 + w, lane l % 16 = voxel,
@@ -492,7 +468,6 @@ __global__ void __launch_bounds__(kFsThreads, 6) k_fwd_short(
     const int* __restrict__ sorted_gauss, int M, const void* __restrict__ features, float* __restrict__ density,
     void* __restrict__ grid_feats_out, int smax) {
     __shared__ FsSmem sm;
->>>>>>> Stashed changes
     const int T = scene_tiles(G);
     const int tb = uniform(xcd_remap(blockIdx.x, gridDim.x));   // the batch's tile (its list)
     if (tb >= T * G.scenes) return;
@@ -511,28 +486,6 @@ __global__ void __launch_bounds__(kFsThreads, 6) k_fwd_short(
         return;
     }
     typedef typename std::conditional<OBF16, __bf16, float>::type FT;   // element of the features
-<<<<<<< Updated upstream
-    const FT* feats = static_cast<const FT*>(features);
-    FT* out = static_cast<FT*>(grid_feats_out);
-    const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
-    const int j = lane & 15, q = lane >> 4;
-    int x, y, z;
-    tile_voxel(G, tile, 16 * wave + j, x, y, z);   // the lane's voxel
-    const float cx = centre(G, 0, x), cy = centre(G, 1, y), cz = centre(G, 2, z);
-    const int ns = (Ng + 3) >> 2;
-
-    // the Gaussians of the lane group's entries 4 s + q (the last entry again past the list)
-    const FT* frow[kFsSteps];
-    float w[kFsSteps];
-    float D = 0.0f;
-#pragma unroll
-    for (int s = 0; s < kFsSteps; ++s) {
-        if (s < ns) {   // uniform
-            const int slot = 4 * s + q;
-            const int g = sorted_gauss[j0 + min(slot, Ng - 1)];
-            frow[s] = feats + (int64_t)g * C;
-            const DenParams p = drec[g];
-=======
     const char* fbase = static_cast<const char*>(features);
     const int j = lane & 15, q = lane >> 4;
     const int ns = (Ng + 3) >> 2;
@@ -553,7 +506,6 @@ __global__ void __launch_bounds__(kFsThreads, 6) k_fwd_short(
             // the byte offset of the row (the packed rows' 32-bit bound covers it)
             const uint32_t off = (uint32_t)g * ((uint32_t)C * (uint32_t)sizeof(FT));
             g = list[min(4 * s + 4 + q, Ng - 1)];   // the next step's entry
->>>>>>> Stashed changes
             // fwd_column_weights' operations
             const bool inxy = x >= p.lbx && x <= p.ubx && y >= p.lby && y <= p.uby;
             const bool inz = z >= p.lbz && z <= p.ubz;
@@ -562,89 +514,15 @@ __global__ void __launch_bounds__(kFsThreads, 6) k_fwd_short(
             float F = fmaf(fmaf(p.a00, dx, p.a01 * dy), dx, p.a11 * dy * dy);
             F = inxy ? F : -__builtin_inff();
             const float Gxy = fmaf(p.a02, dx, p.a12 * dy);
-<<<<<<< Updated upstream
-            const float wv = slot < Ng ? p.o * __builtin_amdgcn_exp2f(fmaf(Gxy, dz, F) + fz) : 0.0f;
-            D += wv;
-            w[s] = fmaxf(wv, 0.0f);   // feature gate of the reference (.cu:936)
-        } else {
-            frow[s] = feats;
-            w[s] = 0.0f;
-=======
             const float w = 4 * s + q < Ng ? p.o * __builtin_amdgcn_exp2f(fmaf(Gxy, dz, F) + fz) : 0.0f;
             D += w;
             // feature gate of the reference (.cu:936)
             wl[64 * s] = fmaxf(w, 0.0f);
             if (j == 0) offs[4 * s] = off;
->>>>>>> Stashed changes
         }
     }
     D += xor_shfl<16>(D);   // the four lane groups' entries
     D += __shfl_xor(D, 32, 64);
-<<<<<<< Updated upstream
-    const bool ok = in_grid(G, x, y, z);
-    const int v = ok ? (int)voxel_index(G, x, y, z) : -1;
-    if (ok && q == 0) density[v] = D;
-    const float inv = 1.0f / fmaxf(D, kEps);
-    float rinv[4];   // of the lane's result rows, voxels 4 q + i of the wave
-    int rv[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        rinv[i] = __shfl(inv, 4 * q + i, 64);
-        rv[i] = __shfl(v, 4 * q + i, 64);
-    }
-
-    const bool tail = 4 * (ns - 1) + q >= Ng;   // the lane's entry of the last step lies past the list
-    for (int cb = 0; cb < C; cb += 64) {
-        f32x4 acc[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        // component i of a lane's four channels: cb + 4 j + i (VEC) or cb + 16 i + j
-        const int c0 = VEC ? min(cb + 4 * j, C - 4) : cb + j;
-#pragma unroll
-        for (int s0 = 0; s0 < kFsSteps; s0 += 4) {
-            if (s0 >= ns) break;   // uniform
-            f32x4 f[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {   // the loads of four steps before their products
-                const int s = s0 + k;
-                if constexpr (VEC) {
-                    f[k] = load4_row(frow[s], c0, C);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) f[k][i] = (float)frow[s][min(c0 + 16 * i, C - 1)];
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int s = s0 + k;
-                if (s >= ns) break;   // uniform
-                const bool past = tail && s == ns - 1;
-#pragma unroll
-                for (int i = 0; i < 4; ++i)   // an entry past the list reads as zeros
-                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[s], past ? 0.0f : f[k][i], acc[i], 0, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (rv[r] < 0) continue;
-            FT* row = out + (int64_t)rv[r] * C;
-            if constexpr (VEC) {
-                if (cb + 4 * j < C) {
-                    const f32x4 o = {acc[0][r] * rinv[r], acc[1][r] * rinv[r], acc[2][r] * rinv[r], acc[3][r] * rinv[r]};
-                    if constexpr (OBF16) {
-                        typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-                        *reinterpret_cast<bf16x4*>(row + cb + 4 * j) = __builtin_convertvector(o, bf16x4);
-                    } else {
-                        __builtin_nontemporal_store(o, reinterpret_cast<f32x4*>(row + cb + 4 * j));
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int c = cb + 16 * i + j;
-                    if (c < C) row[c] = (FT)(acc[i][r] * rinv[r]);
-                }
-=======
     if (q == 0 && in_grid(G, x, y, z)) density[voxel_index(G, x, y, z)] = D;
     // the lane's result rows: voxels 4 q + i of the slab, i.e. (x, y of the tile + q, z of the tile + i)
     const int yr = (y & ~(kTile - 1)) + q, zr = z & ~(kTile - 1);
@@ -705,7 +583,6 @@ __global__ void __launch_bounds__(kFsThreads, 6) k_fwd_short(
                 if (r >= nz) break;
                 const f32x4 o = {acc[0][r] * rinv[r], acc[1][r] * rinv[r], acc[2][r] * rinv[r], acc[3][r] * rinv[r]};
                 store4_row(orow + (int64_t)r * C, cb + 4 * j, C, o);
->>>>>>> Stashed changes
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -985,36 +862,19 @@ hipError_t launch_forward_feats(const Grid& G, int C, const int* tile_offsets, c
         tlist = tl_ws + 1;
     }
     const int lblocks = (int)ceil_div(nlong, 8) * 8;
-    // whole aligned groups of four channels (float: 16 bytes, bfloat16: 8)
-    const uintptr_t am = fdt == kDtBF16 ? 7 : 15;
-    const bool vec = (C & 3) == 0 && ((uintptr_t)features & am) == 0 && ((uintptr_t)grid_feats & am) == 0;
-#define G2V_FS(F, V)                                                                                               \
-    G2V_LAUNCH((k_fwd_short<F, V>), dim3(blocks), dim3(kFsThreads), 0, s, G, C, drec, tile_offsets, sorted_gauss, M, \
-               features, density, grid_feats, smax)
     if (fdt == kDtBF16) {
-<<<<<<< Updated upstream
-        if (vec) G2V_FS(true, true);
-        else G2V_FS(true, false);
-=======
         G2V_LAUNCH(k_fwd_short<true>, dim3(blocks), dim3(kFsThreads), 0, s, G, C, drec, tile_offsets, sorted_gauss, M,
                    features, density, grid_feats, smax);
->>>>>>> Stashed changes
         if (nlong > 0)
             G2V_LAUNCH(k_fwd_feats<true>, dim3(lblocks), dim3(kFwdThreads), 0, s, G, C, drec, tile_offsets,
                        sorted_gauss, M, n, Cp, (const uint32_t*)fpk, density, grid_feats, smax, tlist, tcount);
     } else {
-<<<<<<< Updated upstream
-        if (vec) G2V_FS(false, true);
-        else G2V_FS(false, false);
-=======
         G2V_LAUNCH(k_fwd_short<false>, dim3(blocks), dim3(kFsThreads), 0, s, G, C, drec, tile_offsets, sorted_gauss, M,
                    features, density, grid_feats, smax);
->>>>>>> Stashed changes
         if (nlong > 0)
             G2V_LAUNCH(k_fwd_feats<false>, dim3(lblocks), dim3(kFwdThreads), 0, s, G, C, drec, tile_offsets,
                        sorted_gauss, M, n, Cp, (const uint32_t*)fpk, density, grid_feats, smax, tlist, tcount);
     }
-#undef G2V_FS
     return hipGetLastError();
 }
 
