@@ -56,24 +56,6 @@ __device__ __forceinline__ void write_grads(const float (&gr)[kNumGrads], int g,
     grad_opacity[g] = gr[9];
 }
 
-// Regions of the feature-gradient phase: 2 x 2 tiles in x, y and up to 4 tiles in z.
-struct Regions {
-    int cell[3];   // voxels per region along each axis
-    int n[3];      // region grid
-    int total;
-};
-
-static Regions make_regions(const Grid& G) {
-    Regions R;
-    const int rz = min(G.tiles[2], 4);
-    R.cell[0] = 2 * kTile;
-    R.cell[1] = 2 * kTile;
-    R.cell[2] = rz * kTile;
-    for (int a = 0; a < 3; ++a) R.n[a] = (G.dims[a] + R.cell[a] - 1) / R.cell[a];
-    R.total = R.n[0] * R.n[1] * R.n[2];
-    return R;
-}
-
 // ------------------------------------------------------------------------------------------
 // Density only: one wave per Gaussian walks the voxels of its box.  Per voxel, with d = centre - mu,
 // q = A d and r = gD e, e = exp(-d^T q / 2): the Gaussian's gradients are d mu = o sum r q,
@@ -1400,7 +1382,7 @@ __global__ void __launch_bounds__(kBsThreads, 4) k_bwd_tile_short(
 // Phase B's row table: for every region row (a Gaussian of the region's ascending list) and
 // every tile slot of the region, the Tile->Gaussian entry of that (tile, Gaussian) pair.
 // ------------------------------------------------------------------------------------------
-constexpr int kBrSlots = 16;   // tiles per region (2 x 2 x up to 4), slot ((tx&1)*2 + (ty&1))*RZ + tz%RZ
+constexpr int kBrSlots = kRegionSlots;
 
 // Fills n ints with v (also used where a stream may be captured: no memset nodes).
 __global__ void __launch_bounds__(256) k_fill_i32(int64_t n, int v, int* __restrict__ dst) {
@@ -2102,16 +2084,17 @@ static FeatBufs carve_feats(void* ws, const Grid& G, int n, int C, int64_t M, in
     b.fsp = c.take<__bf16>((int64_t)(n + 1) * feature_chunks(C) * 2 * kBtKc);
     b.partials = c.take<float>(m * kNumGrads);
     b.wt = c.take<__bf16>((m + 1) * kWtRow);   // row M is zero (rows of absent pairs read it)
-    b.r_cells = c.take<int>(mr);
-    b.r_pairs = c.take<int>(mr);
-    b.r_gauss = c.take<int>(mr);
-    b.r_cells_sorted = c.take<int>(mr);
+    const int64_t ms = lists_fit(G, n) ? 1 : mr;   // what only the sorted build holds
+    b.r_cells = c.take<int>(ms);
+    b.r_pairs = c.take<int>(ms);
+    b.r_gauss = c.take<int>(ms);
+    b.r_cells_sorted = c.take<int>(ms);
     b.r_pairs_sorted = c.take<int>(mr);
-    b.r_gids = c.take<int>(mr);
+    b.r_gids = c.take<int>(ms);
     b.table = c.take<int>(mr * kBrSlots);
     const int nreg = RG.total * G.scenes;   // regions of the batch
     b.roff = c.take<int>(nreg + 1);
-    b.sort_ws = c.take<char>(sort_workspace(MR, nreg));
+    b.sort_ws = c.take<char>(lists_fit(G, n) ? lists_workspace(G, n) : sort_workspace(MR, nreg));
     b.gpart = c.take<float>(mr * (C > 0 ? C : 1));
     {   // long-tile list of phase A: a count, then at most min(T, M) tiles
         const int64_t T = (int64_t)scene_tiles(G) * G.scenes;
@@ -2148,6 +2131,11 @@ hipError_t launch_backward_prepare(const Grid& G, int n, int C, const void* feat
     // Region -> Gaussian CSR (pairs carry their G->R slot so partial rows land Gaussian-major) and
     // the row table of phase B
     const int nreg = RG.total * G.scenes;   // regions of the batch: scene b's region r is b R + r
+    const bool lists = lists_fit(G, n);   // built from the boxes; the pairs' buffers are not there
+    if (lists && MR > 0 && M > 0)
+        return launch_region_lists(G, n, lb, ub, pb.g2r_offsets, M, MR, b.roff, b.r_pairs_sorted, b.table,
+                                   reinterpret_cast<int*>(b.wt + M * kWtRow), kWtRow / 2, b.sort_ws, s);
+    if (lists) MR = 0;
     if (MR > 0) {
         e = launch_fill_cells(n, lb, ub, pb.g2r_offsets, RG.cell, RG.n, b.r_cells, b.r_pairs, b.r_gauss, s,
                               G.scenes > 1 ? G.scene_n : 0, RG.total);

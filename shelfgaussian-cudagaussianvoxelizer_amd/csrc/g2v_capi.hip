@@ -79,12 +79,13 @@ SplatBufs carve_splat(void* ws, int n, int64_t M, const Grid& G, int feat_dim = 
     const int T = num_tiles(G);
     Carver c(ws, (size_t)-1);
     SplatBufs b;
-    b.keys = G.scenes > 1 ? c.take<int>(m) : nullptr;
-    b.gauss_ids = c.take<int>(m);
+    const bool lists = lists_fit(G, n);   // the lists come from the boxes: no keys, values or sort buffers
+    b.keys = G.scenes > 1 && !lists ? c.take<int>(m) : nullptr;
+    b.gauss_ids = c.take<int>(lists ? 1 : m);
     b.sorted_tiles = c.take<int>(m);
     b.sorted_gauss = c.take<int>(m);
     b.tile_offsets = c.take<int>(T + 1);
-    b.sort_ws = c.take<char>(sort_workspace(M, T));
+    b.sort_ws = c.take<char>(lists ? lists_workspace(G, n) : sort_workspace(M, T));
     b.fpk = feat_dim > 0 && with_packed ? c.take<uint32_t>((int64_t)(n + 1) * packed_channels(feat_dim)) : nullptr;
     b.tl = feat_dim > 0 ? c.take<int>(long_list_ints(M, T, feat_dim)) : nullptr;
     b.drec = with_records ? c.take<DenParams>(n > 0 ? n : 1) : nullptr;
@@ -92,7 +93,8 @@ SplatBufs carve_splat(void* ws, int n, int64_t M, const Grid& G, int feat_dim = 
     return b;
 }
 
-// G->T gauss ids, stable sort by tile, tile offsets: the Tile->Gaussian CSR.  A batch sorts by
+// The Tile->Gaussian CSR: built from the boxes (lists_fit), or G->T gauss ids, stable sort by tile, tile
+// offsets.  A batch sorts by
 // the batch's tile ids (b.keys, written beside the scene-local g2t_tile_ids_out).  With b.drec, the
 // G->T fill also packs the Gaussians' records (from means, opacity and cov_inv).
 int build_t2g(const Grid& G, int n, const int* lb, const int* ub, const int* g2t_offsets,
@@ -100,6 +102,11 @@ int build_t2g(const Grid& G, int n, const int* lb, const int* ub, const int* g2t
               hipStream_t s, const float* means = nullptr, const float* opacity = nullptr,
               const float* cov_inv = nullptr) {
     const int T = num_tiles(G);
+    if (M > 0 && lists_fit(G, n)) {
+        G2V_HIP(launch_tile_lists(G, n, lb, ub, g2t_offsets, M, g2t_tile_ids_out, means, opacity, cov_inv, b.drec,
+                                  b.sorted_tiles, b.sorted_gauss, b.tile_offsets, b.sort_ws, s));
+        return G2V_OK;
+    }
     if (M > 0) {
         G2V_HIP(launch_fill_g2t(G, n, lb, ub, g2t_offsets, g2t_tile_ids_out, b.gauss_ids, s, b.keys, means, opacity,
                                 cov_inv, b.drec));

@@ -317,19 +317,12 @@ hipError_t scan_i32_pair(const int* in_a, int* out_a, int64_t n_a, long long* to
 // tile_ids keeps the scene-local ids.
 constexpr int kFillLanes = 16;
 
-__global__ void __launch_bounds__(256) k_fill_g2t(Grid G, int n, const int* __restrict__ lb,
-                                                  const int* __restrict__ ub,
-                                                  const int* __restrict__ g2t_offsets,
-                                                  int* __restrict__ tile_ids,
-                                                  int* __restrict__ gauss_ids,
-                                                  int* __restrict__ keys,
-                                                  const float* __restrict__ means,
-                                                  const float* __restrict__ opacity,
-                                                  const float* __restrict__ cov_inv,
-                                                  DenParams* __restrict__ drec) {
-    const int l = threadIdx.x & (kFillLanes - 1);
-    const int g = blockIdx.x * (256 / kFillLanes) + threadIdx.x / kFillLanes;
-    if (g >= n) return;
+__device__ __forceinline__ void fill_g2t(const Grid& G, int g, int l, const int* __restrict__ lb,
+                                         const int* __restrict__ ub, const int* __restrict__ g2t_offsets,
+                                         int* __restrict__ tile_ids, int* __restrict__ gauss_ids,
+                                         int* __restrict__ keys, const float* __restrict__ means,
+                                         const float* __restrict__ opacity, const float* __restrict__ cov_inv,
+                                         DenParams* __restrict__ drec) {
     const int base = g2t_offsets[g];
     const int cnt = g2t_offsets[g + 1] - base;
     if (cnt <= 0) return;
@@ -368,7 +361,7 @@ __global__ void __launch_bounds__(256) k_fill_g2t(Grid G, int n, const int* __re
         const int t = ((tx0 + lx) * G.tiles[1] + (ty0 + ly)) * G.tiles[2] + (tz0 + lz);
         if (tile_ids) tile_ids[base + i] = t;
         if (keys) keys[base + i] = kb + t;
-        gauss_ids[base + i] = g;
+        if (gauss_ids) gauss_ids[base + i] = g;
         lz += sz;
         const int cz = lz >= dz ? 1 : 0;
         lz -= cz * dz;
@@ -377,6 +370,21 @@ __global__ void __launch_bounds__(256) k_fill_g2t(Grid G, int n, const int* __re
         ly -= cy * dy;
         lx += sx + cy;
     }
+}
+
+__global__ void __launch_bounds__(256) k_fill_g2t(Grid G, int n, const int* __restrict__ lb,
+                                                  const int* __restrict__ ub,
+                                                  const int* __restrict__ g2t_offsets,
+                                                  int* __restrict__ tile_ids,
+                                                  int* __restrict__ gauss_ids,
+                                                  int* __restrict__ keys,
+                                                  const float* __restrict__ means,
+                                                  const float* __restrict__ opacity,
+                                                  const float* __restrict__ cov_inv,
+                                                  DenParams* __restrict__ drec) {
+    const int l = threadIdx.x & (kFillLanes - 1);
+    const int g = blockIdx.x * (256 / kFillLanes) + threadIdx.x / kFillLanes;
+    if (g < n) fill_g2t(G, g, l, lb, ub, g2t_offsets, tile_ids, gauss_ids, keys, means, opacity, cov_inv, drec);
 }
 
 hipError_t launch_fill_g2t(const Grid& G, int n, const int* lb, const int* ub,
@@ -761,6 +769,532 @@ hipError_t launch_tile_offsets(const int* sorted_keys, int64_t M, int T, int* ti
     if (T < 0) return hipErrorInvalidValue;
     G2V_LAUNCH(k_tile_offsets, dim3((unsigned)ceil_div((int64_t)T + 1, 256)), dim3(256), 0, s,
                sorted_keys, M, T, tile_offsets);
+    return hipGetLastError();
+}
+
+// ------------------------------------------------------------------------------------------
+// Lists from the boxes.  A tile's list is the ascending sequence of the Gaussians whose box meets it, so
+// it need not be sorted out of the G->T pairs: one workgroup per region (2 x 2 x up to 4 tiles) walks the
+// Gaussians in order, keeps those that reach the region, and one wave per tile picks its own from them by
+// ballot.  The sort moved every pair through memory twice per pass in three dependent launches per pass
+// (eight launches from the fill to the tile offsets, and as many again for the regions, whose row table
+// then searched each pair); here a count, a scan and a fill remain.
+//
+// The Gaussians are walked 64 at a time, a word of hit bits each.  With more than kDirectN per scene a
+// first kernel keeps, for every x row of regions and segment of kSegN Gaussians, those whose box reaches the
+// row, with their region ranges in y and z (rowlist, rowcnt), so that a region walks a few percent of them
+// and gathers no box it does not keep; below, the region walks them all.  The hit words stay in LDS with
+// their running counts; row r of the region is then found by one thread (a search of the counts and the
+// bit's place in its word), so that the kept boxes are gathered by all threads at once however the hits
+// are spread.  The kept Gaussians and the tiles of the region each one reaches (a bit per slot) are laid
+// out in LDS in chunks of kRegRows rows, in list order.
+// ------------------------------------------------------------------------------------------
+constexpr int kSegN = 1024;                 // Gaussians per segment
+constexpr int kSegWords = kSegN / 64;
+constexpr int kMaxWords = 4096;             // hit words that fit in LDS (262,144 Gaussians)
+constexpr int kDirectN = 4096;              // without row lists up to here
+constexpr int kListThreads = 512;
+constexpr int kListWaves = kListThreads / 64;
+constexpr int kRegRows = 2048;              // kept Gaussians laid out in LDS at a time
+constexpr int kRowYBits = 10, kRowZBits = 6;   // region ranges of a row list's entry
+
+static int scene_gaussians(const Grid& G, int n) { return G.scenes > 1 ? G.scene_n : n; }
+
+// The region walks visit a region's share of the Gaussians 64 at a time; the path is taken while the
+// visits of all regions (of a row's, with row lists) stay below kMaxWalk and the row lists below
+// kMaxRowBytes.  Beyond (very many Gaussians or scenes, many regions along y and z), sorting the pairs, whose
+// cost follows their number alone, is the better way.  Kernel time of a density-only step on 200 x 200 x
+// 16 voxels, sorted -> listed: 10,000 Gaussians (3,925 visits) 0.123 -> 0.094 ms, 30,000 0.152 -> 0.128, 60,000
+// (23,450) 0.198 -> 0.193, 90,000 (35,175) 0.239 -> 0.247, 200,000 0.402 -> 0.440; 1.5 x larger Gaussians 60,000
+// 0.413 -> 0.371.  6 scenes of 300 (18,750 visits) gain, 24 scenes (75,000) lose 4 %.
+constexpr int64_t kMaxWalk = 32768;
+constexpr int64_t kMaxRowBytes = int64_t(64) << 20;
+
+bool lists_fit(const Grid& G, int n) {
+    const int ns = scene_gaussians(G, n);
+    if (ns <= 0 || ns > kMaxWords * 64) return false;
+    const Regions RG = make_regions(G);
+    const int64_t visits = ceil_div(ns, 64);
+    if (ns <= kDirectN) return (int64_t)RG.total * G.scenes * visits <= kMaxWalk;
+    return (int64_t)RG.n[1] * RG.n[2] * G.scenes * visits <= kMaxWalk && RG.n[1] <= 1 << kRowYBits &&
+           RG.n[2] <= 1 << kRowZBits && RG.n[0] <= 65535 && G.scenes <= 65535 &&
+           (int64_t)RG.n[0] * G.scenes * ceil_div(ns, kSegN) * kSegN * (int64_t)sizeof(int2) <= kMaxRowBytes;
+}
+
+struct ListBufs {
+    int* tcnt;      // Gaussians per tile of the batch
+    int* rcnt;      // and per region
+    int* toff;      // their offsets (launch_region_lists)
+    int* rowcnt;    // row lists: [scene][row][segment]
+    int2* rowlist;  // [scene][row][segment][kSegN]: Gaussian, packed region ranges
+    void* scan_t;
+    void* scan_r;
+    size_t bytes;
+};
+
+static ListBufs carve_lists(void* ws, const Grid& G, int n) {
+    const Regions RG = make_regions(G);
+    const int ns = scene_gaussians(G, n);
+    const int64_t T = (int64_t)scene_tiles(G) * G.scenes, R = (int64_t)RG.total * G.scenes;
+    const int64_t segs = ns > kDirectN ? (int64_t)RG.n[0] * G.scenes * ceil_div(ns, kSegN) : 0;
+    Carver c(ws, (size_t)-1);
+    ListBufs b;
+    b.tcnt = c.take<int>(T);
+    b.rcnt = c.take<int>(R);
+    b.toff = c.take<int>(T + 1);
+    b.rowcnt = c.take<int>(segs);
+    b.rowlist = c.take<int2>(segs * kSegN);
+    b.scan_t = c.take<char>(scan_workspace(T));
+    b.scan_r = c.take<char>(scan_workspace(R));
+    b.bytes = c.off + 256;
+    return b;
+}
+
+size_t lists_workspace(const Grid& G, int n) { return carve_lists(nullptr, G, n).bytes; }
+
+// Workgroup (segment, x row of regions, scene): the segment's Gaussians whose box reaches the row, in order.
+__global__ void __launch_bounds__(256) k_row_lists(Regions RG, int ns, int nseg, const int* __restrict__ lb,
+                                                   const int* __restrict__ ub, int* __restrict__ rowcnt,
+                                                   int2* __restrict__ rowlist) {
+    constexpr int kIts = kSegN / 256;
+    __shared__ int cnt[kIts * 4];
+    const int seg = blockIdx.x, row = blockIdx.y, scene = blockIdx.z;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int x0 = row * RG.cell[0], x1 = x0 + RG.cell[0] - 1;
+    const int g0 = scene * ns + seg * kSegN, cntg = min(kSegN, ns - seg * kSegN);
+    int l[kIts][3], u[kIts][3];
+#pragma unroll
+    for (int i = 0; i < kIts; ++i) {   // every load before any is used
+        const int64_t k = 3 * (int64_t)(g0 + min(i * 256 + (int)threadIdx.x, cntg - 1));
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            l[i][a] = lb[k + a];
+            u[i][a] = ub[k + a];
+        }
+    }
+    unsigned long long m[kIts];
+#pragma unroll
+    for (int i = 0; i < kIts; ++i) {
+        // an empty box (0, -1) reaches no row
+        m[i] = __ballot(i * 256 + (int)threadIdx.x < cntg && l[i][0] <= x1 && u[i][0] >= x0);
+        if (lane == 0) cnt[i * 4 + wave] = __popcll(m[i]);
+    }
+    __syncthreads();
+    const int64_t out = ((int64_t)scene * gridDim.y + row) * nseg + seg;
+    int base = 0;
+#pragma unroll
+    for (int i = 0; i < kIts; ++i) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            if (w == wave && ((m[i] >> lane) & 1ull)) {
+                const unsigned r = (unsigned)(l[i][1] / RG.cell[1]) | (unsigned)(u[i][1] / RG.cell[1]) << kRowYBits |
+                                   (unsigned)(l[i][2] / RG.cell[2]) << (2 * kRowYBits) |
+                                   (unsigned)(u[i][2] / RG.cell[2]) << (2 * kRowYBits + kRowZBits);
+                rowlist[out * kSegN + base + __popcll(m[i] & ((1ull << lane) - 1ull))] =
+                    make_int2(g0 + i * 256 + (int)threadIdx.x, (int)r);
+            }
+            base += cnt[i * 4 + w];
+        }
+    }
+    if (threadIdx.x == 0) rowcnt[out] = base;
+}
+
+template <int WORDS>
+struct ListSmem {
+    unsigned long long mask[WORDS];       // hit words
+    int pre[WORDS];                       // hits before each word
+    int rg[kRegRows];                     // kept Gaussians of the chunk
+    unsigned short rm[kRegRows];          // and the region's tiles they reach
+    int tab[64][kRegionSlots + 1];
+    int wsum[5][kListWaves];
+};
+
+enum ListMode { kListCount, kListTiles, kListTable };
+
+// What the modes write: kListCount the lists' lengths (tcnt, rcnt); kListTiles every tile's list at
+// toff[tile] (sorted_gauss, and sorted_tiles when not null); kListTable, per region row (at roff[region]),
+// its G->R slot and the T->G index of its pair with every tile slot of the region (M: no pair).
+struct ListOut {
+    int* tcnt;
+    int* rcnt;
+    int* first[2];   // kListCount: cleared (the offsets' leading zeros)
+    int* zero;       // and zero[0 .. nzero)
+    int nzero;
+    int* toff;
+    int* sorted_tiles;
+    int* sorted_gauss;
+    int* roff;
+    int own;         // the workgroups sum the counts before their tiles (toff) and region (roff) themselves
+    const int* g2r_offsets;
+    int* r_pairs;
+    int* table;
+    int M, MR;
+};
+
+// The G->T fill that rides on a kListCount launch: workgroups past the regions take its Gaussians.
+struct FillJob {
+    int n;
+    const int* g2t_offsets;
+    int* tile_ids;
+    const float* means;
+    const float* opacity;
+    const float* cov_inv;
+    DenParams* drec;
+};
+
+// DIRECT: no row lists, at most kDirectN Gaussians per scene.
+template <ListMode MODE, bool DIRECT>
+__global__ void __launch_bounds__(kListThreads) k_region_lists(Grid G, Regions RG, int ns, int nseg,
+                                                               const int* __restrict__ lb, const int* __restrict__ ub,
+                                                               const int* __restrict__ rowcnt,
+                                                               const int2* __restrict__ rowlist, ListOut o, FillJob f) {
+    constexpr int kWords = DIRECT ? kDirectN / 64 : kMaxWords;
+    __shared__ ListSmem<kWords> sm;
+    const int Rb = blockIdx.x;   // the batch's region
+    if (MODE == kListCount && Rb >= RG.total * G.scenes) {
+        const int g = (Rb - RG.total * G.scenes) * (kListThreads / kFillLanes) + threadIdx.x / kFillLanes;
+        if (g < f.n)
+            fill_g2t(G, g, threadIdx.x & (kFillLanes - 1), lb, ub, f.g2t_offsets, f.tile_ids, nullptr, nullptr, f.means,
+                     f.opacity, f.cov_inv, f.drec);
+        return;
+    }
+    if (MODE == kListCount && Rb == 0) {
+        if (threadIdx.x < 2 && o.first[threadIdx.x]) *o.first[threadIdx.x] = 0;
+        if ((int)threadIdx.x < o.nzero) o.zero[threadIdx.x] = 0;
+    }
+    const int scene = Rb / RG.total, R = Rb - scene * RG.total;
+    const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
+    const int rnyz = RG.n[1] * RG.n[2];
+    const int rx = R / rnyz, ry = (R - rx * rnyz) / RG.n[2], rz = R % RG.n[2];
+    const int x0 = rx * RG.cell[0], y0 = ry * RG.cell[1], z0 = rz * RG.cell[2];
+    const int x1 = x0 + RG.cell[0] - 1, y1 = y0 + RG.cell[1] - 1, z1 = z0 + RG.cell[2] - 1;
+    const int tpz = RG.cell[2] / kTile, nslot = 4 * tpz;
+    // words of the walk: 64 consecutive Gaussians of the scene, or of a segment's row list
+    const int64_t row = ((int64_t)scene * RG.n[0] + rx) * nseg;   // the region's row lists
+    const int nwords = DIRECT ? (ns + 63) >> 6 : nseg * kSegWords;
+
+    // the walk, four words' loads at a time
+    if constexpr (!DIRECT) {   // wave w takes segments w, w + kListWaves, ...; the next one's first loads run ahead
+        for (int w = threadIdx.x; w < nwords; w += kListThreads) sm.mask[w] = 0;
+        __syncthreads();
+        int n_e = 0;
+        int2 e[4];
+        auto load = [&](int s, int i0, int2 (&v)[4]) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = rowlist[(row + s) * kSegN + min(i0 + 64 * k + lane, kSegN - 1)];
+        };
+        if (wave < nseg) {
+            n_e = uniform(rowcnt[row + wave]);
+            load(wave, 0, e);
+        }
+        for (int s = wave; s < nseg; s += kListWaves) {
+            const int sn = s + kListWaves;
+            int n_n = 0;
+            int2 en[4] = {};
+            if (sn < nseg) {
+                n_n = uniform(rowcnt[row + sn]);
+                load(sn, 0, en);
+            }
+#pragma unroll 1
+            for (int i0 = 0; i0 < n_e; i0 += 256) {
+                if (i0 > 0) load(s, i0, e);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    constexpr unsigned ym = (1u << kRowYBits) - 1, zm = (1u << kRowZBits) - 1;
+                    const unsigned r = (unsigned)e[k].y;   // past the list: whatever the slot holds, not used
+                    const unsigned long long m =
+                        __ballot(i0 + 64 * k + lane < n_e && (r & ym) <= (unsigned)ry && ((r >> kRowYBits) & ym) >= (unsigned)ry &&
+                                 ((r >> (2 * kRowYBits)) & zm) <= (unsigned)rz &&
+                                 ((r >> (2 * kRowYBits + kRowZBits)) & zm) >= (unsigned)rz);
+                    if (lane == 0) sm.mask[s * kSegWords + (i0 >> 6) + k] = m;
+                }
+            }
+            n_e = n_n;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) e[k] = en[k];
+        }
+    } else {
+        for (int w0 = 4 * wave; w0 < nwords; w0 += 4 * kListWaves) {
+            int l[4][3], u[4][3];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int64_t g = 3 * (int64_t)(scene * ns + min((w0 + k) * 64 + lane, ns - 1));
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    l[k][a] = lb[g + a];
+                    u[k][a] = ub[g + a];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const unsigned long long m =
+                    __ballot((w0 + k) * 64 + lane < ns && l[k][0] <= x1 && u[k][0] >= x0 && l[k][1] <= y1 &&
+                             u[k][1] >= y0 && l[k][2] <= z1 && u[k][2] >= z0);
+                if (lane == 0 && w0 + k < nwords) sm.mask[w0 + k] = m;
+            }
+        }
+    }
+    __syncthreads();
+    // hits before each word: thread t takes words kPer t .. kPer t + kPer - 1
+    constexpr int kPer = (kWords + kListThreads - 1) / kListThreads;
+    {
+        int sum = 0, v[kPer];
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int w = threadIdx.x * kPer + k;
+            v[k] = w < nwords ? __popcll(sm.mask[w]) : 0;
+            sum += v[k];
+        }
+        int x = sum;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int t = __shfl_up(x, off, 64);
+            if (lane >= off) x += t;
+        }
+        if (lane == 63) sm.wsum[0][wave] = x;
+        __syncthreads();
+        int run = x - sum;
+        for (int w = 0; w < wave; ++w) run += sm.wsum[0][w];
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const int w = threadIdx.x * kPer + k;
+            if (w < nwords) sm.pre[w] = run;
+            run += v[k];
+        }
+    }
+    int KR = 0;
+#pragma unroll
+    for (int w = 0; w < kListWaves; ++w) KR += sm.wsum[0][w];
+    KR = uniform(KR);
+    __syncthreads();
+    // this wave's tile slots wave and wave + kListWaves: tile id, or -1 outside the grid
+    int tid[2], run[2] = {0, 0};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int slot = wave + kListWaves * h, ab = slot / tpz, cz = slot - ab * tpz;
+        const int tx = 2 * rx + (ab >> 1), ty = 2 * ry + (ab & 1), tz = rz * tpz + cz;
+        const bool in = slot < nslot && tx < G.tiles[0] && ty < G.tiles[1] && tz < G.tiles[2];
+        tid[h] = in ? scene * scene_tiles(G) + (tx * G.tiles[1] + ty) * G.tiles[2] + tz : -1;
+        if (MODE != kListCount && !o.own && in) run[h] = o.toff[tid[h]];
+    }
+    int r0 = MODE == kListTable && !o.own ? o.roff[Rb] : 0;
+    if (MODE != kListCount && o.own) {
+        // the counts before the region's four tile columns and before the region, summed here (a launch
+        // that scanned them would take longer than every workgroup reading them)
+        const int TB = scene_tiles(G) * G.scenes;
+        int first[4], sum[5] = {0, 0, 0, 0, 0};
+        int last = 0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {   // a column outside the grid: any value
+            const int tx = min(2 * rx + (c >> 1), G.tiles[0] - 1), ty = min(2 * ry + (c & 1), G.tiles[1] - 1);
+            first[c] = scene * scene_tiles(G) + (tx * G.tiles[1] + ty) * G.tiles[2] + rz * tpz;
+            last = max(last, first[c]);
+        }
+#pragma unroll 4
+        for (int i = threadIdx.x; i < last; i += kListThreads) {
+            const int v = o.tcnt[i];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) sum[c] += i < first[c] ? v : 0;
+        }
+        if (MODE == kListTable)
+            for (int i = threadIdx.x; i < Rb; i += kListThreads) sum[4] += o.rcnt[i];
+#pragma unroll
+        for (int c = 0; c < 5; ++c) {
+            int v = sum[c];
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+            if (lane == 0) sm.wsum[c][wave] = v;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int slot = wave + kListWaves * h, ab = min(slot / tpz, 3), cz = slot - ab * tpz;
+            int v = 0;
+#pragma unroll
+            for (int w = 0; w < kListWaves; ++w) v += sm.wsum[ab][w];
+            if (tid[h] >= 0) {
+                for (int k = 1; k <= cz; ++k) v += o.tcnt[tid[h] - k];
+                run[h] = v;
+                if (MODE == kListTiles && lane == 0) o.toff[tid[h]] = v;
+            }
+        }
+        if (MODE == kListTable) {
+#pragma unroll
+            for (int w = 0; w < kListWaves; ++w) r0 += sm.wsum[4][w];
+            if (threadIdx.x == 0) {
+                o.roff[Rb] = r0;
+                if (Rb == RG.total * G.scenes - 1) o.roff[Rb + 1] = r0 + KR;
+            }
+        }
+        if (MODE == kListTiles && Rb == 0 && threadIdx.x == 0) o.toff[TB] = o.M;
+    }
+    r0 = min(max(r0, 0), o.MR);
+    for (int c0 = 0; c0 < KR; c0 += kRegRows) {
+        for (int p = threadIdx.x; p < min(kRegRows, KR - c0); p += kListThreads) {
+            // row c0 + p: the last word with at most that many hits before it, and the word's bit
+            int lo = 0, hi = nwords - 1;
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) >> 1;
+                if (sm.pre[mid] <= c0 + p) lo = mid;
+                else hi = mid - 1;
+            }
+            unsigned long long m = sm.mask[lo];
+            int k = c0 + p - sm.pre[lo], bit = 0;   // the k-th set bit of m
+#pragma unroll
+            for (int half = 32; half > 0; half >>= 1) {
+                const int c = __popcll(m & ((1ull << half) - 1ull));
+                if (k >= c) {
+                    k -= c;
+                    bit += half;
+                    m >>= half;
+                }
+            }
+            const int i = lo * 64 + bit;   // segment i / kSegN, entry i % kSegN of it; or Gaussian i of the scene
+            const int g = DIRECT ? scene * ns + i : rowlist[row * kSegN + i].x;
+            int l[3], u[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                l[a] = lb[3 * (int64_t)g + a];
+                u[a] = ub[3 * (int64_t)g + a];
+            }
+            unsigned zm = 0, bits = 0;
+            for (int c = 0; c < tpz; ++c) zm |= (l[2] <= z0 + 4 * c + 3 && u[2] >= z0 + 4 * c) ? 1u << c : 0u;
+#pragma unroll
+            for (int ab = 0; ab < 4; ++ab) {
+                const int xs = x0 + 4 * (ab >> 1), ys = y0 + 4 * (ab & 1);
+                if (l[0] <= xs + 3 && u[0] >= xs && l[1] <= ys + 3 && u[1] >= ys) bits |= zm << (ab * tpz);
+            }
+            sm.rg[p] = g;
+            sm.rm[p] = (unsigned short)bits;
+            if (MODE == kListTable && r0 + c0 + p < o.MR) {
+                // the row's G->R slot: this region's place in the Gaussian's region box
+                const int ax = l[0] / RG.cell[0], ay = l[1] / RG.cell[1], az = l[2] / RG.cell[2];
+                const int ey = u[1] / RG.cell[1] - ay + 1, ez = u[2] / RG.cell[2] - az + 1;
+                o.r_pairs[r0 + c0 + p] = o.g2r_offsets[g] + ((rx - ax) * ey + (ry - ay)) * ez + (rz - az);
+            }
+        }
+        __syncthreads();
+        const int nr = min(kRegRows, KR - c0);
+        for (int i0 = 0; i0 < nr; i0 += 64) {
+            const int i = min(i0 + lane, nr - 1);
+            const unsigned bits = i0 + lane < nr ? sm.rm[i] : 0u;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int slot = wave + kListWaves * h;
+                const unsigned long long m = __ballot((bits >> slot) & 1u);
+                const int p = run[h] + __popcll(m & ((1ull << lane) - 1ull));
+                const bool mine = ((bits >> slot) & 1u) && tid[h] >= 0 && p < o.M;   // inside the lists whatever the boxes
+                if (MODE == kListTiles && mine) {
+                    o.sorted_gauss[p] = sm.rg[i];
+                    if (o.sorted_tiles) o.sorted_tiles[p] = tid[h];
+                }
+                if (MODE == kListTable) sm.tab[lane][slot] = mine ? p : o.M;
+                run[h] += __popcll(m);
+            }
+            if (MODE == kListTable) {   // the 64 rows' table entries, whole rows at a time
+                __syncthreads();
+                const int64_t first = (int64_t)(r0 + c0 + i0) * kRegionSlots;
+#pragma unroll
+                for (int k = 0; k < 64 * kRegionSlots / kListThreads; ++k) {
+                    const int e = threadIdx.x + k * kListThreads, rr = e / kRegionSlots;
+                    if (i0 + rr < nr && r0 + c0 + i0 + rr < o.MR) o.table[first + e] = sm.tab[rr][e % kRegionSlots];
+                }
+                __syncthreads();
+            }
+        }
+        __syncthreads();   // the rows are read
+    }
+    if (MODE == kListCount) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            if (lane == 0 && tid[h] >= 0) o.tcnt[tid[h]] = run[h];
+        if (threadIdx.x == 0) o.rcnt[Rb] = KR;
+    }
+}
+
+// Up to this many tiles of the batch, the list kernels sum the counts before their tiles themselves.
+constexpr int kOwnScanTiles = 16384;
+
+template <ListMode MODE>
+static void run_region_lists(const Grid& G, const Regions& RG, int n, const int* lb, const int* ub, const ListBufs& b,
+                             const ListOut& o, const FillJob& f, hipStream_t s) {
+    const int ns = scene_gaussians(G, n), nseg = (int)ceil_div(ns, kSegN);
+    const dim3 grid((unsigned)(RG.total * G.scenes + ceil_div(f.n, kListThreads / kFillLanes)));
+    if (ns <= kDirectN)
+        G2V_LAUNCH((k_region_lists<MODE, true>), grid, dim3(kListThreads), 0, s, G, RG, ns, nseg, lb, ub, nullptr,
+                   nullptr, o, f);
+    else
+        G2V_LAUNCH((k_region_lists<MODE, false>), grid, dim3(kListThreads), 0, s, G, RG, ns, nseg, lb, ub,
+                   (const int*)b.rowcnt, (const int2*)b.rowlist, o, f);
+}
+
+// The lengths of all lists (b.tcnt, b.rcnt) and, beyond kOwnScanTiles (own false), their offsets toff (T + 1) and,
+// when not null, roff (R + 1); zero[0 .. nzero) is cleared beside them.
+static hipError_t list_offsets(const Grid& G, const Regions& RG, int n, const int* lb, const int* ub, const ListBufs& b,
+                               const FillJob& f, int* toff, int* roff, int* zero, int nzero, bool& own, hipStream_t s) {
+    if (nzero > kListThreads) return hipErrorInvalidValue;
+    const int ns = scene_gaussians(G, n), nseg = (int)ceil_div(ns, kSegN);
+    const int R = RG.total * G.scenes, T = scene_tiles(G) * G.scenes;
+    own = T <= kOwnScanTiles;
+    if (ns > kDirectN)
+        G2V_LAUNCH(k_row_lists, dim3(nseg, RG.n[0], G.scenes), dim3(256), 0, s, RG, ns, nseg, lb, ub, b.rowcnt,
+                   b.rowlist);
+    ListOut o{};
+    o.tcnt = b.tcnt;
+    o.rcnt = b.rcnt;
+    o.first[0] = own ? nullptr : toff;
+    o.first[1] = own ? nullptr : roff;
+    o.zero = zero;
+    o.nzero = nzero;
+    run_region_lists<kListCount>(G, RG, n, lb, ub, b, o, f, s);
+    if (own) return hipGetLastError();
+    // inclusive scans behind a leading zero
+    return scan_i32_pair(b.tcnt, toff + 1, T, nullptr, b.scan_t, b.rcnt, roff ? roff + 1 : nullptr, roff ? R : 0, nullptr,
+                         b.scan_r, s);
+}
+
+hipError_t launch_tile_lists(const Grid& G, int n, const int* lb, const int* ub, const int* g2t_offsets, int64_t M,
+                             int* tile_ids, const float* means, const float* opacity, const float* cov_inv,
+                             DenParams* drec, int* sorted_tiles, int* sorted_gauss, int* toff, void* ws,
+                             hipStream_t s) {
+    if (drec && (!means || !opacity || !cov_inv)) return hipErrorInvalidValue;
+    const Regions RG = make_regions(G);
+    const ListBufs b = carve_lists(ws, G, n);
+    const FillJob f{tile_ids || drec ? n : 0, g2t_offsets, tile_ids, means, opacity, cov_inv, drec};
+    bool own = false;
+    const hipError_t e = list_offsets(G, RG, n, lb, ub, b, f, toff, nullptr, nullptr, 0, own, s);
+    if (e != hipSuccess) return e;
+    ListOut o{};
+    o.tcnt = b.tcnt;
+    o.toff = toff;
+    o.own = own;
+    o.sorted_tiles = sorted_tiles;
+    o.sorted_gauss = sorted_gauss;
+    o.M = (int)M;
+    run_region_lists<kListTiles>(G, RG, n, lb, ub, b, o, FillJob{}, s);
+    return hipGetLastError();
+}
+
+hipError_t launch_region_lists(const Grid& G, int n, const int* lb, const int* ub, const int* g2r_offsets, int64_t M,
+                               int64_t MR, int* roff, int* r_pairs, int* table, int* wt_zero, int wt_zero_ints,
+                               void* ws, hipStream_t s) {
+    const Regions RG = make_regions(G);
+    const ListBufs b = carve_lists(ws, G, n);
+    bool own = false;
+    const hipError_t e = list_offsets(G, RG, n, lb, ub, b, FillJob{}, b.toff, roff, wt_zero, wt_zero_ints, own, s);
+    if (e != hipSuccess) return e;
+    ListOut o{};
+    o.tcnt = b.tcnt;
+    o.rcnt = b.rcnt;
+    o.toff = b.toff;
+    o.roff = roff;
+    o.own = own;
+    o.g2r_offsets = g2r_offsets;
+    o.r_pairs = r_pairs;
+    o.table = table;
+    o.M = (int)M;
+    o.MR = (int)MR;
+    run_region_lists<kListTable>(G, RG, n, lb, ub, b, o, FillJob{}, s);
     return hipGetLastError();
 }
 

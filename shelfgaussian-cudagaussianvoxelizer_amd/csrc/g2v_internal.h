@@ -24,15 +24,34 @@ struct Carver {
     bool fits() const { return off <= cap; }
 };
 
+inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
 // ---- CSR build (g2v_csr.hip) ------------------------------------------------------------
+// Regions: 2 x 2 tiles in x, y and up to 4 tiles in z (the feature-gradient phase's work units, and the
+// coarse boxes by which the tile lists are built).
+struct Regions {
+    int cell[3];   // voxels per region along each axis
+    int n[3];      // region grid
+    int total;
+};
+inline Regions make_regions(const Grid& G) {
+    Regions R;
+    const int rz = G.tiles[2] < 4 ? G.tiles[2] : 4;
+    R.cell[0] = 2 * kTile;
+    R.cell[1] = 2 * kTile;
+    R.cell[2] = rz * kTile;
+    for (int a = 0; a < 3; ++a) R.n[a] = (G.dims[a] + R.cell[a] - 1) / R.cell[a];
+    R.total = R.n[0] * R.n[1] * R.n[2];
+    return R;
+}
+constexpr int kRegionSlots = 16;   // tiles per region, slot ((tx&1)*2 + (ty&1))*RZ + tz%RZ
+
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 16;
 constexpr int kScanTile = kScanThreads * kScanItems;
 constexpr int kSortThreads = 256;
 constexpr int kSortRounds = 16;
 constexpr int kSortTile = kSortThreads * kSortRounds;
-
-inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 size_t scan_workspace(int64_t n);
 // In-place or out-of-place scan of n int32 values (inclusive or exclusive); the int64 total
@@ -81,6 +100,23 @@ hipError_t launch_tile_offsets(const int* sorted_keys, int64_t M, int T, int* ti
                                hipStream_t s);
 hipError_t launch_rle(const int* tile_offsets, int T, int* unique_tiles, int* counts,
                       int* runs_offsets, int* num_runs, void* ws, hipStream_t s);
+
+// Tile and region lists straight from the boxes, without a sort (see k_region_lists).  lists_fit: whether
+// this problem takes that path (else the G->T or G->R pairs are sorted).
+bool lists_fit(const Grid& G, int n);
+size_t lists_workspace(const Grid& G, int n);
+// The Tile->Gaussian CSR of M pairs: tile offsets, Gaussians (and tiles, when not null) in tile order.  The
+// launch also fills tile_ids (when not null) and drec as launch_fill_g2t does.
+hipError_t launch_tile_lists(const Grid& G, int n, const int* lb, const int* ub, const int* g2t_offsets, int64_t M,
+                             int* tile_ids, const float* means, const float* opacity, const float* cov_inv,
+                             DenParams* drec, int* sorted_tiles, int* sorted_gauss, int* toff, void* ws,
+                             hipStream_t s);
+// The Region->Gaussian CSR of MR pairs (offsets roff, each row's G->R slot r_pairs) and phase B's row table:
+// entry (row, tile slot) is the T->G index of the pair, M when the Gaussian does not touch the tile;
+// wt_zero[0 .. wt_zero_ints) is cleared (the weights' zero row).
+hipError_t launch_region_lists(const Grid& G, int n, const int* lb, const int* ub, const int* g2r_offsets, int64_t M,
+                               int64_t MR, int* roff, int* r_pairs, int* table, int* wt_zero, int wt_zero_ints,
+                               void* ws, hipStream_t s);
 
 // The tiles whose list holds more than smax Gaussians (of the M pairs of T tiles), compacted into
 // list[0 .. *count), in unspecified order; count is zeroed first.  cap >= long_tiles_bound(...).
