@@ -244,13 +244,14 @@ __global__ void __launch_bounds__(256) k_split_chunks(const T* __restrict__ src,
 // ------------------------------------------------------------------------------------------
 // Phase A: tile-major U, t_v, gw, geometric partials, split weights.
 // ------------------------------------------------------------------------------------------
-constexpr int kBtThreads = 512;                        // 8 waves
+constexpr int kBtThreads = 256;                        // 4 waves
 constexpr int kBtWaves = kBtThreads / 64;
-constexpr int kBtGroups = 4;                           // Gaussian groups (wave >> 1)
 constexpr int kBtNbw = 2;                              // 32-Gaussian N blocks per wave per pass
-constexpr int kBtPass = kBtGroups * kBtNbw * 32;       // 256 Gaussians per pass
-constexpr int kBtStages = 3;                           // F chunks resident in LDS (loaded 2 ahead)
-constexpr int kBtDma = kBtPass / 8 / kBtWaves;         // 1 KB direct-to-LDS loads per wave per chunk
+constexpr int kBtPass = kBtWaves * kBtNbw * 32;        // 256 Gaussians per pass
+constexpr int kBtStages = 2;                           // F chunks resident in LDS (loaded 1 ahead)
+constexpr int kBtRows = 1024 / kBtRowBytes;            // rows of one 1 KB direct-to-LDS load
+constexpr int kBtDma = kBtPass / kBtRows / kBtWaves;   // such loads per wave per chunk of F
+constexpr int kBtGRows = 64 / kBtWaves;                // voxel rows whose G a wave loads and splits
 constexpr int kWtRow = 128;                            // bf16 per pair: 64 hi then 64 lo
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
@@ -268,71 +269,36 @@ __device__ __forceinline__ int swz(int r) { return (r ^ (r >> 3)) & 7; }
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
     return (uint32_t)(uintptr_t)(lds_ptr_t)p;
 }
-__device__ __forceinline__ void dma16(const void* gptr, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                 :: "v"(gptr), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(const void* gptr, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
-                 :: "v"(gptr), "s"(lds) : "memory", "m0");
-}
 // Scalar-base forms: the wave-uniform base in SGPRs and a 32-bit per-lane byte offset, so that a
 // chunk's advance is scalar work and the per-lane offsets stay fixed across the chunk loop.
 __device__ __forceinline__ void dma16s(const void* sbase, uint32_t voff, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :: "v"(voff), "s"(sbase), "s"(lds) : "memory", "m0");
 }
-__device__ __forceinline__ void dma16s_nt(const void* sbase, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
-                 :: "v"(voff), "s"(sbase), "s"(lds) : "memory", "m0");
-}
-// Streaming variants (non-temporal): for data read once, so that it does not evict the feature
-// rows that many tiles re-read.
-__device__ __forceinline__ void dma16_nt(const void* gptr, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
-                 :: "v"(gptr), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ void dma4_nt(const void* gptr, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off nt"
-                 :: "v"(gptr), "s"(lds) : "memory", "m0");
-}
-
 // FU: the upstream feature gradient is the cosine loss's, G = k1 target + k2 grid_feats per voxel,
-// formed on chip from two raw chunks (target and grid_feats) per stage; the F rows then use two
-// buffers (loaded one chunk ahead) so that the second raw chunk fits.
+// formed on chip from the target and grid_feats.
 template <bool FU>
 struct BtSmem {
-    static constexpr int kFStages = FU ? 2 : kBtStages;   // F chunk buffers
-    static constexpr int kSrc = FU ? 2 : 1;               // raw G sources per stage
     union {
-        // F chunk rows of the pass's Gaussians; the 16-byte piece q of row r sits at slot
-        // q ^ swz(r), so that the lanes of one LDS cycle (8 or 16 consecutive rows) hit distinct
-        // 16-byte bank groups
-        unsigned char frow[kFStages][kBtPass * kBtRowBytes];
-        float xch[2][kBtPass][kNumGrads];   // epilogue exchange, used after the K loop has drained
         struct {
-            float xch_room[2][kBtPass][kNumGrads];
-            // the exponentials of epilogue 1, read again by epilogue 2: [wave][N block][q4][lane]
-            // (FU: no room beside the two F buffers; epilogue 2 evaluates them again)
-            float4 e[FU ? 1 : kBtWaves][kBtNbw][4][64];
-        } ep;
-    } u;
-    // G chunks as loaded (fp32, voxel-major, pieces at q ^ swz(v)); FU: [0] target, [1] grid_feats
-    float graw[kBtStages][kSrc][64][kBtKc];
-    bf16x8 ahi[2][2][2][64];   // A operand (G chunk), hi: [buffer][k half][voxel block][lane]
-    bf16x8 alo[2][2][2][64];
+            // F chunk rows of the pass's Gaussians; the 16-byte piece q of row r sits at slot
+            // q ^ swz(r), so that the lanes of one LDS cycle (8 or 16 consecutive rows) hit distinct
+            // 16-byte bank groups
+            unsigned char frow[kBtStages][kBtPass * kBtRowBytes];
+            // A operand (G of one k half of a chunk), hi and lo: [k half][voxel block][lane]
+            bf16x8 ahi[2][2][64];
+            bf16x8 alo[2][2][64];
+        };
+        // the exponentials of epilogue 1, read again by epilogue 2: [wave][voxel block][N block][q4][lane]
+        float4 e[kBtWaves][2][kBtNbw][4][64];
+    };
     int vlin[64];
     float gD[64], inv[64], tv[64], D[64];
     float kc[2][FU ? 64 : 1];  // FU: the voxel's k1, k2 (scaled by the loss's upstream gradient)
-    ParamTile<kBtPass> pt;     // parameters of this pass's list entries
-    int pidx[kBtPass];         // G->T pair of each entry with this tile (-1: none)
-    float tpart[kBtGroups][64];
+    float tpart[kBtWaves][64];
 };
-static_assert(sizeof(float) * 2 * kBtNbw * 16 * 64 * kBtGroups <= BtSmem<true>::kFStages * kBtPass * kBtRowBytes,
-              "the k-half exchange fits in the F buffers");
-static_assert(sizeof(BtSmem<false>::u) == sizeof(BtSmem<false>::u.frow) && sizeof(BtSmem<true>::u) == sizeof(BtSmem<true>::u.frow),
-              "the epilogue's exponentials fit in the F buffers");
-
+static_assert(sizeof(BtSmem<false>::e) <= sizeof(BtSmem<false>::frow), "the epilogue's exponentials take the F rows' place");
+static_assert(sizeof(BtSmem<false>) <= 80 * 1024 && sizeof(BtSmem<true>) <= 80 * 1024, "two workgroups per CU");
 
 // s_waitcnt immediate that waits for vmcnt <= n and leaves the other counters alone.
 __device__ constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
@@ -383,19 +349,38 @@ struct LaneExp {
 
 // Contraction is off in these helpers, so that every phase A instantiation that inlines them
 // computes the same e (and so the same split weights) for the same pair, whatever the code around.
-__device__ __forceinline__ void lane_exp(const GaussParams& p, const LaneGeom& L, LaneExp& E) {
+struct SymA {   // what a quadratic form needs of A: the diagonal and the off-diagonal sums
+    float xx, yy, zz, xy, xz, yz;
+};
+
+__device__ __forceinline__ void sym_a(const GaussParams& p, SymA& A) {
 #pragma clang fp contract(off)
-    const float sxy = p.A[1] + p.A[3], sxz = p.A[2] + p.A[6], syz = p.A[5] + p.A[7];
+    A.xx = p.A[0];
+    A.yy = p.A[4];
+    A.zz = p.A[8];
+    A.xy = p.A[1] + p.A[3];
+    A.xz = p.A[2] + p.A[6];
+    A.yz = p.A[5] + p.A[7];
+}
+
+__device__ __forceinline__ void lane_exp(const SymA& A, const LaneGeom& L, LaneExp& E) {
+#pragma clang fp contract(off)
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
             const float dx = L.dx[a], dy = L.dy[b];
-            E.Fxy[a][b] = kq * fmaf(fmaf(p.A[0], dx, sxy * dy), dx, p.A[4] * dy * dy);
-            E.Gxy[a][b] = kq * fmaf(sxz, dx, syz * dy);
+            E.Fxy[a][b] = kq * fmaf(fmaf(A.xx, dx, A.xy * dy), dx, A.yy * dy * dy);
+            E.Gxy[a][b] = kq * fmaf(A.xz, dx, A.yz * dy);
         }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) E.Fz[c] = kq * (p.A[8] * L.dz[c] * L.dz[c]);
+    for (int c = 0; c < 4; ++c) E.Fz[c] = kq * (A.zz * L.dz[c] * L.dz[c]);
+}
+
+__device__ __forceinline__ void lane_exp(const GaussParams& p, const LaneGeom& L, LaneExp& E) {
+    SymA A;
+    sym_a(p, A);
+    lane_exp(A, L, E);
 }
 
 __device__ __forceinline__ float lane_e(const LaneExp& E, const LaneGeom& L, int a, int b, int c) {
@@ -403,13 +388,23 @@ __device__ __forceinline__ float lane_e(const LaneExp& E, const LaneGeom& L, int
     return __builtin_amdgcn_exp2f(fmaf(E.Gxy[a][b], L.dz[c], E.Fxy[a][b] + E.Fz[c]));
 }
 
+// One workgroup of four waves per tile, two per CU: wave w multiplies the tile's 64 voxels with its 64 of a
+// pass's 256 Gaussians (N blocks w and w + 4), so that each F value is read from LDS once, no sum crosses
+// waves, and the wave keeps its accumulators in registers through both epilogues.  A tile is a chain (list
+// bounds, list, rows, chunk steps with barriers, two epilogues) of which most is latency; what bounds the
+// kernel is what runs beside it on the CU, so the LDS (76 KB: two F chunks, one A operand, G in registers) and
+// the registers (256) are sized for two workgroups.  Against one workgroup of eight waves per CU (three F chunks
+// and three of G in LDS): 200 x 200 x 16, 18000 Gaussians x 1024 channels 1.49 -> 1.21 ms (2.62 GB of gF, 0.48 ms
+// at the copy rate), in bfloat16 0.98 -> 0.81; 9000 x 768 0.95 -> 0.71; lists of 640 x 512 channels 3.1 -> 2.6; 2000
+// x 64 in 50 x 50 x 8 (set-up and epilogues) 0.049 -> 0.033; fused cosine gradient 9000 x 512 0.89 -> 0.75.
+//
 // BF: features and grad_feats are bfloat16.  A chunk is then 64 channels (the split rows hold the
-// values themselves, 128 bytes per chunk row, as k_split_chunks<__bf16> writes them; the grad_feats
-// chunk rows are 128 bytes of bfloat16), and each k half of 32 channels is two 16-channel slices:
-// the A and B "hi" operands carry slice 0 and the "lo" operands slice 1, with one MFMA each.
+// values themselves, 128 bytes per chunk row, as k_split_chunks<__bf16> writes them), and each k half of
+// 32 channels is two 16-channel slices: the A and B "hi" operands carry slice 0 and the "lo" operands
+// slice 1, with one MFMA each.
 // FU (with VEC, float32): the upstream feature gradient is the cosine loss's (cg), gF_ is unused.
 template <bool VEC, bool BF, bool FU>
-__global__ void __launch_bounds__(kBtThreads, 1) k_bwd_tile(
+__global__ void __launch_bounds__(kBtThreads, 2) k_bwd_tile(
     Grid G, int n, int C, int nchk, const float* __restrict__ gD, const void* __restrict__ gF_,
     const float* __restrict__ means, const float* __restrict__ opacity,
     const float* __restrict__ cov_inv, const int* __restrict__ lb, const int* __restrict__ ub,
@@ -444,8 +439,7 @@ __global__ void __launch_bounds__(kBtThreads, 1) k_bwd_tile(
             cg.coef += 2 * vb;
         }
     }
-    const int lane = threadIdx.x & 63, wave = uniform(threadIdx.x >> 6);
-    const int mb = wave >> 2, ngrp = wave & 3;   // voxel block (epilogues) / k half (K loop), N group
+    const int lane_ = threadIdx.x & 63, wave_ = uniform(threadIdx.x >> 6);
     const int tyz = G.tiles[1] * G.tiles[2];
     const int tx = tile / tyz, ty = (tile - tx * tyz) / G.tiles[2], tz = tile % G.tiles[2];
     // every voxel of the tile inside the grid (no row of the A operand is cleared)
@@ -469,12 +463,13 @@ __global__ void __launch_bounds__(kBtThreads, 1) k_bwd_tile(
     if (Ng <= skip_le) return;   // empty, or a short list that k_bwd_tile_short takes
     // the first pass's list entries, requested before the voxel values are staged (raw values at
     // clamped positions; the entries past the pass are selected away where they are used)
-    const int lwave = uniform(threadIdx.x >> 6), llane = threadIdx.x & 63;
     const int pc0 = min(kBtPass, Ng);
-    const int l0 = sorted_gauss[j0 + min((int)threadIdx.x, pc0 - 1)];
-    int lrow0[kBtDma];
+    int gld[kBtNbw], grow[kBtDma];   // the Gaussians of the lane's columns and of its F rows (clamped to the list)
 #pragma unroll
-    for (int i = 0; i < kBtDma; ++i) lrow0[i] = sorted_gauss[j0 + min((lwave + kBtWaves * i) * 8 + (llane >> 3), pc0 - 1)];
+    for (int j = 0; j < kBtNbw; ++j) gld[j] = sorted_gauss[j0 + min((wave_ + kBtWaves * j) * 32 + (lane_ & 31), pc0 - 1)];
+#pragma unroll
+    for (int i = 0; i < kBtDma; ++i)
+        grow[i] = sorted_gauss[j0 + min((wave_ + kBtWaves * i) * kBtRows + lane_ / 8, pc0 - 1)];
     if (threadIdx.x < 64) {
         const bool ok = vok;
         const int64_t v = vx;
@@ -497,10 +492,10 @@ __global__ void __launch_bounds__(kBtThreads, 1) k_bwd_tile(
     // Lists longer than one pass: t_v = sum_c gF_vc F_vc straight from grid_feats.
     const bool multi = Ng > kBtPass;
     if (multi && VEC && !BF && (FU || gdt != kDtBF16) && ((uintptr_t)grid_feats & 15) == 0) {
-        // float rows of 16-byte multiples: the wave's 8 voxels at once, 8 lanes per row reading
-        // 16-byte pieces (many loads in flight), then a sum over the row's 8 lanes.  FU: G = k1
+        // float rows of 16-byte multiples: the wave's 16 voxels at once, 4 lanes per row reading
+        // 16-byte pieces (many loads in flight), then a sum over the row's 4 lanes.  FU: G = k1
         // target + k2 grid_feats formed per value, as the loss's own backward forms it.
-        const int r = wave * 8 + (lane >> 3), q = lane & 7;
+        const int r = wave_ * kBtGRows + lane_ / 4, q = lane_ & 3;
         const int v = sm.vlin[r];
         float s = 0.0f;
         if (v >= 0) {
@@ -513,8 +508,8 @@ __global__ void __launch_bounds__(kBtThreads, 1) k_bwd_tile(
                 k1 = sm.kc[0][r];
                 k2 = sm.kc[1][r];
             }
-#pragma unroll 4
-            for (int c4 = q; c4 < n4; c4 += 8) {
+#pragma unroll 8
+            for (int c4 = q; c4 < n4; c4 += 4) {
                 float4 x = a4[c4];
                 const float4 y = b4[c4];
                 if constexpr (FU) {
@@ -531,11 +526,10 @@ __global__ void __launch_bounds__(kBtThreads, 1) k_bwd_tile(
         }
         s += __shfl_xor(s, 1, 64);
         s += __shfl_xor(s, 2, 64);
-        s += __shfl_xor(s, 4, 64);
         if (q == 0 && v >= 0) sm.tv[r] = sm.D[r] >= kEps ? s : 0.0f;
     } else if (multi) {
-        for (int k = 0; k < 8; ++k) {
-            const int r = wave * 8 + k;
+        for (int k = 0; k < kBtGRows; ++k) {
+            const int r = wave_ * kBtGRows + k;
             const int v = sm.vlin[r];
             if (v < 0) continue;
             const GT* a = gF + (int64_t)v * C;
@@ -545,131 +539,107 @@ __global__ void __launch_bounds__(kBtThreads, 1) k_bwd_tile(
                 const float k1 = sm.kc[0][r], k2 = sm.kc[1][r];
                 const float* tg = cg.tgt + (int64_t)v * C;
                 const float* b = static_cast<const float*>(grid_feats) + (int64_t)v * C;
-                for (int c = lane; c < C; c += 64) {
+                for (int c = lane_; c < C; c += 64) {
                     const float gv = k1 * tg[c] + k2 * b[c];
                     s += gv * b[c];
                 }
             } else if (gdt == kDtBF16) {
                 const __bf16* b = static_cast<const __bf16*>(grid_feats) + (int64_t)v * C;
-                for (int c = lane; c < C; c += 64) s += (float)a[c] * (float)b[c];
+                for (int c = lane_; c < C; c += 64) s += (float)a[c] * (float)b[c];
             } else {
                 const float* b = static_cast<const float*>(grid_feats) + (int64_t)v * C;
-                for (int c = lane; c < C; c += 64) s += (float)a[c] * b[c];
+                for (int c = lane_; c < C; c += 64) s += (float)a[c] * b[c];
             }
             s = wave_sum(s);
-            if (lane == 0) sm.tv[r] = sm.D[r] >= kEps ? s : 0.0f;
+            if (lane_ == 0) sm.tv[r] = sm.D[r] >= kEps ? s : 0.0f;
         }
     }
-
-    // G staging: direct-to-LDS loads of the raw chunk (voxel rows clamped to a valid row, channels
-    // clamped into the row).  Row v of a stage keeps its 16-byte piece p (channels 4p..4p+3) at
-    // slot p ^ swz(v), so that the A-operand reads (8 or 16 consecutive rows per LDS cycle) are
-    // free of bank conflicts.  VEC: one 16-byte load per lane, lane = (row, slot); otherwise four 4-byte
-    // loads per lane, each covering two rows.
-    // BF: a chunk row is 128 bytes of bfloat16; with VEC (C % 8 == 0, 16-byte aligned rows) lane l
-    // loads 16-byte piece l % 8 of row l / 8 of the wave's 8 rows (stage rows of 128 bytes, pieces
-    // in order, read whole by write_a); without VEC write_a loads the A operand itself.
-    // FU: the target and grid_feats chunks of the same rows, into sources 0 and 1 of the stage.
-    constexpr int kNG = BF ? (VEC ? 1 : 0) : (VEC ? 1 : 4);   // G loads per wave per chunk and source
-    constexpr int kNGs = kNG > 0 ? kNG : 1;
-    constexpr int kSrc = FU ? 2 : 1;
-    const GT* gsrc[kSrc][kNGs];
-    int gcoff[kNGs];   // channel of this lane's load within a chunk
-    // VEC float: chunks wholly inside the rows are loaded from a wave-uniform base (the source's
-    // start plus the chunk) and the lane's fixed 32-bit byte offset, when every row offset fits
-    const GT* gbase[kSrc];
-    uint32_t goff[kNGs];
-    gbase[0] = FU ? reinterpret_cast<const GT*>(cg.tgt) : gF;
-    gbase[kSrc - 1] = FU ? static_cast<const GT*>(grid_feats) : gF;
-    const bool g32 = (int64_t)G.dims[0] * G.dims[1] * G.dims[2] * C * (int64_t)sizeof(GT) <= 0xffffffffLL;
-#pragma unroll
-    for (int k = 0; k < kNG; ++k) {
-        const int v = (BF || VEC) ? wave * 8 + (lane >> 3) : wave * 8 + 2 * k + (lane >> 5);
-        const int64_t row = (int64_t)max(sm.vlin[v], 0) * C;
-        if constexpr (FU) {
-            gsrc[0][k] = reinterpret_cast<const GT*>(cg.tgt) + row;
-            gsrc[kSrc - 1][k] = static_cast<const GT*>(grid_feats) + row;
-        } else {
-            gsrc[0][k] = gF + row;
-        }
-        gcoff[k] = BF ? 8 * (lane & 7)
-                      : (VEC ? 4 * ((lane & 7) ^ swz(v)) : 4 * (((lane & 31) >> 2) ^ swz(v)) + (lane & 3));
-        goff[k] = (uint32_t)((row + gcoff[k]) * (int64_t)sizeof(GT));
-    }
-    auto dma_g = [&](int chunk, int stage) {
-#pragma unroll
-        for (int sr = 0; sr < kSrc; ++sr)
-#pragma unroll
-            for (int k = 0; k < kNG; ++k) {
-                if constexpr (BF) {
-                    dma16_nt(gsrc[sr][k] + min(chunk * kKc + gcoff[k], C - 8),
-                             uniform(lds_addr(reinterpret_cast<char*>(&sm.graw[stage][sr][0][0]) + wave * 8 * 128)));
-                } else if (VEC) {
-                    const uint32_t lds = uniform(lds_addr(&sm.graw[stage][sr][wave * 8][0]));
-                    if (g32 && chunk * kBtKc + kBtKc <= C)   // wave-uniform
-                        dma16s_nt(gbase[sr] + chunk * kBtKc, goff[k], lds);
-                    else
-                        dma16_nt(gsrc[sr][k] + min(chunk * kBtKc + gcoff[k], C - 4), lds);
-                } else {
-                    dma4_nt(gsrc[sr][k] + min(chunk * kBtKc + gcoff[k], C - 1),
-                            uniform(lds_addr(&sm.graw[stage][sr][wave * 8 + 2 * k][0])));
-                }
-            }
-    };
 
     const uint32_t fstride = (uint32_t)nchk * kBtRowBytes;   // bytes of one Gaussian's split row
     const char* fbase = reinterpret_cast<const char*>(fsp);
-    const int ks = mb;                // k half of every chunk this wave multiplies (channels 16ks..16ks+15)
-    const int h = lane >> 5;
 
     for (int pbase = 0; pbase < Ng; pbase += kBtPass) {
         const int pcount = min(kBtPass, Ng - pbase);
+        // The thread's indices are hidden from the compiler at the start of a pass and again at its epilogues:
+        // it would otherwise compute all that depends on them before the pass loop and spill it
+        // through the K loop (41 registers; 1.43 -> 1.21 ms at 18000 Gaussians x 1024 channels without).
+        int lane = lane_, wave = wave_;
+        asm volatile("" : "+v"(lane));
+        asm volatile("" : "+s"(wave));
+        const int h = lane >> 5;
         // LDS-only barriers here and in the epilogues: the weight and partial stores (read by later
         // kernels only) stay in flight while the next steps run
         lds_barrier();
 
+        // G goes from memory to registers three chunks ahead: thread (voxel sv, piece sq) loads 16 bytes of each
+        // k half of its row (float: channels 4 sq .. of the half's 16; bfloat16: 8 sq .. of its 32), channels
+        // clamped into the row and rows to a valid one.  float: the wave's lane = (sq / 2, voxel, sq & 1), so that its
+        // 8-byte writes of the split values are contiguous runs.
+        constexpr int kSrc = FU ? 2 : 1;
+        constexpr int kPc = BF ? 8 : 4;   // channels of a piece
+        const int sv = wave * kBtGRows + (BF ? lane & 15 : (lane >> 1) & 15);
+        const int sq = BF ? lane >> 4 : 2 * h + (lane & 1);
+        const bool svok = sm.vlin[sv] >= 0;
+        const int64_t srow = (int64_t)max(sm.vlin[sv], 0) * C;
+        typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+        // chunks wholly inside the rows are loaded from a wave-uniform base and the thread's fixed 32-bit offset, when
+        // every row offset fits
+        const bool g32 = (int64_t)G.dims[0] * G.dims[1] * G.dims[2] * C * (int64_t)sizeof(GT) <= 0xffffffffLL;
+        const uint32_t goff = (uint32_t)((srow + kPc * sq) * (int64_t)sizeof(GT));
+        auto load_g = [&](int chunk, u32x4 (&g)[kSrc][2]) {
+#pragma unroll
+            for (int sr = 0; sr < kSrc; ++sr) {
+                const GT* base = FU ? (sr == 0 ? reinterpret_cast<const GT*>(cg.tgt) : static_cast<const GT*>(grid_feats)) : gF;
+                const GT* row = base + srow;
+                if (VEC && g32 && chunk * kKc + kKc <= C) {   // wave-uniform
+                    const char* ub = reinterpret_cast<const char*>(base + chunk * kKc);
+                    g[sr][0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(ub + goff));
+                    g[sr][1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(ub + goff + kKc / 2 * sizeof(GT)));
+                    continue;
+                }
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    const int c = chunk * kKc + ks * (kKc / 2) + kPc * sq;
+                    if constexpr (VEC) {
+                        g[sr][ks] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + min(c, C - kPc)));
+                    } else if constexpr (BF) {
+                        const unsigned short* r16 = reinterpret_cast<const unsigned short*>(row);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            g[sr][ks][i] = r16[min(c + 2 * i, C - 1)] | ((unsigned)r16[min(c + 2 * i + 1, C - 1)] << 16);
+                    } else {
+                        const unsigned* r32 = reinterpret_cast<const unsigned*>(row);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) g[sr][ks][i] = r32[min(c + i, C - 1)];
+                    }
+                }
+            }
+        };
+
         // F rows by direct-to-LDS loads: row group rg = wave + kBtWaves*i (8 rows, 1 KB) is
         // loaded by this wave; lane = (row rg*8 + lane/8, slot lane%8) and slot p carries the
         // 16-byte piece p ^ swz(row) of the row's chunk.  Rows past the list read the zero row;
-        // groups wholly past it are not loaded (no wave reads them).  A wave issues exactly
-        // nld = (its groups within the list) + kNG loads per chunk, so the wait counts below are
-        // exact.  The rows' Gaussians come straight from the list, so that the first chunks' loads
-        // are issued before the parameters are staged and both are in flight together.
-        const int* list = sorted_gauss + j0 + pbase;
-        const int kent = threadIdx.x;                        // this thread's list entry (staging)
-        int gk, grow[kBtDma];
-        if (pbase == 0) {   // requested at the tile start
-            gk = kent < pcount ? l0 : -1;
-#pragma unroll
-            for (int i = 0; i < kBtDma; ++i) grow[i] = (wave + kBtWaves * i) * 8 + (lane >> 3) < pcount ? lrow0[i] : n;
-        } else {
-            gk = kent < pcount ? list[kent] : -1;
-#pragma unroll
-            for (int i = 0; i < kBtDma; ++i) {
-                const int r = (wave + kBtWaves * i) * 8 + (lane >> 3);
-                grow[i] = r < pcount ? list[r] : n;
-            }
-        }
+        // groups wholly past it are not loaded (no wave reads them).  128-byte rows: a miss of L2 brings a
+        // whole 128-byte line, so 64-byte chunk rows fetched most lines twice.
         uint32_t doff[kBtDma];
 #pragma unroll
         for (int i = 0; i < kBtDma; ++i) {
-            const int rg = wave + kBtWaves * i;
-            const int r = rg * 8 + (lane >> 3);
+            const int r = (wave + kBtWaves * i) * kBtRows + lane / 8;
             const int piece = (lane & 7) ^ swz(r);
-            doff[i] = (rg * 8 < pcount) ? (uint32_t)grow[i] * fstride + (uint32_t)piece * 16u : (uint32_t)n * fstride;
+            doff[i] = (uint32_t)(r < pcount ? grow[i] : n) * fstride + (uint32_t)piece * 16u;
         }
         // the wave's groups within the list are its first nf (rg grows with i)
         int nf = 0;
 #pragma unroll
-        for (int i = 0; i < kBtDma; ++i) nf += ((wave + kBtWaves * i) * 8 < pcount) ? 1 : 0;
+        for (int i = 0; i < kBtDma; ++i) nf += ((wave + kBtWaves * i) * kBtRows < pcount) ? 1 : 0;
         nf = uniform(nf);
-        auto dma_f = [&](int chunk, int buf, int i0, int i1) {
+        auto dma_f = [&](int chunk, int buf) {
 #pragma unroll
             for (int i = 0; i < kBtDma; ++i) {
-                if (i < i0 || i >= i1) continue;
+                if (i >= nf) break;   // wave-uniform
                 const int rg = wave + kBtWaves * i;
                 dma16s(fbase + (size_t)chunk * kBtRowBytes, doff[i],
-                       uniform(lds_addr(&sm.u.frow[buf][rg * 8 * kBtRowBytes])));
+                       uniform(lds_addr(&sm.frow[buf][rg * kBtRows * kBtRowBytes])));
             }
         };
         const int clast = nchk - 1;
@@ -679,164 +649,88 @@ __global__ void __launch_bounds__(kBtThreads, 1) k_bwd_tile(
         const bool rev = ((pbase / kBtPass) & 1) != 0;
         auto cm = [&](int c) { return (rev && c <= clast) ? clast - c : c; };
 
-        // this thread's entry: parameters and its G->T pair with this tile, requested first
-        float emu[3] = {0.f, 0.f, 0.f}, eA[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, eo = 0.f;
-        int elb[3] = {0, 0, 0}, eub[3] = {0, 0, 0}, eoff = 0;
-        if (gk >= 0) {
-#pragma unroll
-            for (int q = 0; q < 3; ++q) {
-                emu[q] = means[gk * 3 + q];
-                elb[q] = lb[gk * 3 + q];
-                eub[q] = ub[gk * 3 + q];
-            }
-#pragma unroll
-            for (int q = 0; q < 9; ++q) eA[q] = cov_inv[gk * 9 + q];
-            eo = opacity[gk];
-            eoff = g2t_offsets[gk];
-        }
-        // the first chunks' loads (G three chunks ahead, F two, or one with FU), in flight with them
-        dma_g(cm(0), 0);
-        dma_f(cm(0), 0, 0, nf);
-        dma_g(cm(min(1, clast)), 1);
-        if constexpr (!FU) dma_f(cm(min(1, clast)), 1, 0, nf);
-        dma_g(cm(min(2, clast)), 2);
-        if (kent < kBtPass) {
-            sm.pt.gid[kent] = gk;
-            int pair = -1;
-            if (gk >= 0) {
-#pragma unroll
-                for (int q = 0; q < 3; ++q) {
-                    sm.pt.mu[q][kent] = emu[q];
-                    sm.pt.lb[q][kent] = elb[q];
-                    sm.pt.ub[q][kent] = eub[q];
-                }
-#pragma unroll
-                for (int q = 0; q < 9; ++q) sm.pt.A[q][kent] = eA[q];
-                sm.pt.o[kent] = eo;
-                const int tx0 = elb[0] / kTile, ty0 = elb[1] / kTile, tz0 = elb[2] / kTile;
-                const int dy = eub[1] / kTile - ty0 + 1, dz = eub[2] / kTile - tz0 + 1;
-                const int64_t pr = (int64_t)eoff + ((tx - tx0) * dy + (ty - ty0)) * dz + (tz - tz0);
-                pair = (pr >= 0 && pr < M) ? (int)pr : -1;   // malformed CSR: never write outside the buffer
-            }
-            sm.pidx[kent] = pair;
-        }
-        // Every load of the pass start complete (the first chunks' too: the parameter stores above
-        // already waited for most of them).  A thread that staged no entry would otherwise reach the
-        // K loop with the parameter loads still pending for the compiler's wait counts, which
-        // then wait for all loads inside the K loop wherever their registers are reused there.
+        u32x4 gs[3][kSrc][2];   // G of chunks ch (half 0 already split), ch + 1 and ch + 2, chunk c in set c % 3
+        load_g(cm(0), gs[0]);
+        dma_f(cm(0), 0);
+        load_g(cm(min(1, clast)), gs[1]);
+        load_g(cm(min(2, clast)), gs[2]);
+        // Every load of the pass start complete: parameter loads still pending for the compiler's wait counts
+        // would make it wait for all loads inside the K loop wherever their registers are used.
         wait_vm<0>();
-        lds_barrier();
 
-        // wave (ks, ngrp) accumulates k half ks of every chunk for both voxel blocks m and its N
-        // blocks ngrp + 4j; the halves are added after the K loop
-        f32x16 acc2[2][kBtNbw];
+        f32x16 acc[2][kBtNbw];   // [voxel block m][N block wave + kBtWaves j]
 #pragma unroll
         for (int m = 0; m < 2; ++m)
 #pragma unroll
-            for (int j = 0; j < kBtNbw; ++j) acc2[m][j] = f32x16{};
+            for (int j = 0; j < kBtNbw; ++j) acc[m][j] = f32x16{};
         int nact = 0;
-        int gcol[kBtNbw];
 #pragma unroll
-        for (int j = 0; j < kBtNbw; ++j) {
-            nact += ((ngrp + kBtGroups * j) * 32 < pcount) ? 1 : 0;
-            gcol[j] = sm.pt.gid[(ngrp + kBtGroups * j) * 32 + (lane & 31)];
-        }
+        for (int j = 0; j < kBtNbw; ++j) nact += ((wave + kBtWaves * j) * 32 < pcount) ? 1 : 0;
         nact = uniform(nact);
-        // A operand of chunk ch, split once per value: thread (voxel sv, channel quad sq) reads its
-        // four raw G values (stage gs), masks them (row outside the grid, channels past C),
-        // splits them and writes hi and lo into A buffer ab: channels 4sq.. of the chunk are k
-        // half sq/4, lane group (sq/2)&1, half sq&1 of the lane's 16-byte fragment.
-        // float: wave w writes the fragments of voxel block w&1, lane group (w/2)&1, k half w/4,
-        // lane (sv&31, sq&1): 32 whole 16-byte fragments, one contiguous 512-byte run per array, so
-        // the 8-byte writes are free of bank conflicts (a wave of 8 voxels x 8 quads would put four
-        // writes on every bank); its reads, 16 bytes of 32 consecutive rows at pieces sq and sq^1,
-        // stay conflict-free through the row swizzle.  bfloat16 rows are not swizzled, so there the
-        // wave keeps 8 voxels x 8 octets (each read covers whole rows).
-        const int sv = BF ? threadIdx.x >> 3 : (((threadIdx.x >> 6) & 1) << 5) | ((threadIdx.x & 63) >> 1);
-        const int sq = BF ? threadIdx.x & 7 : ((threadIdx.x >> 8) << 2) | (((threadIdx.x >> 7) & 1) << 1) | (threadIdx.x & 1);
-        const bool svok = sm.vlin[sv] >= 0;
-        auto write_a = [&](int ch, int gs, int ab) {
-            const int lim = svok ? min(max(C - (ch * kKc + 4 * sq), 0), 4) : 0;
+        // A operand of k half ks of chunk ch, split once per value: the thread masks its 16 bytes (row
+        // outside the grid, channels past C), splits them and writes hi and lo.  float: channels 4 sq .. are lane
+        // group sq/2, half sq&1 of the voxel's 16-byte fragment; bfloat16: channels 8 sq .. are slice sq/2, lane
+        // group sq&1.
+        auto write_a = [&](int ch, int ks, const u32x4 (&g)[kSrc][2]) {
+            const int c0 = ch * kKc + ks * (kKc / 2) + kPc * sq;
+            const int lim = svok ? min(max(C - c0, 0), kPc) : 0;
             typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
             typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
             typedef float f32x2 __attribute__((ext_vector_type(2)));
-            const int L = ((sq >> 1) & 1) * 32 + (sv & 31);
+            const int L = (sq >> 1) * 32 + (sv & 31);
+            const bool whole = tile_in && ch * kKc + kKc <= C;   // wave-uniform: nothing to clear
+            u32x4 xr = g[0][ks];
             if constexpr (BF) {
-                // bfloat16: thread (sv, sq) takes channels 8sq..8sq+7 of the 64-channel chunk, i.e.
-                // k half sq/4, slice (sq/2)&1 (A buffer ahi for slice 0, alo for slice 1), lane
-                // group sq&1 of the voxel's fragment; values past the row or the grid are cleared
-                const int lim8 = svok ? min(max(C - (ch * kKc + 8 * sq), 0), 8) : 0;
-                uint4 xr;
-                if constexpr (VEC) {
-                    xr = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(&sm.graw[gs][0][0][0]) +
-                                                         sv * 128 + sq * 16);
-                } else {
-                    const unsigned short* row =
-                        reinterpret_cast<const unsigned short*>(gF + (int64_t)max(sm.vlin[sv], 0) * C);
-                    unsigned e[8];
+                if (!whole) {
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) e[i] = row[min(ch * kKc + 8 * sq + i, C - 1)];
-                    xr = make_uint4(e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16));
+                    for (int w = 0; w < 4; ++w)
+                        xr[w] &= (2 * w < lim ? 0x0000ffffu : 0u) | (2 * w + 1 < lim ? 0xffff0000u : 0u);
                 }
-                auto keep = [&](int w) {   // mask of word w (elements 2w and 2w + 1)
-                    return (2 * w < lim8 ? 0x0000ffffu : 0u) | (2 * w + 1 < lim8 ? 0xffff0000u : 0u);
-                };
-                xr.x &= keep(0);
-                xr.y &= keep(1);
-                xr.z &= keep(2);
-                xr.w &= keep(3);
                 const int Lb = (sq & 1) * 32 + (sv & 31);
-                bf16x8* dst = ((sq >> 1) & 1) ? &sm.alo[ab][sq >> 2][sv >> 5][Lb] : &sm.ahi[ab][sq >> 2][sv >> 5][Lb];
-                *reinterpret_cast<uint4*>(dst) = xr;
+                bf16x8* dst = (sq >> 1) ? &sm.alo[ks][sv >> 5][Lb] : &sm.ahi[ks][sv >> 5][Lb];
+                *reinterpret_cast<u32x4*>(dst) = xr;
                 return;
             }
-            // one 16-byte LDS read, then the values past the row or the grid are cleared with bit
-            // masks (a select per value would let the compiler split the read into guarded parts)
-            uint4 xr = *reinterpret_cast<const uint4*>(&sm.graw[gs][0][sv][4 * (sq ^ swz(sv))]);
             if constexpr (FU) {
                 // G = k1 target + k2 grid_feats (the expression of the loss's own backward)
-                const uint4 xf = *reinterpret_cast<const uint4*>(&sm.graw[gs][kSrc - 1][sv][4 * (sq ^ swz(sv))]);
+                const u32x4 xf = g[kSrc - 1][ks];
                 const float k1 = sm.kc[0][sv], k2 = sm.kc[1][sv];
-                xr.x = __float_as_uint(k1 * __uint_as_float(xr.x) + k2 * __uint_as_float(xf.x));
-                xr.y = __float_as_uint(k1 * __uint_as_float(xr.y) + k2 * __uint_as_float(xf.y));
-                xr.z = __float_as_uint(k1 * __uint_as_float(xr.z) + k2 * __uint_as_float(xf.z));
-                xr.w = __float_as_uint(k1 * __uint_as_float(xr.w) + k2 * __uint_as_float(xf.w));
+#pragma unroll
+                for (int w = 0; w < 4; ++w)
+                    xr[w] = __float_as_uint(k1 * __uint_as_float(xr[w]) + k2 * __uint_as_float(xf[w]));
             }
-            if (!(tile_in && ch * kKc + kKc <= C)) {   // wave-uniform: rows or channels to clear
-                xr.x &= 0u - (unsigned)(0 < lim);
-                xr.y &= 0u - (unsigned)(1 < lim);
-                xr.z &= 0u - (unsigned)(2 < lim);
-                xr.w &= 0u - (unsigned)(3 < lim);
+            if (!whole) {   // bit masks: a value not in the row may be anything
+#pragma unroll
+                for (int w = 0; w < 4; ++w) xr[w] &= 0u - (unsigned)(w < lim);
             }
-            const f32x2 x01 = {__uint_as_float(xr.x), __uint_as_float(xr.y)};
-            const f32x2 x23 = {__uint_as_float(xr.z), __uint_as_float(xr.w)};
+            const f32x2 x01 = {__uint_as_float(xr[0]), __uint_as_float(xr[1])};
+            const f32x2 x23 = {__uint_as_float(xr[2]), __uint_as_float(xr[3])};
             const bf16x2 h01 = __builtin_convertvector(x01, bf16x2), h23 = __builtin_convertvector(x23, bf16x2);
             const bf16x2 l01 = __builtin_convertvector(x01 - __builtin_convertvector(h01, f32x2), bf16x2);
             const bf16x2 l23 = __builtin_convertvector(x23 - __builtin_convertvector(h23, f32x2), bf16x2);
             const bf16x4 hv = {h01[0], h01[1], h23[0], h23[1]}, lv = {l01[0], l01[1], l23[0], l23[1]};
-            *reinterpret_cast<bf16x4*>(reinterpret_cast<char*>(&sm.ahi[ab][sq >> 2][sv >> 5][L]) + (sq & 1) * 8) = hv;
-            *reinterpret_cast<bf16x4*>(reinterpret_cast<char*>(&sm.alo[ab][sq >> 2][sv >> 5][L]) + (sq & 1) * 8) = lv;
+            *reinterpret_cast<bf16x4*>(reinterpret_cast<char*>(&sm.ahi[ks][sv >> 5][L]) + (sq & 1) * 8) = hv;
+            *reinterpret_cast<bf16x4*>(reinterpret_cast<char*>(&sm.alo[ks][sv >> 5][L]) + (sq & 1) * 8) = lv;
         };
-        // N block j of chunk ch (F stage st, A buffer ab) against both voxel blocks
-        // Operands of one chunk step, A (both voxel blocks) and B (both N blocks), read from LDS
-        // together at the step's start, so that one LDS latency precedes the step's MFMAs (the B
-        // rows of an N block past the list hold stale values and are not multiplied).
+        // Operands of one half step, A (both voxel blocks) and B (both N blocks), read from LDS
+        // together at its start, so that one LDS latency precedes its MFMAs (the B rows of an N block
+        // past the list hold stale values and are not multiplied).
         struct StepOps {
             bf16x8 ah[2], al[2], bh[kBtNbw], bl[kBtNbw];
         };
-        auto load_ops = [&](int st, int ab, StepOps& o) {
+        auto load_ops = [&](int st, int ks, StepOps& o) {
 #pragma unroll
             for (int m = 0; m < 2; ++m) {
-                o.ah[m] = sm.ahi[ab][ks][m][lane];
-                o.al[m] = sm.alo[ab][ks][m][lane];
+                o.ah[m] = sm.ahi[ks][m][lane];
+                o.al[m] = sm.alo[ks][m][lane];
             }
 #pragma unroll
             for (int j = 0; j < kBtNbw; ++j) {
                 // float: pieces 2ks+h (hi) and 4+2ks+h (lo); bfloat16: pieces 4ks+h (slice 0) and
                 // 4ks+2+h (slice 1)
-                const int r = (ngrp + kBtGroups * j) * 32 + (lane & 31), sr = swz(r);
                 const int qh = BF ? 4 * ks + h : 2 * ks + h, ql = BF ? 4 * ks + 2 + h : 4 + 2 * ks + h;
-                const unsigned char* rowp = &sm.u.frow[st][r * kBtRowBytes];
+                const int r = (wave + kBtWaves * j) * 32 + (lane & 31), sr = swz(r);
+                const unsigned char* rowp = &sm.frow[st][r * kBtRowBytes];
                 o.bh[j] = *reinterpret_cast<const bf16x8*>(rowp + ((qh ^ sr) << 4));
                 o.bl[j] = *reinterpret_cast<const bf16x8*>(rowp + ((ql ^ sr) << 4));
             }
@@ -847,194 +741,205 @@ __global__ void __launch_bounds__(kBtThreads, 1) k_bwd_tile(
 #pragma unroll
                 for (int m = 0; m < 2; ++m) {
                     if constexpr (BF) {   // slices 0 and 1
-                        acc2[m][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.ah[m], o.bh[j], acc2[m][j], 0, 0, 0);
-                        acc2[m][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.al[m], o.bl[j], acc2[m][j], 0, 0, 0);
+                        acc[m][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.ah[m], o.bh[j], acc[m][j], 0, 0, 0);
+                        acc[m][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.al[m], o.bl[j], acc[m][j], 0, 0, 0);
                     } else {
-                        acc2[m][j] = mfma_split_32x32x16<false, false>(o.ah[m], o.al[m], o.bh[j], o.bl[j], acc2[m][j]);
+                        acc[m][j] = mfma_split_32x32x16<false, false>(o.ah[m], o.al[m], o.bh[j], o.bl[j], acc[m][j]);
                     }
                 }
             }
         };
 
-        // Pipeline over chunks (every load is direct-to-LDS; F two chunks ahead, G three).  Step
-        // ch starts with the A operand of chunk ch (A buffer ch&1), the F rows of chunk ch and the
-        // G values of chunk ch+1 in LDS.  Between its MFMAs (which run on in the matrix unit) it
-        // writes the A operand of chunk ch+1 and issues the loads of F(ch+2) and G(ch+3); then it
-        // waits until only those loads are outstanding.  G(ch+3) goes to the stage of G(ch), whose
-        // A operand was written in the previous step.
-        // The chunk loop, instantiated for the wave's group count NF (exact wait immediates;
-        // waves of one workgroup may run different instantiations, with the same barriers).
-        auto chunk_loop = [&](auto nfc) {
-            constexpr int NF = decltype(nfc)::value;
-            constexpr int kLd = NF + kNG;   // loads per wave per chunk
-            // G(0), F(0), G(1), F(1), G(2) were issued at the pass start
-            wait_vm<kLd>();               // G(0), F(0), G(1) complete
+        // Pipeline over chunks: half step (ch, ks) multiplies k half ks of chunk ch while the A operand of the
+        // half after it is written.  Step ch loads F(ch+1) into the other stage and then G(ch+3) into the
+        // registers of G(ch), and waits at its end until only that G is outstanding (without VEC, whose loads
+        // are not counted one by one, until nothing is).  The last steps (LOOP false) load no more G.
+        auto step = [&](auto loop, int ch, u32x4 (&gc)[kSrc][2], const u32x4 (&gn)[kSrc][2]) {
+            constexpr bool LOOP = decltype(loop)::value;
+            const int st = ch & 1;
+            StepOps ops;
+            load_ops(st, 0, ops);
+            dma_f(cm(min(ch + 1, clast)), st ^ 1);
+            mult(0, ops);
+            __builtin_amdgcn_sched_barrier(0);
+            write_a(cm(ch), 1, gc);
+            if constexpr (LOOP) load_g(cm(min(ch + 3, clast)), gc);
+            __builtin_amdgcn_sched_barrier(0);
+            mult(1, ops);
+            __builtin_amdgcn_sched_barrier(0);
             lds_barrier();
-            write_a(cm(0), 0, 0);
+            load_ops(st, 1, ops);
+            __builtin_amdgcn_sched_barrier(0);
+            mult(0, ops);
+            __builtin_amdgcn_sched_barrier(0);
+            write_a(cm(ch + 1), 0, gn);
+            __builtin_amdgcn_sched_barrier(0);
+            mult(1, ops);
+            asm volatile("" ::: "memory");
+            wait_vm<LOOP && VEC ? 2 * kSrc : 0>();
             lds_barrier();
-            for (int ch = 0; ch < nchk; ++ch) {
-                const int st = ch % kBtStages, ab = ch & 1;
-                StepOps ops;
-                load_ops(st, ab, ops);
-                asm volatile("" ::: "memory");   // every operand read issued before the first MFMA
-                mult(0, ops);
-                __builtin_amdgcn_sched_barrier(0);
-                write_a(cm(ch + 1), (ch + 1) % kBtStages, ab ^ 1);
-                dma_f(cm(min(ch + 2, clast)), (ch + 2) % kBtStages, 0, min(NF, kBtDma / 2));
-                __builtin_amdgcn_sched_barrier(0);
-                mult(1, ops);
-                __builtin_amdgcn_sched_barrier(0);
-                dma_f(cm(min(ch + 2, clast)), (ch + 2) % kBtStages, kBtDma / 2, NF);
-                dma_g(cm(min(ch + 3, clast)), st);
-                wait_vm<kLd>();           // F(ch+1) and G(ch+2) complete
-                lds_barrier();
-            }
         };
-        // FU: two F buffers, so F(ch+1) is loaded at the start of step ch into the buffer that step
-        // ch-1 read, and waited for at its end; G (two sources) is still three chunks ahead.
-        auto chunk_loop_fu = [&](auto nfc) {
-            constexpr int NF = decltype(nfc)::value;
-            constexpr int kLg = kSrc * kNG;   // G loads per wave per chunk
-            // G(0), F(0), G(1), G(2) were issued at the pass start
-            wait_vm<kLg>();               // G(0), F(0), G(1) complete
-            lds_barrier();
-            write_a(cm(0), 0, 0);
-            lds_barrier();
-            for (int ch = 0; ch < nchk; ++ch) {
-                const int st = ch % kBtStages, fb = ch & 1, ab = ch & 1;
-                dma_f(cm(min(ch + 1, clast)), fb ^ 1, 0, NF);
-                StepOps ops;
-                load_ops(fb, ab, ops);
-                asm volatile("" ::: "memory");   // every operand read issued before the first MFMA
-                mult(0, ops);
-                __builtin_amdgcn_sched_barrier(0);
-                write_a(cm(ch + 1), (ch + 1) % kBtStages, ab ^ 1);
-                __builtin_amdgcn_sched_barrier(0);
-                mult(1, ops);
-                __builtin_amdgcn_sched_barrier(0);
-                dma_g(cm(min(ch + 3, clast)), st);
-                wait_vm<kLg>();           // F(ch+1) and G(ch+2) complete
-                lds_barrier();
-            }
-        };
-        static_assert(kBtDma == 4, "group-count dispatch");
-        auto run = [&](auto nfc) {
-            if constexpr (FU) chunk_loop_fu(nfc);
-            else chunk_loop(nfc);
-        };
-        switch (nf) {
-            case 4: run(std::integral_constant<int, 4>{}); break;
-            case 3: run(std::integral_constant<int, 3>{}); break;
-            case 2: run(std::integral_constant<int, 2>{}); break;
-            case 1: run(std::integral_constant<int, 1>{}); break;
-            default: run(std::integral_constant<int, 0>{}); break;
+        lds_barrier();
+        write_a(cm(0), 0, gs[0]);
+        lds_barrier();
+        // whole turns of three, then the rest (no path of the loop passes over a step, so that the compiler
+        // knows which loads are still out at each step's first use of G)
+        int ch = 0;
+        for (int t = nchk / 3; t > 0; --t) {
+            step(std::true_type{}, ch, gs[0], gs[1]);
+            step(std::true_type{}, ch + 1, gs[1], gs[2]);
+            step(std::true_type{}, ch + 2, gs[2], gs[0]);
+            ch += 3;
         }
-        // drain the surplus loads of the last steps before the F buffers are reused
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-        __syncthreads();
+        wait_vm<0>();
+        if (ch < nchk) {
+            step(std::false_type{}, ch, gs[0], gs[1]);
+            if (ch + 1 < nchk) step(std::false_type{}, ch + 1, gs[1], gs[2]);
+        }
 
-        // Sum the two k halves: wave (ks, ngrp) keeps voxel block mb = ks and hands the other
-        // block to its partner through LDS.  Both partners add (half 0) + (half 1).
-        f32x16 acc[kBtNbw];
+        // ---- epilogues
         {
-            // [ngrp][m][j][i][lane]: block m of N group ngrp, written by the wave that does not keep it
-            float* xb = reinterpret_cast<float*>(&sm.u.frow[0][0]) + ngrp * (2 * kBtNbw * 16 * 64) + lane;
-            constexpr int kXm = kBtNbw * 16 * 64;
-            if (ks == 0) {
-#pragma unroll
-                for (int j = 0; j < kBtNbw; ++j)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) xb[kXm + (j * 16 + i) * 64] = acc2[1][j][i];
-            } else {
-#pragma unroll
-                for (int j = 0; j < kBtNbw; ++j)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) xb[(j * 16 + i) * 64] = acc2[0][j][i];
-            }
-            __syncthreads();
-            if (ks == 0) {
-#pragma unroll
-                for (int j = 0; j < kBtNbw; ++j)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[j][i] = acc2[0][j][i] + xb[(j * 16 + i) * 64];
-            } else {
-#pragma unroll
-                for (int j = 0; j < kBtNbw; ++j)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[j][i] = xb[kXm + (j * 16 + i) * 64] + acc2[1][j][i];
-            }
-            __syncthreads();   // the exchange area is reused by the epilogues
-        }
-
-        // ---- epilogue 1: split weights w / max(D, eps) of every pair; t_v from U (single pass).
-        // Lane = Gaussian column lane%32 of N block j; element i is the tile's voxel row
-        // r = 32 mb + 8 (i/4) + 4 (lane/32) + i%4.  Branch-free: an element outside the grid, the
-        // Gaussian's box or the list gets e = 0 (and so w = 0).  The validity bits are kept in
-        // registers and the exponentials in LDS (the F buffers are free after the K loop), where
-        // epilogue 2 reads them back instead of evaluating them again (FU: the two F buffers leave no
-        // room, and epilogue 2 evaluates them again).
-        unsigned rowok = 0;   // bit i: row r of element i lies in the grid
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            rowok |= (sm.vlin[mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3)] >= 0) ? (1u << i) : 0u;
-        float rowt[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) rowt[i] = 0.0f;
-        unsigned okm[kBtNbw];
+        int lane = lane_, wave = wave_;
+        asm volatile("" : "+v"(lane));
+        asm volatile("" : "+s"(wave));
+        const int h = lane >> 5;
+        // the lane's Gaussians: what the epilogues need of them stays in registers
+        GaussParams gp[kBtNbw];
+        int pairs[kBtNbw];
 #pragma unroll
         for (int j = 0; j < kBtNbw; ++j) {
-            okm[j] = 0;
-            if (j >= nact) continue;   // wave-uniform
-            const int slot = (ngrp + kBtGroups * j) * 32 + (lane & 31);
-            const bool gok = gcol[j] >= 0;
-            GaussParams p;
-            read_params(sm.pt, slot, p);
-            LaneGeom L;
-            lane_geom(G, p, tx * kTile + 2 * mb, ty * kTile + h, tz * kTile, L);
-            LaneExp E;
-            lane_exp(p, L, E);
-            __bf16* wrow = wt + (int64_t)(j0 + pbase + slot) * kWtRow;
+            const int g = gld[j];
 #pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                __bf16 hs[4], ls[4];
-                float ev[4];
-                const int a = q4 >> 1, b = q4 & 1;
+            for (int q = 0; q < 3; ++q) {
+                gp[j].mu[q] = means[g * 3 + q];
+                gp[j].lb[q] = lb[g * 3 + q];
+                gp[j].ub[q] = ub[g * 3 + q];
+            }
 #pragma unroll
-                for (int ii = 0; ii < 4; ++ii) {
-                    // element i: voxel row r = mb*32 + 8 q4 + 4h + ii, at x = x0 + a, y = y0 + 2b,
-                    // z = z0 + ii; the exponential is always evaluated, then selected
-                    const int i = q4 * 4 + ii;
-                    const int r = mb * 32 + 8 * q4 + 4 * h + ii;
-                    const bool ok = gok & (((rowok >> i) & (L.inx >> a) & (L.iny >> b) & (L.inz >> ii) & 1u) != 0u);
-                    const float e = ok ? lane_e(E, L, a, b, ii) : 0.0f;
-                    ev[ii] = e;
-                    okm[j] |= ok ? (1u << i) : 0u;
-                    const float w = p.o * e;
-                    const float wtil = w * sm.inv[r];
-                    split_bf16(wtil, hs[ii], ls[ii]);
-                    // a select, not a product with 0: columns past the list hold whatever
-                    // the unloaded F rows left in LDS
-                    rowt[i] += (w > 0.0f) ? wtil * acc[j][i] : 0.0f;
-                }
-                if constexpr (!FU) sm.u.ep.e[wave][j][q4][lane] = make_float4(ev[0], ev[1], ev[2], ev[3]);
-                if (gok) {
-                    const int r0 = mb * 32 + 8 * q4 + 4 * h;
+            for (int q = 0; q < 9; ++q) gp[j].A[q] = cov_inv[g * 9 + q];
+            gp[j].o = opacity[g];
+            pairs[j] = g2t_offsets[g];
+        }
+        float mu[kBtNbw][3], op[kBtNbw];
+        SymA sa[kBtNbw];
+        unsigned inb[kBtNbw];   // the lane's voxels in the box: x (4 bits), y0 + h + 2 b (2 bits), z (4 bits); 0: no entry
+#pragma unroll
+        for (int j = 0; j < kBtNbw; ++j) {
+            const GaussParams& p = gp[j];
+            const int tx0 = p.lb[0] / kTile, ty0 = p.lb[1] / kTile, tz0 = p.lb[2] / kTile;
+            const int ey = p.ub[1] / kTile - ty0 + 1, ez = p.ub[2] / kTile - tz0 + 1;
+            const int64_t pr = (int64_t)pairs[j] + ((tx - tx0) * ey + (ty - ty0)) * ez + (tz - tz0);
+            // the pair of the Gaussian with this tile (malformed CSR: never write outside the buffer)
+            pairs[j] = ((wave + kBtWaves * j) * 32 + (lane & 31) < pcount && pr >= 0 && pr < M) ? (int)pr : -1;
+            unsigned in = 0;
+#pragma unroll
+            for (int k = 0; k < kTile; ++k) {
+                const int x = tx * kTile + k, z = tz * kTile + k;
+                in |= (x >= p.lb[0] && x <= p.ub[0] && x < G.dims[0]) ? 1u << k : 0u;
+                in |= (z >= p.lb[2] && z <= p.ub[2] && z < G.dims[2]) ? 64u << k : 0u;
+            }
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const int y = ty * kTile + h + 2 * b;
+                in |= (y >= p.lb[1] && y <= p.ub[1] && y < G.dims[1]) ? 16u << b : 0u;
+            }
+            inb[j] = (wave + kBtWaves * j) * 32 + (lane & 31) < pcount ? in : 0u;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) mu[j][q] = p.mu[q];
+            op[j] = p.o;
+            sym_a(p, sa[j]);
+        }
+        // offsets of the lane's 2 x 2 x 4 voxels of block m from the Gaussian of block j
+        auto geom = [&](int m, int j, LaneGeom& L) {
+#pragma clang fp contract(off)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                L.dx[a] = centre(G, 0, tx * kTile + 2 * m + a) - mu[j][0];
+                L.dy[a] = centre(G, 1, ty * kTile + h + 2 * a) - mu[j][1];
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) L.dz[c] = centre(G, 2, tz * kTile + c) - mu[j][2];
+        };
+        // element (a, b, c) of block m lies in the box and the grid
+        auto inside = [&](int m, int j, int a, int b, int c) {
+            return ((inb[j] >> (2 * m + a)) & (inb[j] >> (4 + b)) & (inb[j] >> (6 + c)) & 1u) != 0u;
+        };
+        // ---- epilogue 1: split weights w / max(D, eps) of every pair; t_v from U (single pass).
+        // Lane = Gaussian column lane%32 of N block j; element i of voxel block m is the tile's voxel row
+        // r = 32 m + 8 (i/4) + 4 (lane/32) + i%4.  Branch-free: an element outside the grid, the
+        // Gaussian's box or the list gets e = 0 (and so w = 0).  The exponentials wait in LDS for epilogue 2.
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            float rowt[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) rowt[i] = 0.0f;
+#pragma unroll
+            for (int j = 0; j < kBtNbw; ++j) {
+                if (j >= nact) continue;   // wave-uniform
+                const bool gok = (wave + kBtWaves * j) * 32 + (lane & 31) < pcount;
+                LaneGeom L;
+                geom(m, j, L);
+                LaneExp E;
+                lane_exp(sa[j], L, E);
+                __bf16* wrow = wt + (int64_t)(j0 + pbase + (wave + kBtWaves * j) * 32 + (lane & 31)) * kWtRow + 32 * m + 8 * h;
+                typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+                u32x2 whi[2], wlo[2];   // split weights of groups q4 = 2a and 2a + 1
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4) {
+                    __bf16 hs[4], ls[4];
+                    float ev[4];
+                    const int a = q4 >> 1, b = q4 & 1, r0 = m * 32 + 8 * q4 + 4 * h;
+                    const float4 iv4 = *reinterpret_cast<const float4*>(&sm.inv[r0]);
+                    const float iv[4] = {iv4.x, iv4.y, iv4.z, iv4.w};
+#pragma unroll
+                    for (int ii = 0; ii < 4; ++ii) {
+                        // element i: voxel row r0 + ii, at x = x0 + a, y = y0 + 2b, z = z0 + ii; the
+                        // exponential is always evaluated, then selected
+                        const int i = q4 * 4 + ii;
+                        const float e = inside(m, j, a, b, ii) ? lane_e(E, L, a, b, ii) : 0.0f;
+                        ev[ii] = e;
+                        const float w = op[j] * e;
+                        const float wtil = w * iv[ii];
+                        split_bf16(wtil, hs[ii], ls[ii]);
+                        // a select, not a product with 0: columns past the list hold whatever
+                        // the unloaded F rows left in LDS
+                        rowt[i] += (w > 0.0f) ? wtil * acc[m][j][i] : 0.0f;
+                    }
                     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-                    bf16x4 hv = {hs[0], hs[1], hs[2], hs[3]};
-                    bf16x4 lv = {ls[0], ls[1], ls[2], ls[3]};
-                    *reinterpret_cast<bf16x4*>(wrow + r0) = hv;
-                    *reinterpret_cast<bf16x4*>(wrow + 64 + r0) = lv;
+                    const bf16x4 hv = {hs[0], hs[1], hs[2], hs[3]}, lv = {ls[0], ls[1], ls[2], ls[3]};
+                    whi[b] = __builtin_bit_cast(u32x2, hv);
+                    wlo[b] = __builtin_bit_cast(u32x2, lv);
+                    if (b == 1) {
+                        u32x4 hq, lq;
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            const auto hx = __builtin_amdgcn_permlane32_swap(whi[0][u], whi[1][u], false, false);
+                            const auto lx = __builtin_amdgcn_permlane32_swap(wlo[0][u], wlo[1][u], false, false);
+                            hq[u] = hx[0];
+                            hq[2 + u] = hx[1];
+                            lq[u] = lx[0];
+                            lq[2 + u] = lx[1];
+                        }
+                        if (gok) {
+                            *reinterpret_cast<u32x4*>(wrow + 16 * a) = hq;
+                            *reinterpret_cast<u32x4*>(wrow + 64 + 16 * a) = lq;
+                        }
+                    }
+                    sm.e[wave][m][j][q4][lane] = make_float4(ev[0], ev[1], ev[2], ev[3]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (!multi) {
+                // rows are shared by the 32 lanes of each half-wave: reduce over them (lanes 2i and
+                // 2i+1 of a half end up with the sum of element i)
+                const float rs = transpose_sum16(rowt, lane & 31);
+                if ((lane & 1) == 0) {
+                    const int i = (lane >> 1) & 15;
+                    sm.tpart[wave][m * 32 + 8 * (i >> 2) + 4 * h + (i & 3)] = rs;
                 }
             }
         }
         if (!multi) {
-            // rows are shared by the 32 lanes of each half-wave: reduce over them (lanes 2i and
-            // 2i+1 of a half end up with the sum of element i)
-            const float rs = transpose_sum16(rowt, lane & 31);
-            if ((lane & 1) == 0) {
-                const int i = (lane >> 1) & 15;
-                sm.tpart[ngrp][mb * 32 + 8 * (i >> 2) + 4 * h + (i & 3)] = rs;
-            }
             lds_barrier();
             if (threadIdx.x < 64) {
                 const int r = threadIdx.x;
@@ -1046,43 +951,37 @@ __global__ void __launch_bounds__(kBtThreads, 1) k_bwd_tile(
         }
 
         // ---- epilogue 2: r = gw e of every element (e from epilogue 1; an invalid element
-        // adds exact zeros) and its moments over the lane's 2 x 2 x 4 voxels relative to the
+        // adds exact zeros) and its moments over the lane's two 2 x 2 x 4 voxel blocks relative to the
         // mean (d = centre - mu): sum r d, sum r d d^T (times o) and sum r.  Phase C turns them
         // into d mu = A (o sum r d), d Sigma = A (o sum r d d^T) A^T / 2 and d o = sum r, since
         // q = A d, sum gw w q = o A sum r d and sum gw w q q^T = o A (sum r d d^T) A^T.
 #pragma unroll
         for (int j = 0; j < kBtNbw; ++j) {
-            const int slot = (ngrp + kBtGroups * j) * 32 + (lane & 31);
-            float gr[kNumGrads] = {};
-            if (j < nact) {   // wave-uniform
-                GaussParams p;
-                read_params(sm.pt, slot, p);
+            if (j >= nact) continue;   // wave-uniform
+            float m0 = 0.f, mx = 0.f, my = 0.f, mz = 0.f, mxx = 0.f, myy = 0.f, mzz = 0.f, mxy = 0.f, mxz = 0.f, myz = 0.f;
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
                 LaneGeom L;
-                lane_geom(G, p, tx * kTile + 2 * mb, ty * kTile + h, tz * kTile, L);
-                // e from epilogue 1 (FU: evaluated again; no LDS is free to keep it)
-                LaneExp E;
-                if constexpr (FU) lane_exp(p, L, E);
-                float m0 = 0.f, mx = 0.f, my = 0.f, mz = 0.f, mxx = 0.f, myy = 0.f, mzz = 0.f, mxy = 0.f,
-                      mxz = 0.f, myz = 0.f;
+                geom(m, j, L);
 #pragma unroll
                 for (int q4 = 0; q4 < 4; ++q4) {
-                    const int a = q4 >> 1, b = q4 & 1;
-                    float ev[4] = {0.f, 0.f, 0.f, 0.f};
-                    if constexpr (!FU) {
-                        const float4 e4 = sm.u.ep.e[wave][j][q4][lane];
-                        ev[0] = e4.x;
-                        ev[1] = e4.y;
-                        ev[2] = e4.z;
-                        ev[3] = e4.w;
-                    }
+                    const int a = q4 >> 1, b = q4 & 1, r0 = m * 32 + 8 * q4 + 4 * h;
+                    const float4 iv4 = *reinterpret_cast<const float4*>(&sm.inv[r0]);
+                    const float4 tv4 = *reinterpret_cast<const float4*>(&sm.tv[r0]);
+                    const float4 gd4 = *reinterpret_cast<const float4*>(&sm.gD[r0]);
+                    const float iv[4] = {iv4.x, iv4.y, iv4.z, iv4.w}, tv[4] = {tv4.x, tv4.y, tv4.z, tv4.w};
+                    const float gd[4] = {gd4.x, gd4.y, gd4.z, gd4.w};
+                    const float4 e4 = sm.e[wave][m][j][q4][lane];
+                    const float ev[4] = {e4.x, e4.y, e4.z, e4.w};
+                    const unsigned inxy = (inb[j] >> (2 * m + a)) & (inb[j] >> (4 + b)) & 1u;
+                    const unsigned inv4 = (0u - inxy) & (inb[j] >> 6);   // the group's four validity bits
                     float s0 = 0.f, sz = 0.f, szz = 0.f;
 #pragma unroll
                     for (int ii = 0; ii < 4; ++ii) {
                         const int i = q4 * 4 + ii;
-                        const int r = mb * 32 + 8 * q4 + 4 * h + ii;
-                        const float gw = sm.gD[r] + (acc[j][i] - sm.tv[r]) * sm.inv[r];
-                        const float e = FU ? lane_e(E, L, a, b, ii) : ev[ii];
-                        const float rr = ((okm[j] >> i) & 1u) ? gw * e : 0.0f;
+                        const float gw = gd[ii] + (acc[m][j][i] - tv[ii]) * iv[ii];
+                        const float re = gw * ev[ii];
+                        const float rr = ((inv4 >> ii) & 1u) != 0u ? re : 0.0f;
                         s0 += rr;
                         const float rz = rr * L.dz[ii];
                         sz += rz;
@@ -1100,38 +999,34 @@ __global__ void __launch_bounds__(kBtThreads, 1) k_bwd_tile(
                     mxz = fmaf(dx, sz, mxz);
                     myz = fmaf(dy, sz, myz);
                 }
-                gr[0] = p.o * mx;
-                gr[1] = p.o * my;
-                gr[2] = p.o * mz;
-                gr[3] = p.o * mxx;
-                gr[4] = p.o * myy;
-                gr[5] = p.o * mzz;
-                gr[6] = p.o * mxy;
-                gr[7] = p.o * mxz;
-                gr[8] = p.o * myz;
-                gr[9] = m0;
+                __builtin_amdgcn_sched_barrier(0);
             }
+            const float o = op[j];
+            float gr[kNumGrads] = {o * mx, o * my, o * mz, o * mxx, o * myy, o * mzz, o * mxy, o * mxz, o * myz, m0};
 #pragma unroll
             for (int k = 0; k < kNumGrads; ++k) gr[k] += __shfl_xor(gr[k], 32, 64);
-            if (lane < 32) {
+            if (lane < 32 && pairs[j] >= 0) {
+                float* out = pair_partials + (int64_t)pairs[j] * kNumGrads;
 #pragma unroll
-                for (int k = 0; k < kNumGrads; ++k) sm.u.xch[mb][slot][k] = gr[k];
+                for (int k = 0; k < kNumGrads; ++k) out[k] = gr[k];
             }
         }
-        lds_barrier();
-        for (int slot = threadIdx.x; slot < pcount; slot += kBtThreads) {
-            const int pair = sm.pidx[slot];
-            if (pair < 0) continue;
-            float* out = pair_partials + (int64_t)pair * kNumGrads;
+        }
+        // the next pass's list entries
+        const int* list = sorted_gauss + j0 + pbase + kBtPass;
+        const int left = Ng - pbase - kBtPass;
+        if (left > 0) {
 #pragma unroll
-            for (int k = 0; k < kNumGrads; ++k) out[k] = sm.u.xch[0][slot][k] + sm.u.xch[1][slot][k];
+            for (int j = 0; j < kBtNbw; ++j) gld[j] = list[min((wave + kBtWaves * j) * 32 + (lane & 31), min(left, kBtPass) - 1)];
+#pragma unroll
+            for (int i = 0; i < kBtDma; ++i) grow[i] = list[min((wave + kBtWaves * i) * kBtRows + lane / 8, min(left, kBtPass) - 1)];
         }
     }
 }
 
 // ------------------------------------------------------------------------------------------
-// Phase A for short lists (1 .. smax <= kBsMax Gaussians).  k_bwd_tile holds one tile per CU (its LDS is
-// sized for 256-Gaussian passes), so a short list leaves that tile's chain of loads and barriers
+// Phase A for short lists (1 .. smax <= kBsMax Gaussians).  k_bwd_tile holds two tiles per CU (its LDS is
+// sized for 256-Gaussian passes), so a short list leaves those tiles' chains of loads and barriers
 // bare; here a 4-wave workgroup with 17 KB of LDS takes the tile and many run per CU.
 //
 // U = G F^T on the float32 matrix cores (16x16x4), straight from the caller's rows: wave w owns the
