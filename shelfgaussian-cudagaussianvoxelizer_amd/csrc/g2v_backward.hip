@@ -1341,8 +1341,8 @@ __global__ void __launch_bounds__(256) k_region_table(Grid G, Regions RG, int M,
 // ------------------------------------------------------------------------------------------
 // Phase B: per-region partial feature gradients, accumulated in registers.
 //
-// Work item = (region, 128-channel chunk); 8 waves.  A pass covers up to 384 rows of the region's
-// Gaussian list in 16-row blocks; block b of the pass belongs to wave b % 8, so a wave owns
+// Work item = (region, channel chunk), in the wide shape 128 channels and 8 waves.  A pass covers up to 384 rows of the
+// region's Gaussian list in 16-row blocks; block b of the pass belongs to wave b % 8, so a wave owns
 // RB = ceil(blocks / 8) or one fewer blocks (RB <= 3) and every wave's work follows the row
 // count, not a fixed 256-row step.  For every tile of the region the tile's gF chunk (64 voxels x
 // 128 channels) is staged in LDS, split hi/lo in the MFMA B layout, and each wave adds
@@ -1354,22 +1354,29 @@ __global__ void __launch_bounds__(256) k_region_table(Grid G, Regions RG, int M,
 // tile k+1 are written to the other LDS buffer, and the gF values of tile k+2 are loaded into
 // registers.
 // ------------------------------------------------------------------------------------------
-constexpr int kBrThreads = 512;   // 8 waves
-constexpr int kBrWaves = kBrThreads / 64;
-constexpr int kBrCc = 128;        // channels per work item
-constexpr int kBrCb = kBrCc / 16; // 16-channel MFMA column blocks
-constexpr int kBrRbMax = 3;       // 16-row blocks per wave and pass
-constexpr int kBrPass = kBrWaves * kBrRbMax * 16;   // region rows per pass
-static_assert(kBrPass * kBrSlots % kBrThreads == 0 && kBrPass <= 2 * kBrThreads, "row-table staging shape");
+// The kernel's two shapes: N waves take N x 16 channels a work item, in passes of RB 16-row blocks per wave.
+template <int N, int RB>
+struct BrShape {
+    static constexpr int kWaves = N, kThreads = 64 * N;
+    static constexpr int kCc = 16 * N;               // channels per work item
+    static constexpr int kCb = kCc / 16;             // 16-channel MFMA column blocks
+    static constexpr int kRbMax = RB;                // 16-row blocks per wave and pass
+    static constexpr int kPass = kWaves * RB * 16;   // region rows per pass
+    static constexpr int kPer = kPass * kBrSlots / kThreads;   // row-table entries per thread
+    static_assert(kPass * kBrSlots % kThreads == 0 && kPass <= 2 * kThreads && kBrSlots * 64 % kThreads == 0, "staging shape");
+};
+typedef BrShape<8, 3> BrWide;     // one workgroup per CU
+typedef BrShape<4, 5> BrNarrow;   // two workgroups per CU
+constexpr int kBrNarrowMax = 64;  // widest row that BrNarrow takes
 
 // FU: the upstream feature gradient is the cosine loss's (k1 target + k2 grid_feats per voxel);
 // kc holds (k1, k2) of the voxels of the region's tiles, in the order of tl_org.
-template <bool FU>
+template <class BR, bool FU>
 struct BrSmem {
-    bf16x8 bhi[2][2][kBrCb][64];   // B operand (gF chunk): [buffer][k step of 32 voxels][channel block][lane]
-    bf16x8 blo[2][2][kBrCb][64];
-    int tab[kBrPass][kBrSlots + 1];       // row table of this pass's rows (M: absent pair); padded row
-    int rslot[kBrPass];                   // G->R slot of each row of the pass
+    bf16x8 bhi[2][2][BR::kCb][64];   // B operand (gF chunk): [buffer][k step of 32 voxels][channel block][lane]
+    bf16x8 blo[2][2][BR::kCb][64];
+    int tab[BR::kPass][kBrSlots + 1];       // row table of this pass's rows (M: absent pair); padded row
+    int rslot[BR::kPass];                   // G->R slot of each row of the pass
     int tl_org[kBrSlots][3], tl_s[kBrSlots];   // tiles of the region (inside the grid): first voxel, slot
     int ntl;
     float2 kc[FU ? kBrSlots : 1][FU ? 64 : 1];
@@ -1497,15 +1504,17 @@ __device__ __forceinline__ unsigned br_load_tile2(const Grid& G, int C, int c0, 
 // so loads stay in flight across the barrier and the compiler waits for each where its registers
 // are used.
 // FU: gF is the target and gF2 grid_feats; a staged value is k1 target + k2 grid_feats.
-template <int NB, bool GB, bool P2, bool FU, bool IN>
-__device__ __forceinline__ void br_tiles(BrSmem<FU>& sm, const Grid& G, int C, int c0, int ntl, int prow,
+template <class BR, int NB, bool GB, bool P2, bool FU, bool IN>
+__device__ __forceinline__ void br_tiles(BrSmem<BR, FU>& sm, const Grid& G, int C, int c0, int ntl, int prow,
                                          const void* __restrict__ gF, const void* __restrict__ gF2,
                                          const __bf16* __restrict__ wt, float* __restrict__ gpart) {
     constexpr int NR = NB > 0 ? NB : 1;   // register arrays (unused when NB == 0)
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // hidden: what depends on it is computed here, not kept through the caller (255 -> 231 registers)
+    const int lane = tid & 63, wave = tid >> 6;
     // staging: channel sc, octets so and so + 4; or (P2) channels 2 cp and 2 cp + 1, octet ot
-    const int sc = threadIdx.x & (kBrCc - 1), so = threadIdx.x >> 7;
-    const int cp2 = 2 * (threadIdx.x & (kBrCc / 2 - 1)), ot = threadIdx.x / (kBrCc / 2);
+    const int sc = tid & (BR::kCc - 1), so = tid / BR::kCc;
+    const int cp2 = 2 * (tid & (BR::kCc / 2 - 1)), ot = tid / (BR::kCc / 2);
     const int q = lane >> 4, cl = lane & 15;
 
     float pre[2][8];
@@ -1545,7 +1554,7 @@ __device__ __forceinline__ void br_tiles(BrSmem<FU>& sm, const Grid& G, int C, i
     auto rows_of = [&](int k) {
         const int slot = sm.tl_s[k];
 #pragma unroll
-        for (int b = 0; b < NB; ++b) wj[b] = sm.tab[16 * (wave + kBrWaves * b) + cl][slot];
+        for (int b = 0; b < NB; ++b) wj[b] = sm.tab[16 * (wave + BR::kWaves * b) + cl][slot];
     };
     auto load_w = [&](int s) {
 #pragma unroll
@@ -1555,11 +1564,11 @@ __device__ __forceinline__ void br_tiles(BrSmem<FU>& sm, const Grid& G, int C, i
             wl[b][s] = *reinterpret_cast<const bf16x8*>(wrow + 64);
         }
     };
-    f32x4 acc[NR][kBrCb];
+    f32x4 acc[NR][BR::kCb];
 #pragma unroll
     for (int b = 0; b < NR; ++b)
 #pragma unroll
-        for (int cb = 0; cb < kBrCb; ++cb) acc[b][cb] = f32x4{};
+        for (int cb = 0; cb < BR::kCb; ++cb) acc[b][cb] = f32x4{};
     // k step s of the tile in LDS buffer buf.  B fragments are read one channel block ahead of
     // their MFMAs; the scheduling barriers keep the compiler from hoisting every LDS read of the
     // step into registers.
@@ -1569,8 +1578,8 @@ __device__ __forceinline__ void br_tiles(BrSmem<FU>& sm, const Grid& G, int C, i
             bh[0] = sm.bhi[buf][s][0][lane];
             bl[0] = sm.blo[buf][s][0][lane];
 #pragma unroll
-            for (int cb = 0; cb < kBrCb; ++cb) {
-                if (cb + 1 < kBrCb) {
+            for (int cb = 0; cb < BR::kCb; ++cb) {
+                if (cb + 1 < BR::kCb) {
                     bh[(cb + 1) & 1] = sm.bhi[buf][s][cb + 1][lane];
                     bl[(cb + 1) & 1] = sm.blo[buf][s][cb + 1][lane];
                 }
@@ -1622,11 +1631,11 @@ __device__ __forceinline__ void br_tiles(BrSmem<FU>& sm, const Grid& G, int C, i
     for (int b = 0; b < NB; ++b) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int lr = 16 * (wave + kBrWaves * b) + 4 * q + i;
+            const int lr = 16 * (wave + BR::kWaves * b) + 4 * q + i;
             if (lr >= prow) continue;
             float* dst = gpart + (int64_t)sm.rslot[lr] * C + c0 + cl;
 #pragma unroll
-            for (int cb = 0; cb < kBrCb; ++cb)
+            for (int cb = 0; cb < BR::kCb; ++cb)
                 if (c0 + 16 * cb + cl < C) dst[16 * cb] = acc[b][cb][i];
         }
     }
@@ -1634,17 +1643,18 @@ __device__ __forceinline__ void br_tiles(BrSmem<FU>& sm, const Grid& G, int C, i
 
 // A pass's row table (this thread's entries) and G->R slots, as loaded (rows past the pass read the
 // region's last row).
-constexpr int kBrPer = kBrPass * kBrSlots / kBrThreads;
+template <class BR>
 struct BrRows {
-    int tv[kBrPer];
+    int tv[BR::kPer];
     int rs[2];
 };
 
-__device__ __forceinline__ void br_load_rows(BrRows& L, int rp, int KR, int M, int MR, int jr0,
+template <class BR>
+__device__ __forceinline__ void br_load_rows(BrRows<BR>& L, int rp, int KR, int M, int MR, int jr0,
                                              const int* __restrict__ r_pairs, const int* __restrict__ table) {
 #pragma unroll
-    for (int e0 = 0; e0 < kBrPer; ++e0) {
-        const int e = threadIdx.x + e0 * kBrThreads;
+    for (int e0 = 0; e0 < BR::kPer; ++e0) {
+        const int e = threadIdx.x + e0 * BR::kThreads;
         const int r = min(rp + e / kBrSlots, KR - 1);
         // clamped: a row table or slot list from a workspace that was not prepared for these
         // Gaussians cannot send a load or a store outside the weights or the partial rows
@@ -1652,48 +1662,56 @@ __device__ __forceinline__ void br_load_rows(BrRows& L, int rp, int KR, int M, i
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        const int r = threadIdx.x + h * kBrThreads;
-        L.rs[h] = r < kBrPass ? min(max(r_pairs[jr0 + min(rp + r, KR - 1)], 0), MR - 1) : 0;
+        const int r = threadIdx.x + h * BR::kThreads;
+        L.rs[h] = r < BR::kPass ? min(max(r_pairs[jr0 + min(rp + r, KR - 1)], 0), MR - 1) : 0;
     }
 }
 
-// One pass of phase B over rows rp .. rp + prow - 1 of the region (prow <= 384): stages the
+// One pass of phase B over rows rp .. rp + prow - 1 of the region (prow <= kPass): stages the
 // pass's row table and G->R slots (L, from br_load_rows; the first pass's are requested together with
 // the region's tile list), then runs the tile loop with this wave's block count.
-template <bool GB, bool P2, bool FU>
-__device__ __forceinline__ void br_pass(BrSmem<FU>& sm, const Grid& G, int C, int c0, int ntl, int rp,
+template <class BR, bool GB, bool P2, bool FU>
+__device__ __forceinline__ void br_pass(BrSmem<BR, FU>& sm, const Grid& G, int C, int c0, int ntl, int rp,
                                         int KR, int M, int MR, int jr0, const void* __restrict__ gF,
                                         const void* __restrict__ gF2, const int* __restrict__ r_pairs,
                                         const int* __restrict__ table, const __bf16* __restrict__ wt,
-                                        float* __restrict__ gpart, bool interior, const BrRows& L) {
+                                        float* __restrict__ gpart, bool interior, const BrRows<BR>& L) {
     const int wave = threadIdx.x >> 6;
-    const int prow = min(KR - rp, kBrPass);
+    const int prow = min(KR - rp, BR::kPass);
     const int nblk = (prow + 15) >> 4;
-    const int nb = uniform((nblk - wave + kBrWaves - 1) / kBrWaves);   // row blocks of this wave
+    const int nb = uniform((nblk - wave + BR::kWaves - 1) / BR::kWaves);   // row blocks of this wave
     __syncthreads();   // the previous pass is done with both buffers and the row tables
     {
-        constexpr int kPer = kBrPer;
+        constexpr int kPer = BR::kPer;
         const int (&tv)[kPer] = L.tv;
         const int (&rs)[2] = L.rs;
 #pragma unroll
         for (int e0 = 0; e0 < kPer; ++e0) {
-            const int e = threadIdx.x + e0 * kBrThreads;
+            const int e = threadIdx.x + e0 * BR::kThreads;
             sm.tab[e / kBrSlots][e % kBrSlots] = e / kBrSlots < prow ? tv[e0] : M;
         }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const int r = threadIdx.x + h * kBrThreads;
-            if (r < kBrPass) sm.rslot[r] = rs[h];
+            const int r = threadIdx.x + h * BR::kThreads;
+            if (r < BR::kPass) sm.rslot[r] = rs[h];
         }
     }
     __syncthreads();
-    static_assert(kBrRbMax == 3, "block-count dispatch");
+    static_assert(BR::kRbMax >= 3 && BR::kRbMax <= 5, "block-count dispatch");
     auto run = [&](auto inc) {
         constexpr bool IN = decltype(inc)::value;
-        if (nb >= 3) br_tiles<3, GB, P2, FU, IN>(sm, G, C, c0, ntl, prow, gF, gF2, wt, gpart);
-        else if (nb == 2) br_tiles<2, GB, P2, FU, IN>(sm, G, C, c0, ntl, prow, gF, gF2, wt, gpart);
-        else if (nb == 1) br_tiles<1, GB, P2, FU, IN>(sm, G, C, c0, ntl, prow, gF, gF2, wt, gpart);
-        else br_tiles<0, GB, P2, FU, IN>(sm, G, C, c0, ntl, prow, gF, gF2, wt, gpart);
+        auto tiles = [&](auto nbc) {
+            constexpr int NB = decltype(nbc)::value;
+            if constexpr (NB <= BR::kRbMax) br_tiles<BR, NB, GB, P2, FU, IN>(sm, G, C, c0, ntl, prow, gF, gF2, wt, gpart);
+        };
+        switch (nb) {
+            case 0: tiles(std::integral_constant<int, 0>{}); break;
+            case 1: tiles(std::integral_constant<int, 1>{}); break;
+            case 2: tiles(std::integral_constant<int, 2>{}); break;
+            case 3: tiles(std::integral_constant<int, 3>{}); break;
+            case 4: tiles(std::integral_constant<int, 4>{}); break;
+            default: tiles(std::integral_constant<int, 5>{}); break;
+        }
     };
     if (interior) run(std::true_type{});
     else run(std::false_type{});
@@ -1702,24 +1720,24 @@ __device__ __forceinline__ void br_pass(BrSmem<FU>& sm, const Grid& G, int C, in
 // P2: even C with rows aligned to two channels, so the gF staging loads take two channels at once.
 // FU (float32): the upstream feature gradient is the cosine loss's (cg; gF unused), formed per
 // value from the target and grid_feats.
-template <bool GB, bool P2, bool FU>
-__global__ void __launch_bounds__(kBrThreads, 1) k_bwd_region(
+template <bool GB, bool P2, bool FU, class BR = BrWide>
+__global__ void __launch_bounds__(BR::kThreads, 2) k_bwd_region(
     Grid G, Regions RG, int C, int nchunk, const void* __restrict__ gF,
     const int* __restrict__ toff, int M, const int* __restrict__ roff,
     const int* __restrict__ r_pairs, const int* __restrict__ table, int MR,
     const __bf16* __restrict__ wt, float* __restrict__ gpart, const void* __restrict__ grid_feats, CosG cg) {
     static_assert(!FU || !GB, "the fused cosine gradient takes float32 rows");
-    __shared__ BrSmem<FU> sm;
+    __shared__ BrSmem<BR, FU> sm;
     const int idx = xcd_remap(blockIdx.x, gridDim.x);
     const int Rb = uniform(idx / nchunk);   // the batch's region (its list)
     const int chunk = uniform(idx - Rb * nchunk);
     if (Rb >= RG.total * G.scenes) return;
-    const int c0 = chunk * kBrCc;
+    const int c0 = chunk * BR::kCc;
     const int jr0 = uniform(min(max(roff[Rb], 0), MR));
     const int KR = uniform(min(max(roff[Rb + 1], jr0), MR)) - jr0;
     if (KR <= 0) return;
     // the first pass's row table, requested together with the region's tile list below
-    BrRows rows;
+    BrRows<BR> rows;
     br_load_rows(rows, 0, KR, M, MR, jr0, r_pairs, table);
     const int scene = uniform(Rb / RG.total), R = Rb - scene * RG.total;   // R: the scene's region
     const int tbase = scene * scene_tiles(G);                               // its first tile in the batch
@@ -1763,15 +1781,14 @@ __global__ void __launch_bounds__(kBrThreads, 1) k_bwd_region(
     if (ntl == 0) return;   // every row stays zero: phase C reads no partial row of this region
     if constexpr (FU) {
         // (k1, k2) of every voxel of the region's tiles (0 outside the grid; those values are
-        // masked anyway); the first pass's barrier orders these stores before their reads.  Two
-        // guarded entries per thread (ntl * 64 <= 2 * kBrThreads) and the tile origins from
+        // masked anyway); the first pass's barrier orders these stores before their reads.  A fixed
+        // count of guarded entries per thread (ntl * 64 <= kBrSlots * 64) and the tile origins from
         // tl_org: a loop with a per-thread trip count here would leave values that the tile loop
         // shares with it divergent, and its buffer descriptors with them.
-        static_assert(kBrSlots * 64 <= 2 * kBrThreads, "two coefficient entries per thread");
         const float scale = cg.grad_loss[0] * cg.inv_count;   // as the loss's own backward forms it
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int e = threadIdx.x + h * kBrThreads;
+        for (int h = 0; h < kBrSlots * 64 / BR::kThreads; ++h) {
+            const int e = threadIdx.x + h * BR::kThreads;
             if (e < ntl * 64) {
                 const int* org = sm.tl_org[e >> 6];
                 const int lv = e & 63;
@@ -1794,14 +1811,14 @@ __global__ void __launch_bounds__(kBrThreads, 1) k_bwd_region(
         const int rnyz = RG.n[1] * RG.n[2];
         const int rx = R / rnyz, ry = (R - rx * rnyz) / RG.n[2], rz = R % RG.n[2];
         interior = uniform((rx + 1) * RG.cell[0] <= G.dims[0] && (ry + 1) * RG.cell[1] <= G.dims[1] &&
-                           (rz + 1) * RG.cell[2] <= G.dims[2] && c0 + kBrCc <= C) != 0;
+                           (rz + 1) * RG.cell[2] <= G.dims[2] && c0 + BR::kCc <= C) != 0;
     }
-    br_pass<GB, P2, FU>(sm, G, C, c0, ntl, 0, KR, M, MR, jr0, gF, grid_feats, r_pairs, table, wt, gpart,
+    br_pass<BR, GB, P2, FU>(sm, G, C, c0, ntl, 0, KR, M, MR, jr0, gF, grid_feats, r_pairs, table, wt, gpart,
                         interior, rows);
-    for (int rp = kBrPass; rp < KR; rp += kBrPass) {
-        BrRows more;
+    for (int rp = BR::kPass; rp < KR; rp += BR::kPass) {
+        BrRows<BR> more;
         br_load_rows(more, rp, KR, M, MR, jr0, r_pairs, table);
-        br_pass<GB, P2, FU>(sm, G, C, c0, ntl, rp, KR, M, MR, jr0, gF, grid_feats, r_pairs, table, wt, gpart,
+        br_pass<BR, GB, P2, FU>(sm, G, C, c0, ntl, rp, KR, M, MR, jr0, gF, grid_feats, r_pairs, table, wt, gpart,
                             interior, more);
     }
 }
@@ -2122,23 +2139,35 @@ hipError_t launch_backward_feats(const Grid& G, int n, int C, const float* grad_
 #undef G2V_BT
     }
     if (MR > 0 && M > 0) {
-        const int nchunk = (C + kBrCc - 1) / kBrCc;
+        // Rows of at most 64 channels: half of BrWide's columns would be padding, and the narrow shape runs two
+        // workgroups per CU (ms, wide -> narrow: 6 scenes of 300 x 64 0.313 -> 0.136, 2000 x 64 0.085 -> 0.055, 6000 x
+        // 64 0.112 -> 0.080, 9000 x 64 with wide boxes 0.413 -> 0.403, 18000 x 64 0.218 -> 0.228). Wider rows would read
+        // the weights once per 64 channels instead of 128: 18000 x 128 0.237 -> 0.295, 18000 x 1024 1.17 -> 1.74.
+        // The fused cosine gradient keeps the wide shape (the narrow one spills its second source's registers). A
+        // row's sums run over the same tiles in the same order in both shapes.
+        const bool narrow = !cos && C <= kBrNarrowMax;
+        const int cc = narrow ? BrNarrow::kCc : BrWide::kCc;
+        const int nchunk = (C + cc - 1) / cc;
         const int64_t items = (int64_t)RG.total * G.scenes * nchunk;
         const int blocks = (int)ceil_div(items, 8) * 8;
         // two-channel staging loads: even C and a grad_feats base aligned to two elements
         const bool pair = (C & 1) == 0 && ((uintptr_t)grad_feats & (fdt == kDtBF16 ? 3 : 7)) == 0;
-#define G2V_BR(GBV, P2V, FU)                                                                                  \
-    G2V_LAUNCH((k_bwd_region<GBV, P2V, FU>), dim3(blocks), dim3(kBrThreads), 0, s, G, RG, C, nchunk, grad_feats,   \
+#define G2V_BR(BR, ...)                                                                                       \
+    G2V_LAUNCH((k_bwd_region<__VA_ARGS__>), dim3(blocks), dim3(BR::kThreads), 0, s, G, RG, C, nchunk, grad_feats,   \
                tile_offsets, (int)M, (const int*)b.roff, (const int*)b.r_pairs_sorted, (const int*)b.table, (int)MR, \
                (const __bf16*)b.wt, b.gpart, grid_feats, cg)
         if (cos) {   // C % 4 == 0 and 16-byte aligned rows: the paired loads apply
-            G2V_BR(false, true, true);
+            G2V_BR(BrWide, false, true, true);
         } else if (fdt == kDtBF16) {
-            if (pair) G2V_BR(true, true, false);
-            else G2V_BR(true, false, false);
+            if (narrow && pair) G2V_BR(BrNarrow, true, true, false, BrNarrow);
+            else if (narrow) G2V_BR(BrNarrow, true, false, false, BrNarrow);
+            else if (pair) G2V_BR(BrWide, true, true, false);
+            else G2V_BR(BrWide, true, false, false);
         } else {
-            if (pair) G2V_BR(false, true, false);
-            else G2V_BR(false, false, false);
+            if (narrow && pair) G2V_BR(BrNarrow, false, true, false, BrNarrow);
+            else if (narrow) G2V_BR(BrNarrow, false, false, false, BrNarrow);
+            else if (pair) G2V_BR(BrWide, false, true, false);
+            else G2V_BR(BrWide, false, false, false);
         }
 #undef G2V_BR
     }

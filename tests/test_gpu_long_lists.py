@@ -1,7 +1,8 @@
 """Tiles with long lists (phase A's passes of 256 Gaussians on the bfloat16 matrix cores) at the edges of
 their blocks: lists around one block of 32 entries, one pass (256) and two, channel counts that give 1 to 7
 chunks (the chunk loop takes three at a time) with and without 16-byte rows, and a grid that no tile
-divides.
+divides; and phase B's two shapes (rows of up to 64 channels and wider ones) around their passes of 320 and
+384 region rows.
 
 Every Gaussian covers the whole grid, so every tile's list holds all of them.  The split leaves 2^-17 =
 7.6e-6 of each product and the float32 sums of at most 520 terms less than 520 * 2^-24 = 3.1e-5 of the sum of the
@@ -31,7 +32,7 @@ def _scene(n, C, seed):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,C", [(65, 1), (65, 32), (96, 64), (97, 97), (128, 128), (129, 161), (160, 260), (255, 200),
-                                 (256, 224), (257, 96), (300, 33), (520, 36), (33, 384), (225, 448)])
+                                 (256, 224), (257, 96), (300, 33), (520, 36), (321, 64), (320, 63), (385, 66), (33, 384), (225, 448)])
 def test_long_lists(n, C, dtype):
     from CudaGaussianVoxelizer import _C
     dev = torch.device("cuda")
