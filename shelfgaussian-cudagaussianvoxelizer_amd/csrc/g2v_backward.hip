@@ -22,6 +22,7 @@
 //                    partial rows.
 // Without features, k_bwd_density walks each Gaussian's box with one wave.
 #include "g2v_internal.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace g2v {
@@ -1996,17 +1997,27 @@ static FeatBufs carve_feats(void* ws, const Grid& G, int n, int C, int64_t M, in
     b.fsp = c.take<__bf16>((int64_t)(n + 1) * feature_chunks(C) * 2 * kBtKc);
     b.partials = c.take<float>(m * kNumGrads);
     b.wt = c.take<__bf16>((m + 1) * kWtRow);   // row M is zero (rows of absent pairs read it)
-    const int64_t ms = lists_fit(G, n) ? 1 : mr;   // what only the sorted build holds
-    b.r_cells = c.take<int>(ms);
-    b.r_pairs = c.take<int>(ms);
-    b.r_gauss = c.take<int>(ms);
-    b.r_cells_sorted = c.take<int>(ms);
     b.r_pairs_sorted = c.take<int>(mr);
-    b.r_gids = c.take<int>(ms);
     b.table = c.take<int>(mr * kBrSlots);
     const int nreg = RG.total * G.scenes;   // regions of the batch
     b.roff = c.take<int>(nreg + 1);
-    b.sort_ws = c.take<char>(lists_fit(G, n) ? lists_workspace(G, n) : sort_workspace(MR, nreg));
+    // one area for either build, so that no size falls where the build changes with n or MR
+    auto sort_area = [&](void* p) {
+        Carver k(p, (size_t)-1);
+        b.r_cells = k.take<int>(mr);
+        b.r_pairs = k.take<int>(mr);
+        b.r_gauss = k.take<int>(mr);
+        b.r_cells_sorted = k.take<int>(mr);
+        b.r_gids = k.take<int>(mr);
+        b.sort_ws = k.take<char>(sort_workspace(MR, nreg));
+        return k.off;
+    };
+    void* area = c.take<char>(std::max(sort_area(nullptr), lists_workspace(G, n)));
+    sort_area(area);
+    if (lists_fit(G, n)) {
+        b.r_cells = b.r_pairs = b.r_gauss = b.r_cells_sorted = b.r_gids = nullptr;
+        b.sort_ws = area;
+    }
     b.gpart = c.take<float>(mr * (C > 0 ? C : 1));
     {   // long-tile list of phase A: a count, then at most min(T, M) tiles
         const int64_t T = (int64_t)scene_tiles(G) * G.scenes;

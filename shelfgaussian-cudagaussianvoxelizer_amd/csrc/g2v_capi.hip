@@ -5,6 +5,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 #include <string.h>
+#include <algorithm>
 
 #include "../../include/g2v.h"
 #include "g2v_internal.h"
@@ -79,13 +80,24 @@ SplatBufs carve_splat(void* ws, int n, int64_t M, const Grid& G, int feat_dim = 
     const int T = num_tiles(G);
     Carver c(ws, (size_t)-1);
     SplatBufs b;
-    const bool lists = lists_fit(G, n);   // the lists come from the boxes: no keys, values or sort buffers
-    b.keys = G.scenes > 1 && !lists ? c.take<int>(m) : nullptr;
-    b.gauss_ids = c.take<int>(lists ? 1 : m);
+    const bool lists = lists_fit(G, n);
     b.sorted_tiles = c.take<int>(m);
     b.sorted_gauss = c.take<int>(m);
     b.tile_offsets = c.take<int>(T + 1);
-    b.sort_ws = c.take<char>(lists ? lists_workspace(G, n) : sort_workspace(M, T));
+    // one area for either build, so that no size falls where the build changes with n or M
+    auto sort_area = [&](void* p) {
+        Carver k(p, (size_t)-1);
+        b.keys = G.scenes > 1 ? k.take<int>(m) : nullptr;
+        b.gauss_ids = k.take<int>(m);
+        b.sort_ws = k.take<char>(sort_workspace(M, T));
+        return k.off;
+    };
+    void* area = c.take<char>(std::max(sort_area(nullptr), lists_workspace(G, n)));
+    sort_area(area);
+    if (lists) {   // the lists come from the boxes
+        b.keys = b.gauss_ids = nullptr;
+        b.sort_ws = area;
+    }
     b.fpk = feat_dim > 0 && with_packed ? c.take<uint32_t>((int64_t)(n + 1) * packed_channels(feat_dim)) : nullptr;
     b.tl = feat_dim > 0 ? c.take<int>(long_list_ints(M, T, feat_dim)) : nullptr;
     b.drec = with_records ? c.take<DenParams>(n > 0 ? n : 1) : nullptr;

@@ -10,6 +10,7 @@
 //                    (replaces cub::DeviceRunLengthEncode + scan, reference .cu:1708-1772)
 //   k_rle_*          unique tiles / run lengths / run offsets / number of runs
 #include "g2v_internal.h"
+#include <algorithm>
 
 namespace g2v {
 
@@ -810,15 +811,24 @@ static int scene_gaussians(const Grid& G, int n) { return G.scenes > 1 ? G.scene
 constexpr int64_t kMaxWalk = 32768;
 constexpr int64_t kMaxRowBytes = int64_t(64) << 20;
 
+// Most Gaussians per scene that row lists take on this grid (0: none).
+static int row_lists_max(const Grid& G) {
+    const Regions RG = make_regions(G);
+    if (RG.n[1] > 1 << kRowYBits || RG.n[2] > 1 << kRowZBits || RG.n[0] > 65535 || G.scenes > 65535) return 0;
+    const int64_t words = kMaxWalk / ((int64_t)RG.n[1] * RG.n[2] * G.scenes);
+    const int64_t segs = kMaxRowBytes / ((int64_t)RG.n[0] * G.scenes * kSegN * (int64_t)sizeof(int2));
+    const int64_t most = std::min({(int64_t)kMaxWords * 64, words * 64, segs * kSegN});
+    return most > kDirectN ? (int)most : 0;
+}
+
+// Most Gaussians per scene that the direct walk takes on this grid.
+static int direct_max(const Grid& G) {
+    return (int)std::min((int64_t)kDirectN, kMaxWalk / ((int64_t)make_regions(G).total * G.scenes) * 64);
+}
+
 bool lists_fit(const Grid& G, int n) {
     const int ns = scene_gaussians(G, n);
-    if (ns <= 0 || ns > kMaxWords * 64) return false;
-    const Regions RG = make_regions(G);
-    const int64_t visits = ceil_div(ns, 64);
-    if (ns <= kDirectN) return (int64_t)RG.total * G.scenes * visits <= kMaxWalk;
-    return (int64_t)RG.n[1] * RG.n[2] * G.scenes * visits <= kMaxWalk && RG.n[1] <= 1 << kRowYBits &&
-           RG.n[2] <= 1 << kRowZBits && RG.n[0] <= 65535 && G.scenes <= 65535 &&
-           (int64_t)RG.n[0] * G.scenes * ceil_div(ns, kSegN) * kSegN * (int64_t)sizeof(int2) <= kMaxRowBytes;
+    return ns > 0 && ns <= (ns <= kDirectN ? direct_max(G) : row_lists_max(G));
 }
 
 struct ListBufs {
@@ -832,9 +842,9 @@ struct ListBufs {
     size_t bytes;
 };
 
-static ListBufs carve_lists(void* ws, const Grid& G, int n) {
+// ns: Gaussians per scene.
+static ListBufs carve_lists(void* ws, const Grid& G, int ns) {
     const Regions RG = make_regions(G);
-    const int ns = scene_gaussians(G, n);
     const int64_t T = (int64_t)scene_tiles(G) * G.scenes, R = (int64_t)RG.total * G.scenes;
     const int64_t segs = ns > kDirectN ? (int64_t)RG.n[0] * G.scenes * ceil_div(ns, kSegN) : 0;
     Carver c(ws, (size_t)-1);
@@ -850,7 +860,12 @@ static ListBufs carve_lists(void* ws, const Grid& G, int n) {
     return b;
 }
 
-size_t lists_workspace(const Grid& G, int n) { return carve_lists(nullptr, G, n).bytes; }
+// The most that n or fewer Gaussians take, so that a workspace sized for a bound serves every smaller call.
+size_t lists_workspace(const Grid& G, int n) {
+    const int ns = scene_gaussians(G, n), rows = std::min(ns, row_lists_max(G));
+    if (rows > kDirectN) return carve_lists(nullptr, G, rows).bytes;
+    return direct_max(G) > 0 ? carve_lists(nullptr, G, std::min(ns, kDirectN)).bytes : 0;
+}
 
 // Workgroup (segment, x row of regions, scene): the segment's Gaussians whose box reaches the row, in order.
 __global__ void __launch_bounds__(256) k_row_lists(Regions RG, int ns, int nseg, const int* __restrict__ lb,
@@ -1259,7 +1274,7 @@ hipError_t launch_tile_lists(const Grid& G, int n, const int* lb, const int* ub,
                              hipStream_t s) {
     if (drec && (!means || !opacity || !cov_inv)) return hipErrorInvalidValue;
     const Regions RG = make_regions(G);
-    const ListBufs b = carve_lists(ws, G, n);
+    const ListBufs b = carve_lists(ws, G, scene_gaussians(G, n));
     const FillJob f{tile_ids || drec ? n : 0, g2t_offsets, tile_ids, means, opacity, cov_inv, drec};
     bool own = false;
     const hipError_t e = list_offsets(G, RG, n, lb, ub, b, f, toff, nullptr, nullptr, 0, own, s);
@@ -1279,7 +1294,7 @@ hipError_t launch_region_lists(const Grid& G, int n, const int* lb, const int* u
                                int64_t MR, int* roff, int* r_pairs, int* table, int* wt_zero, int wt_zero_ints,
                                void* ws, hipStream_t s) {
     const Regions RG = make_regions(G);
-    const ListBufs b = carve_lists(ws, G, n);
+    const ListBufs b = carve_lists(ws, G, scene_gaussians(G, n));
     bool own = false;
     const hipError_t e = list_offsets(G, RG, n, lb, ub, b, FillJob{}, b.toff, roff, wt_zero, wt_zero_ints, own, s);
     if (e != hipSuccess) return e;

@@ -232,3 +232,32 @@ def test_float_quotient_of_small_integers_is_exact():
     for aa, bb in cases:
         got = (aa.astype(np.float32) / bb.astype(np.float32)).astype(np.int64)
         assert np.array_equal(got, aa // bb)
+
+
+@pytest.mark.parametrize("dims,scenes", [((200, 200, 16), 1), ((50, 50, 8), 1), ((16, 16, 8), 1), ((200, 200, 16), 6),
+                                         ((33, 30, 70), 2)])
+def test_workspace_sizes_grow_with_their_arguments(dims, scenes):
+    """A workspace sized for a bound of the Gaussians and pairs serves every smaller call, on both sides of the
+    counts where the lists' build changes."""
+    L = _lib()
+    lib = L.load()
+    vs, vr = L.floats([0.4] * 3), L.floats([0.0] * 3 + [0.4 * d + 0.1 for d in dims])
+    ns = [0, 1, 300, 3328, 3329, 4096, 4097, 9000, 30000, 80000, 83000, 84000, 120000, 262144, 262145, 600000]
+    pairs = [0, 1, 300, 10_000, 300_000, 3_000_000]
+
+    def sizes(n, M, MR):
+        if scenes > 1:
+            return {"splat": lib.g2v_batch_forward_splat_workspace(scenes, n, 8, M, vs, vr),
+                    "backward": lib.g2v_batch_backward_workspace(scenes, n, 8, M, MR, vs, vr)}
+        return {"splat": lib.g2v_forward_splat_workspace(n, 8, M, vs, vr),
+                "backward": lib.g2v_backward_workspace(n, 8, M, MR, vs, vr), "t2g": lib.g2v_t2g_workspace(n, M, vs, vr)}
+
+    grid = [[[sizes(n, M, MR) for MR in (M // 10, M)] for M in pairs] for n in ns]
+    for i in range(len(ns)):
+        for j in range(len(pairs)):
+            for k in range(2):
+                for what, v in grid[i][j][k].items():
+                    assert v > 0
+                    for di, dj, dk in ((1, 0, 0), (0, 1, 0), (0, 0, 1)):
+                        if i + di < len(ns) and j + dj < len(pairs) and k + dk < 2:
+                            assert grid[i + di][j + dj][k + dk][what] >= v, (what, ns[i], pairs[j], di, dj, dk)
