@@ -2014,7 +2014,7 @@ static FeatBufs carve_feats(void* ws, const Grid& G, int n, int C, int64_t M, in
     };
     void* area = c.take<char>(std::max(sort_area(nullptr), lists_workspace(G, n)));
     sort_area(area);
-    if (lists_fit(G, n)) {
+    if (region_lists_fit(G, n, M, MR)) {
         b.r_cells = b.r_pairs = b.r_gauss = b.r_cells_sorted = b.r_gids = nullptr;
         b.sort_ws = area;
     }
@@ -2054,7 +2054,7 @@ hipError_t launch_backward_prepare(const Grid& G, int n, int C, const void* feat
     // Region -> Gaussian CSR (pairs carry their G->R slot so partial rows land Gaussian-major) and
     // the row table of phase B
     const int nreg = RG.total * G.scenes;   // regions of the batch: scene b's region r is b R + r
-    const bool lists = lists_fit(G, n);   // built from the boxes; the pairs' buffers are not there
+    const bool lists = region_lists_fit(G, n, M, MR);   // built from the boxes; the pairs' buffers are not there
     if (lists && MR > 0 && M > 0)
         return launch_region_lists(G, n, lb, ub, pb.g2r_offsets, M, MR, b.roff, b.r_pairs_sorted, b.table,
                                    reinterpret_cast<int*>(b.wt + M * kWtRow), kWtRow / 2, b.sort_ws, s);

@@ -80,7 +80,7 @@ SplatBufs carve_splat(void* ws, int n, int64_t M, const Grid& G, int feat_dim = 
     const int T = num_tiles(G);
     Carver c(ws, (size_t)-1);
     SplatBufs b;
-    const bool lists = lists_fit(G, n);
+    const bool lists = tile_lists_fit(G, n, M);
     b.sorted_tiles = c.take<int>(m);
     b.sorted_gauss = c.take<int>(m);
     b.tile_offsets = c.take<int>(T + 1);
@@ -105,7 +105,7 @@ SplatBufs carve_splat(void* ws, int n, int64_t M, const Grid& G, int feat_dim = 
     return b;
 }
 
-// The Tile->Gaussian CSR: built from the boxes (lists_fit), or G->T gauss ids, stable sort by tile, tile
+// The Tile->Gaussian CSR: built from the boxes (tile_lists_fit), or G->T gauss ids, stable sort by tile, tile
 // offsets.  A batch sorts by
 // the batch's tile ids (b.keys, written beside the scene-local g2t_tile_ids_out).  With b.drec, the
 // G->T fill also packs the Gaussians' records (from means, opacity and cov_inv).
@@ -114,7 +114,7 @@ int build_t2g(const Grid& G, int n, const int* lb, const int* ub, const int* g2t
               hipStream_t s, const float* means = nullptr, const float* opacity = nullptr,
               const float* cov_inv = nullptr) {
     const int T = num_tiles(G);
-    if (M > 0 && lists_fit(G, n)) {
+    if (M > 0 && tile_lists_fit(G, n, M)) {
         G2V_HIP(launch_tile_lists(G, n, lb, ub, g2t_offsets, M, g2t_tile_ids_out, means, opacity, cov_inv, b.drec,
                                   b.sorted_tiles, b.sorted_gauss, b.tile_offsets, b.sort_ws, s));
         return G2V_OK;

@@ -11,6 +11,7 @@
 //   k_rle_*          unique tiles / run lengths / run offsets / number of runs
 #include "g2v_internal.h"
 #include <algorithm>
+#include <math.h>
 
 namespace g2v {
 
@@ -683,6 +684,12 @@ static void sort_plan(int num_tiles, int& passes, int& dbits) {
     dbits = passes ? (bits + passes - 1) / passes : 0;
 }
 
+static int sort_passes(int num_keys) {
+    int passes, dbits;
+    sort_plan(num_keys, passes, dbits);
+    return passes;
+}
+
 // Carves the sort workspace; with a null base it only measures it.
 struct SortBufs {
     int* pk;
@@ -802,10 +809,10 @@ constexpr int kRowYBits = 10, kRowZBits = 6;   // region ranges of a row list's 
 static int scene_gaussians(const Grid& G, int n) { return G.scenes > 1 ? G.scene_n : n; }
 
 // The region walks visit a region's share of the Gaussians 64 at a time; the path is taken while the
-// visits of all regions (of a row's, with row lists) stay below kMaxWalk and the row lists below
-// kMaxRowBytes.  Beyond (very many Gaussians or scenes, many regions along y and z), sorting the pairs, whose
-// cost follows their number alone, is the better way.  Kernel time of a density-only step on 200 x 200 x
-// 16 voxels, sorted -> listed: 10,000 Gaussians (3,925 visits) 0.123 -> 0.094 ms, 30,000 0.152 -> 0.128, 60,000
+// visits (64-Gaussian word by region) of all regions (of a row's, with row lists) stay below kMaxWalk and the
+// row lists below kMaxRowBytes.  Beyond (very many Gaussians or scenes, many regions along y and z), sorting the
+// pairs, whose cost follows their number alone, is the better way.  Kernel time of a density-only step on 200 x
+// 200 x 16 voxels, sorted -> listed: 10,000 Gaussians (3,925 visits) 0.123 -> 0.094 ms, 30,000 0.152 -> 0.128, 60,000
 // (23,450) 0.198 -> 0.193, 90,000 (35,175) 0.239 -> 0.247, 200,000 0.402 -> 0.440; 1.5 x larger Gaussians 60,000
 // 0.413 -> 0.371.  6 scenes of 300 (18,750 visits) gain, 24 scenes (75,000) lose 4 %.
 constexpr int64_t kMaxWalk = 32768;
@@ -826,9 +833,59 @@ static int direct_max(const Grid& G) {
     return (int)std::min((int64_t)kDirectN, kMaxWalk / ((int64_t)make_regions(G).total * G.scenes) * 64);
 }
 
-bool lists_fit(const Grid& G, int n) {
+static bool walk_fits(const Grid& G, int n) {
     const int ns = scene_gaussians(G, n);
     return ns > 0 && ns <= (ns <= kDirectN ? direct_max(G) : row_lists_max(G));
+}
+
+// A region's rows are one workgroup's chain, 0.010 (its Gaussians next to each other in memory) to 0.018 us a
+// row and 0.01 us a word over both launches, and workgroups beyond the chip's 256 CUs take turns; the sort spreads
+// its pairs over the chip whatever their regions: about 26 us a pass of digits and 10 us a million pairs.  So
+// the lists are built from the boxes while the mean region's rows and words stay below the sort's cost in rows.
+// us, sorted / listed (count, row lists and fill), density forward: 16 x 16 x 8 voxels (4 regions, one pass), 2,000
+// Gaussians (2,000 rows) 43 / 31, 4,096 41 / 50, 8,000 47 / 100, 40,000 48 / 289; 50 x 50 x 8 (49, two passes), 12,000
+// (2,227 rows) 73 / 60, 30,000 (5,550) 79 / 116, 200,000 (16,428) 106 / 370; 100 x 100 x 16 (169), 60,000 (1,489 and, larger
+// Gaussians, 3,459 rows) 82 / 58 and 128 / 97, 120,000 (2,972) 94 / 99.  Regions in the feature backward: 50 x 50 x 8 (one
+// pass), 8,000 Gaussians (1,485 rows) 57 / 53, 12,000 (2,227) 65 / 70, 20,000 (3,703) 72 / 102.
+// The mean is all that the host knows: where most Gaussians crowd into few regions the lists can lose (four fifths of
+// them in a 25th of 200 x 200 x 16 voxels: 6,000 58 / 36, 18,000 87 / 100, 60,000 141 / 286 us).
+static bool rows_fit(const Grid& G, int n, int64_t M, double rows, int passes) {
+    const int ns = scene_gaussians(G, n);
+    const Regions RG = make_regions(G);
+    const double R = (double)RG.total * G.scenes;
+    const double turns = R > 256.0 ? R / 256.0 : 1.0;
+    const double sort_rows = 400.0 + 1300.0 * passes + (double)M / 2000.0 + (ns <= kDirectN ? 700.0 : 0.0);
+    return (rows / R + (double)ceil_div(ns, 64)) * turns <= sort_rows;
+}
+
+// (region, Gaussian) pairs that M (tile, Gaussian) pairs make: boxes of the mean number of tiles, as close to a
+// cube as the grid's axes let them (within 10 % of the counts over grids of 50 to 200 voxels).
+static double mean_region_rows(const Grid& G, int n, int64_t M) {
+    const double g = (double)(M < n ? M : n);   // a Gaussian outside the grid has no pair
+    if (g <= 0) return 0.0;
+    const Regions RG = make_regions(G);
+    int ax[3] = {0, 1, 2};   // the shortest axis first: it cuts the box off
+    for (int i = 0; i < 2; ++i)
+        for (int j = i + 1; j < 3; ++j)
+            if (G.tiles[ax[j]] < G.tiles[ax[i]]) { const int t = ax[i]; ax[i] = ax[j]; ax[j] = t; }
+    double left = (double)M / g, cells = 1.0;
+    for (int i = 0; i < 3; ++i) {
+        const int a = ax[i];
+        double side = pow(left, 1.0 / (3 - i));
+        side = side < 1.0 ? 1.0 : side > G.tiles[a] ? (double)G.tiles[a] : side;
+        left /= side;
+        const double c = (side - 1.0) * kTile / RG.cell[a] + 1.0;
+        cells *= c > RG.n[a] ? (double)RG.n[a] : c;
+    }
+    return g * cells;
+}
+
+bool tile_lists_fit(const Grid& G, int n, int64_t M) {
+    return walk_fits(G, n) && rows_fit(G, n, M, mean_region_rows(G, n, M), sort_passes(scene_tiles(G) * G.scenes));
+}
+
+bool region_lists_fit(const Grid& G, int n, int64_t M, int64_t MR) {
+    return walk_fits(G, n) && rows_fit(G, n, M, (double)MR, sort_passes(make_regions(G).total * G.scenes));
 }
 
 struct ListBufs {

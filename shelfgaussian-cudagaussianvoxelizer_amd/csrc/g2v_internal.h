@@ -101,9 +101,10 @@ hipError_t launch_tile_offsets(const int* sorted_keys, int64_t M, int T, int* ti
 hipError_t launch_rle(const int* tile_offsets, int T, int* unique_tiles, int* counts,
                       int* runs_offsets, int* num_runs, void* ws, hipStream_t s);
 
-// Tile and region lists straight from the boxes, without a sort (see k_region_lists).  lists_fit: whether
-// this problem takes that path (else the G->T or G->R pairs are sorted).
-bool lists_fit(const Grid& G, int n);
+// Tile and region lists straight from the boxes, without a sort (see k_region_lists).  The _fit rules: whether
+// the tiles' (M pairs) or the regions' (MR pairs) lists take that path (else the G->T or G->R pairs are sorted).
+bool tile_lists_fit(const Grid& G, int n, int64_t M);
+bool region_lists_fit(const Grid& G, int n, int64_t M, int64_t MR);
 size_t lists_workspace(const Grid& G, int n);
 // The Tile->Gaussian CSR of M pairs: tile offsets, Gaussians (and tiles, when not null) in tile order.  The
 // launch also fills tile_ids (when not null) and drec as launch_fill_g2t does.

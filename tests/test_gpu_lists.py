@@ -55,3 +55,56 @@ def test_lists(name):
     ref = O.backward_f64(gD.numpy(), gF.numpy(), m.numpy(), o.numpy(), c.numpy(), f.numpy(), b["lb"], b["ub"], vs, vrn,
                          density=out[0].cpu().numpy(), grid_feats=out[5].cpu().numpy())
     assert O.rel_err(res[3].cpu().numpy(), ref[3]) < 1e-4
+
+
+# Few regions and many Gaussians: a region's rows are one workgroup's chain, so beyond a number of rows the pairs are
+# sorted, the tiles' (T->G) and the regions' (feature backward) each by its own count.  On either side of both switches:
+#        n, voxels, variances, tiles sorted, regions sorted
+ROUTES = {
+    "four_regions_2000": (2000, (16, 16, 8), (0.1, 0.6), False, False),
+    "four_regions_8000": (8000, (16, 16, 8), (0.1, 0.6), True, True),
+    "direct_4096_wide": (4096, (16, 16, 8), (0.5, 2.5), True, True),
+    "regions_only_7500": (7500, (40, 40, 16), (0.5, 2.5), False, True),
+    "row_lists_5000": (5000, (40, 40, 16), (0.1, 0.6), False, False),
+}
+
+
+@pytest.mark.parametrize("name", list(ROUTES))
+def test_list_routes(name):
+    from CudaGaussianVoxelizer import _C, _lib
+    from oracle import g2v_oracle_c as OC
+    n, dims, var, tiles_sorted, regions_sorted = ROUTES[name]
+    dev = torch.device("cuda")
+    vr = (0.0, 0.0, 0.0) + tuple(0.4 * d + 0.1 for d in dims)
+    w = W.Workload(name, n, 4, voxel_range=vr, var_range=var)
+    m, o, c, f = W.generate(w, seed=n)
+    vs, vrn = np.array(w.voxel_size, np.float32), np.array(vr, np.float32)
+    b = O.gaussian_boxes(m.numpy(), c.numpy(), vs, vrn)
+    off, tid, gid, toff, sg = OC.csr(b["tile_lo"], b["tile_hi"], b["tiles"])
+    print(f"[routes] {name} n={n} {dims} pairs={len(tid)}", flush=True)
+
+    def kernels(call):
+        _lib.profile_reset()
+        _lib.profile_enable(True)
+        try:
+            out = call()
+            torch.cuda.synchronize()
+            return out, " ".join(_lib.profile_report())
+        finally:
+            _lib.profile_enable(False)
+            _lib.profile_reset()
+
+    out, ran = kernels(lambda: _C.gaussian_voxelizer_forward(m.to(dev), o.to(dev), c.to(dev), w.voxel_size, vr, f.to(dev)))
+    assert ("k_fill_g2t" in ran) == ("k_radix_scatter" in ran) == tiles_sorted, ran
+    g = torch.Generator().manual_seed(1)
+    gD, gF = torch.randn(*dims, generator=g), torch.randn(*dims, 4, generator=g)
+    res, ran = kernels(lambda: _C.gaussian_voxelizer_backward(
+        gD.to(dev), gF.to(dev), m.to(dev), o.to(dev), out[1], w.voxel_size, vr, out[2], out[3], out[4], out[6], out[7],
+        out[0], out[5], f.to(dev)))
+    assert ("k_fill_cells" in ran) == regions_sorted, ran
+    Ainv = np.linalg.inv(c.numpy().reshape(-1, 3, 3).astype(np.float64)).reshape(-1, 9)
+    D, F = OC.forward(m.numpy(), o.numpy(), Ainv, b["lb"], b["ub"], vs, vrn, toff, sg, f.numpy(), b["dims"])
+    assert O.rel_err(out[0].cpu().numpy(), D) < 1e-4 and O.rel_err(out[5].cpu().numpy(), F) < 1e-4
+    ref = OC.backward(m.numpy(), o.numpy(), Ainv, b["lb"], b["ub"], vs, vrn, off, tid, f.numpy(), out[0].cpu().numpy(),
+                      out[5].cpu().numpy(), gD.numpy(), gF.numpy())
+    assert O.rel_err(res[3].cpu().numpy(), ref[3]) < 1e-4
