@@ -87,7 +87,8 @@ size_t g2v_forward_packed_bytes(int n, int feat_dim);
 int g2v_forward_pack_features(int n, int feat_dim, const void* features, int feat_dtype, void* packed,
                               size_t packed_bytes, void* stream);
 
-/* g2v_forward_splat: G->T fill, radix sort into the Tile->Gaussian CSR, per-tile splat of the
+/* g2v_forward_splat: G->T fill, Tile->Gaussian CSR (ascending lists, built from the boxes or by a radix
+ * sort of the pairs, whichever is cheaper for the sizes: the same CSR), per-tile splat of the
  * density and, when feat_dim > 0, of the density-weighted feature average (reference
  * .cu:1634-1904).  density (X,Y,Z) and grid_feats (X,Y,Z,feat_dim) are written completely;
  * features and packed_features may be NULL when feat_dim == 0; otherwise packed_features holds
@@ -126,9 +127,10 @@ int g2v_backward_plan(int n, int feat_dim, const float voxel_size[3], const floa
  * multiplied as it is, with float32 accumulation).  grad_feats/grid_feats/features may be NULL when
  * feat_dim == 0.  plan_workspace is the one given to g2v_backward_plan.  t2g_tiles, t2g_gauss
  * and t2g_offsets may carry the Tile->Gaussian CSR written by g2v_forward_splat for the same
- * Gaussians (all three non-NULL); with NULL it is rebuilt from g2t_offsets/g2t_tile_ids, as the
- * reference's backward signature provides only those.  Asynchronous; atomic-free and
- * deterministic. */
+ * Gaussians (all three non-NULL); with NULL it is rebuilt, as the reference's backward signature
+ * provides only g2t_offsets/g2t_tile_ids.  g2t_tile_ids must be those of the boxes, as
+ * g2v_forward_splat writes them: the rebuild reads the boxes or the ids, whichever is cheaper for the
+ * sizes.  Asynchronous; atomic-free and deterministic. */
 size_t g2v_backward_workspace(int n, int feat_dim, long long num_pairs, long long num_region_pairs,
                               const float voxel_size[3], const float voxel_range[6]);
 int g2v_backward(int n, int feat_dim, const float* grad_density, const void* grad_feats,
@@ -197,8 +199,8 @@ int g2v_backward_cosine(int n, int feat_dim, const float* grad_density, const fl
                         void* stream);
 
 /* ---- Tile->Gaussian CSR (inspection) -------------------------------------------------------
- * The internal Tile->Gaussian CSR of the forward, for parity tests: the stable sort of the G->T
- * pairs by tile (sorted_tiles, sorted_gauss: M each; reference .cu:1673-1691), the list bounds of
+ * The Tile->Gaussian CSR of given G->T pairs, for parity tests: the stable sort of g2t_tile_ids
+ * by tile, which for the ids of a forward is the forward's own CSR (sorted_tiles, sorted_gauss: M each; reference .cu:1673-1691), the list bounds of
  * every tile (tile_offsets: T+1), and the run-length encoding of the sorted tiles (unique_tiles,
  * counts: T each, runs_offsets: T+1, *num_runs on the device; reference .cu:1708-1772). */
 size_t g2v_t2g_workspace(int n, long long num_pairs, const float voxel_size[3],

@@ -611,7 +611,8 @@ def _backward_batched(grad_density, grad_feats, means, opacity, features, batch)
 
 
 def build_t2g(voxel_size, voxel_range, valid_voxel_lb, valid_voxel_ub, g2t_offsets, g2t_tile_ids):
-    """The forward's internal Tile->Gaussian CSR, for inspection and parity tests.
+    """The Tile->Gaussian CSR of a forward's G->T pairs (the stable sort of g2t_tile_ids by tile), for
+    inspection and parity tests.
 
     Returns a dict: sorted_tiles (M,), sorted_gauss (M,), tile_offsets (T+1,), and the run-length
     encoding unique_tiles (U,), counts (U,), runs_offsets (U+1,), num_runs.

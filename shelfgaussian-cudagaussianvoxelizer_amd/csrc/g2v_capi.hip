@@ -65,6 +65,7 @@ struct SplatBufs {
     int* sorted_gauss;
     int* tile_offsets;
     void* sort_ws;
+    bool lists;         // the lists come from the boxes, else from the sorted tile ids
     uint32_t* fpk;      // features as packed bf16 (hi, lo) pairs, forward only
     int* tl;            // long-tile list of the forward (count, then the list), forward only
     DenParams* drec;    // packed per-Gaussian records of the forward's tile kernels
@@ -73,14 +74,14 @@ struct SplatBufs {
 
 // with_packed: room for the packed features (a caller that packs them with
 // g2v_forward_pack_features passes its own buffer instead).  with_records: the forward's packed
-// per-Gaussian records (written by the G->T fill).
+// per-Gaussian records (written by the G->T fill).  of_ids: the CSR of given tile ids, always sorted.
 SplatBufs carve_splat(void* ws, int n, int64_t M, const Grid& G, int feat_dim = 0, bool with_packed = true,
-                      bool with_records = false) {
+                      bool with_records = false, bool of_ids = false) {
     const int64_t m = M > 0 ? M : 1;
     const int T = num_tiles(G);
     Carver c(ws, (size_t)-1);
     SplatBufs b;
-    const bool lists = tile_lists_fit(G, n, M);
+    b.lists = !of_ids && tile_lists_fit(G, n, M);
     b.sorted_tiles = c.take<int>(m);
     b.sorted_gauss = c.take<int>(m);
     b.tile_offsets = c.take<int>(T + 1);
@@ -94,7 +95,7 @@ SplatBufs carve_splat(void* ws, int n, int64_t M, const Grid& G, int feat_dim = 
     };
     void* area = c.take<char>(std::max(sort_area(nullptr), lists_workspace(G, n)));
     sort_area(area);
-    if (lists) {   // the lists come from the boxes
+    if (b.lists) {
         b.keys = b.gauss_ids = nullptr;
         b.sort_ws = area;
     }
@@ -105,16 +106,15 @@ SplatBufs carve_splat(void* ws, int n, int64_t M, const Grid& G, int feat_dim = 
     return b;
 }
 
-// The Tile->Gaussian CSR: built from the boxes (tile_lists_fit), or G->T gauss ids, stable sort by tile, tile
-// offsets.  A batch sorts by
-// the batch's tile ids (b.keys, written beside the scene-local g2t_tile_ids_out).  With b.drec, the
-// G->T fill also packs the Gaussians' records (from means, opacity and cov_inv).
+// The Tile->Gaussian CSR: built from the boxes (b.lists), or G->T gauss ids, stable sort by tile, tile
+// offsets.  A batch sorts by the batch's tile ids (b.keys, written beside the scene-local g2t_tile_ids_out).  With
+// b.drec, the G->T fill also packs the Gaussians' records (from means, opacity and cov_inv).
 int build_t2g(const Grid& G, int n, const int* lb, const int* ub, const int* g2t_offsets,
               int* g2t_tile_ids_out, const int* g2t_tile_ids_in, int64_t M, const SplatBufs& b,
               hipStream_t s, const float* means = nullptr, const float* opacity = nullptr,
               const float* cov_inv = nullptr) {
     const int T = num_tiles(G);
-    if (M > 0 && tile_lists_fit(G, n, M)) {
+    if (M > 0 && b.lists) {
         G2V_HIP(launch_tile_lists(G, n, lb, ub, g2t_offsets, M, g2t_tile_ids_out, means, opacity, cov_inv, b.drec,
                                   b.sorted_tiles, b.sorted_gauss, b.tile_offsets, b.sort_ws, s));
         return G2V_OK;
@@ -696,7 +696,7 @@ int g2v_build_t2g(int n, const float voxel_size[3], const float voxel_range[6],
     Carver c(workspace, workspace_bytes);
     void* splat_ws = c.take<char>(carve_splat(nullptr, n, num_pairs, G).bytes);
     void* rle_ws = c.take<char>(0);
-    const SplatBufs b = carve_splat(splat_ws, n, num_pairs, G);
+    const SplatBufs b = carve_splat(splat_ws, n, num_pairs, G, 0, true, false, true);
     rc = build_t2g(G, n, valid_voxel_lb, valid_voxel_ub, g2t_offsets, nullptr, g2t_tile_ids,
                    num_pairs, b, s);
     if (rc != G2V_OK) return rc;

@@ -46,8 +46,10 @@ def test_lists(name):
     out = _C.gaussian_voxelizer_forward(m.to(dev), o.to(dev), c.to(dev), w.voxel_size, vr, f.to(dev))
     assert np.array_equal(out[6].cpu().numpy(), off) and np.array_equal(out[7].cpu().numpy(), tid)
     d = _C.build_t2g(list(w.voxel_size), list(vr), out[2], out[3], out[6], out[7])
-    for key in ("sorted_tiles", "sorted_gauss", "tile_offsets"):
+    csr = _C._forward(m.to(dev), o.to(dev), c.to(dev), w.voxel_size, vr, f.to(dev), keep_t2g=True)[1]["csr"]
+    for k, key in enumerate(("sorted_tiles", "sorted_gauss", "tile_offsets")):
         assert np.array_equal(d[key].cpu().numpy(), t[key]), key
+        assert np.array_equal(csr[k].cpu().numpy(), t[key]), key   # the forward's own lists
     g = torch.Generator().manual_seed(1)
     gD, gF = torch.randn(*dims, generator=g), torch.randn(*dims, 4, generator=g)
     res = _C.gaussian_voxelizer_backward(gD.to(dev), gF.to(dev), m.to(dev), o.to(dev), out[1], w.voxel_size, vr, out[2],
@@ -108,3 +110,20 @@ def test_list_routes(name):
     ref = OC.backward(m.numpy(), o.numpy(), Ainv, b["lb"], b["ub"], vs, vrn, off, tid, f.numpy(), out[0].cpu().numpy(),
                       out[5].cpu().numpy(), gD.numpy(), gF.numpy())
     assert O.rel_err(res[3].cpu().numpy(), ref[3]) < 1e-4
+
+
+@pytest.mark.parametrize("n,dims", [(600, (17, 9, 7)), (5000, (40, 40, 16)), (9000, (16, 16, 8))])
+def test_build_t2g_sorts_the_given_ids(n, dims):
+    """build_t2g is the stable sort of the ids it is given, also where they are not those of the boxes."""
+    from CudaGaussianVoxelizer import _C
+    dev = torch.device("cuda")
+    vr = (0.0, 0.0, 0.0) + tuple(0.4 * d + 0.1 for d in dims)
+    w = W.Workload("ids", n, None, voxel_range=vr, var_range=(0.1, 0.6))
+    m, o, c, _ = W.generate(w, seed=n)
+    out = _C.gaussian_voxelizer_forward(m.to(dev), o.to(dev), c.to(dev), w.voxel_size, vr)
+    T = int(np.prod([-(-d // 4) for d in dims]))
+    off, tid = out[6].cpu().numpy(), T - 1 - out[7].cpu().numpy()
+    d = _C.build_t2g(list(w.voxel_size), list(vr), out[2], out[3], out[6], torch.from_numpy(tid).to(dev))
+    t = O.t2g_csr(tid, np.repeat(np.arange(n, dtype=np.int32), np.diff(off)), T)
+    for key in ("sorted_tiles", "sorted_gauss", "tile_offsets", "unique_tiles", "counts"):
+        assert np.array_equal(d[key].cpu().numpy(), t[key]), key
