@@ -1,7 +1,8 @@
 """Tile and region lists built from the boxes, at the edges of that build: words of 64 Gaussians, the
 limit of the direct walk (4,096 Gaussians; beyond, row lists of 1,024-Gaussian segments), regions with
 more than the 2,048 rows laid out in LDS at a time, Gaussians ordered in space (every hit of a region in
-a few words) and grids whose tiles or regions are cut off.  The T->G CSR equals the stable sort of the
+a few words) and grids whose tiles or regions are cut off; and the sorted build beyond the rules' limits, alone
+and in batches.  The T->G CSR equals the stable sort of the
 G->T pairs bit for bit; the region lists and the row table show in the feature gradients (float32 sums
 with the 2^-17 split: 1e-4, as the parity tests)."""
 import numpy as np
@@ -22,7 +23,7 @@ CASES = {
     "direct_limit": (4096, (33, 30, 7), (0.05, 0.2), True),
     "row_lists": (4097, (33, 30, 7), (0.05, 0.2), False),
     "row_lists_ordered": (5000, (40, 21, 18), (0.05, 0.2), True),
-    "many_rows": (5000, (10, 11, 6), (0.3, 1.0), False),
+    "many_rows": (5000, (10, 11, 6), (0.3, 1.0), False),   # sorted: about 3,000 rows in each of four regions
 }
 
 
@@ -59,6 +60,20 @@ def test_lists(name):
     assert O.rel_err(res[3].cpu().numpy(), ref[3]) < 1e-4
 
 
+def kernels(call):
+    """The call's result and the names of the library's kernels that it launched."""
+    from CudaGaussianVoxelizer import _lib
+    _lib.profile_reset()
+    _lib.profile_enable(True)
+    try:
+        out = call()
+        torch.cuda.synchronize()
+        return out, " ".join(_lib.profile_report())
+    finally:
+        _lib.profile_enable(False)
+        _lib.profile_reset()
+
+
 # Few regions and many Gaussians: a region's rows are one workgroup's chain, so beyond a number of rows the pairs are
 # sorted, the tiles' (T->G) and the regions' (feature backward) each by its own count.  On either side of both switches:
 #        n, voxels, variances, tiles sorted, regions sorted
@@ -68,33 +83,30 @@ ROUTES = {
     "direct_4096_wide": (4096, (16, 16, 8), (0.5, 2.5), True, True),
     "regions_only_7500": (7500, (40, 40, 16), (0.5, 2.5), False, True),
     "row_lists_5000": (5000, (40, 40, 16), (0.1, 0.6), False, False),
+    # 33,125 visits of the direct walk: everything is sorted
+    "many_visits_3329": (3329, (200, 200, 16), (0.1, 0.6), True, True),
+    # 20,800 tiles: the lists' offsets are scanned, not summed by the workgroups
+    "scanned_offsets_1000": (1000, (160, 160, 52), (0.3, 1.5), False, False),
+    # regions of more than the 2,048 rows laid out at a time, in the direct walk and (all Gaussians about four
+    # regions, which the mean does not show) with row lists
+    "row_chunks_2300": (2300, (16, 16, 8), (2.0, 12.0), False, False),
+    "crowded_6000": (6000, (200, 200, 16), (0.1, 0.6), False, False, (38.0, 38.0, 1.0, 42.0, 42.0, 5.0)),
 }
 
 
 @pytest.mark.parametrize("name", list(ROUTES))
 def test_list_routes(name):
-    from CudaGaussianVoxelizer import _C, _lib
+    from CudaGaussianVoxelizer import _C
     from oracle import g2v_oracle_c as OC
-    n, dims, var, tiles_sorted, regions_sorted = ROUTES[name]
+    n, dims, var, tiles_sorted, regions_sorted, *crowd = ROUTES[name]
     dev = torch.device("cuda")
     vr = (0.0, 0.0, 0.0) + tuple(0.4 * d + 0.1 for d in dims)
-    w = W.Workload(name, n, 4, voxel_range=vr, var_range=var)
+    w = W.Workload(name, n, 4, voxel_range=vr, var_range=var, extra={"mean_box": crowd[0]} if crowd else {})
     m, o, c, f = W.generate(w, seed=n)
     vs, vrn = np.array(w.voxel_size, np.float32), np.array(vr, np.float32)
     b = O.gaussian_boxes(m.numpy(), c.numpy(), vs, vrn)
     off, tid, gid, toff, sg = OC.csr(b["tile_lo"], b["tile_hi"], b["tiles"])
     print(f"[routes] {name} n={n} {dims} pairs={len(tid)}", flush=True)
-
-    def kernels(call):
-        _lib.profile_reset()
-        _lib.profile_enable(True)
-        try:
-            out = call()
-            torch.cuda.synchronize()
-            return out, " ".join(_lib.profile_report())
-        finally:
-            _lib.profile_enable(False)
-            _lib.profile_reset()
 
     out, ran = kernels(lambda: _C.gaussian_voxelizer_forward(m.to(dev), o.to(dev), c.to(dev), w.voxel_size, vr, f.to(dev)))
     assert ("k_fill_g2t" in ran) == ("k_radix_scatter" in ran) == tiles_sorted, ran
@@ -127,3 +139,55 @@ def test_build_t2g_sorts_the_given_ids(n, dims):
     t = O.t2g_csr(tid, np.repeat(np.arange(n, dtype=np.int32), np.diff(off)), T)
     for key in ("sorted_tiles", "sorted_gauss", "tile_offsets", "unique_tiles", "counts"):
         assert np.array_equal(d[key].cpu().numpy(), t[key]), key
+
+
+# A batch's lists against those of its scenes alone, where the builds differ: the batch sorts (by the batch's tile
+# ids and regions) what each scene lists; its offsets are scanned where each scene's workgroups sum them; and row
+# lists of more than one scene.
+#        scenes, n, voxels, variances, the batch sorts
+BATCHES = {
+    "sorted_2x1700": (2, 1700, (200, 200, 16), (0.1, 0.6), True),
+    "scanned_2x300": (2, 300, (200, 200, 16), (0.5, 2.5), False),
+    "row_lists_2x4200": (2, 4200, (40, 33, 16), (0.05, 0.2), False),
+}
+
+
+@pytest.mark.parametrize("name", list(BATCHES))
+def test_batched_list_builds(name):
+    from CudaGaussianVoxelizer import _C, PyCudaGaussianVoxelizer
+    B, n, dims, var, sorts = BATCHES[name]
+    dev = torch.device("cuda")
+    vr = (0.0, 0.0, 0.0) + tuple(0.4 * d + 0.1 for d in dims)
+    w = W.Workload(name, n, 4, voxel_range=vr, var_range=var, mean_pad=0.5)
+    scenes = [[t.to(dev) for t in W.generate(w, seed=n + b)] for b in range(B)]
+    vox = PyCudaGaussianVoxelizer(voxel_size=list(w.voxel_size), voxel_range=list(vr))
+    g = torch.Generator(device=dev).manual_seed(2)
+    gD = torch.randn(B, *dims, generator=g, device=dev)
+    gF = torch.randn(B, *dims, 4, generator=g, device=dev)
+    print(f"[batches] {name} {B} x {n} {dims}", flush=True)
+
+    def step(leaves, *grads):
+        leaves = [t.detach().clone().requires_grad_() for t in leaves]
+        out = vox(*leaves)[:2]
+        torch.autograd.backward(out, grads)
+        return [t.detach() for t in out] + [t.grad for t in leaves]
+
+    batch, ran = kernels(lambda: step([torch.stack(t) for t in zip(*scenes)], gD, gF))
+    for kernel in ("k_fill_g2t", "k_fill_cells", "k_radix_scatter", "k_region_table"):
+        assert (kernel in ran) == sorts, (kernel, ran)
+    for b in range(B):
+        alone, ran = kernels(lambda: step(scenes[b], gD[b], gF[b]))
+        assert "k_radix_scatter" not in ran and "k_region_lists" in ran, ran
+        for k, (x, y) in enumerate(zip(batch, alone)):
+            assert torch.equal(x[b], y), (b, k)
+    csr = _C._forward_batched(*[torch.stack(t) for t in zip(*scenes)][:3], w.voxel_size, vr,
+                              torch.stack([s[3] for s in scenes]), keep_t2g=True)[3]["csr"]
+    T = int(np.prod([-(-d // 4) for d in dims]))
+    at = 0
+    for b in range(B):
+        one = _C._forward(*scenes[b][:3], w.voxel_size, vr, scenes[b][3], keep_t2g=True)[1]["csr"]
+        M = one[0].numel()
+        assert torch.equal(csr[0][at:at + M], one[0] + b * T) and torch.equal(csr[1][at:at + M], one[1] + b * n)
+        assert torch.equal(csr[2][b * T:(b + 1) * T + 1], one[2] + at)
+        at += M
+    assert at == csr[0].numel()
