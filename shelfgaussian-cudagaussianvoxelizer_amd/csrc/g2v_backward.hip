@@ -1367,8 +1367,11 @@ struct BrShape {
     static_assert(kPass * kBrSlots % kThreads == 0 && kPass <= 2 * kThreads && kBrSlots * 64 % kThreads == 0, "staging shape");
 };
 typedef BrShape<8, 3> BrWide;     // one workgroup per CU
-typedef BrShape<4, 5> BrNarrow;   // two workgroups per CU
+// Two workgroups per CU.  Five row blocks a wave spill 24 registers (paired float loads; odd float rows 5, odd bfloat16
+// rows 9); four spill none, but their 256-row passes cost more: 12000 x 64 0.137 -> 0.144 ms, 18000 x 64 0.225 -> 0.266.
+typedef BrShape<4, 5> BrNarrow;
 constexpr int kBrNarrowMax = 64;  // widest row that BrNarrow takes
+constexpr int64_t kBrNarrowItems = 2 * 256;   // its workgroups that run at once
 
 // FU: the upstream feature gradient is the cosine loss's (k1 target + k2 grid_feats per voxel);
 // kc holds (k1, k2) of the voxels of the region's tiles, in the order of tl_org.
@@ -1511,7 +1514,7 @@ __device__ __forceinline__ void br_tiles(BrSmem<BR, FU>& sm, const Grid& G, int 
                                          const __bf16* __restrict__ wt, float* __restrict__ gpart) {
     constexpr int NR = NB > 0 ? NB : 1;   // register arrays (unused when NB == 0)
     int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));   // hidden: what depends on it is computed here, not kept through the caller (255 -> 231 registers)
+    asm volatile("" : "+v"(tid));   // hidden: what depends on it is computed here, not kept through the caller (the wide shape: 255 -> 231 registers)
     const int lane = tid & 63, wave = tid >> 6;
     // staging: channel sc, octets so and so + 4; or (P2) channels 2 cp and 2 cp + 1, octet ot
     const int sc = tid & (BR::kCc - 1), so = tid / BR::kCc;
@@ -2151,15 +2154,21 @@ hipError_t launch_backward_feats(const Grid& G, int n, int C, const float* grad_
     }
     if (MR > 0 && M > 0) {
         // Rows of at most 64 channels: half of BrWide's columns would be padding, and the narrow shape runs two
-        // workgroups per CU (ms, wide -> narrow: 6 scenes of 300 x 64 0.313 -> 0.136, 2000 x 64 0.085 -> 0.055, 6000 x
-        // 64 0.112 -> 0.080, 9000 x 64 with wide boxes 0.413 -> 0.403, 18000 x 64 0.218 -> 0.228). Wider rows would read
-        // the weights once per 64 channels instead of 128: 18000 x 128 0.237 -> 0.295, 18000 x 1024 1.17 -> 1.74.
+        // workgroups per CU (ms, wide -> narrow: 6 scenes of 300 x 64 0.305 -> 0.134, 2000 x 64 0.085 -> 0.054, 6000 x
+        // 64 0.109 -> 0.076, 15000 x 64 0.185 -> 0.170, 24000 x 64 0.327 -> 0.294, 120000 small ones x 32 0.453 -> 0.365; in
+        // 100 x 100 x 16 12000 x 64 0.171 -> 0.151). Only where most lists (those of the inner regions, 1.15 times the
+        // mean) are too long for one of its passes and fit one of the wide shape's, and the regions are too many to run
+        // all at once, does the second pass with its restaged gF cost more: 17000 x 64 0.204 / 0.209, 18000 x 64 0.216
+        // -> 0.227, 20000 x 64 0.231 -> 0.283. Wider rows would read the weights once per 64 channels instead of 128:
+        // 18000 x 128 0.237 -> 0.295, 18000 x 1024 1.17 -> 1.74.
         // The fused cosine gradient keeps the wide shape (the narrow one spills its second source's registers). A
         // row's sums run over the same tiles in the same order in both shapes.
-        const bool narrow = !cos && C <= kBrNarrowMax;
+        const int64_t regions = (int64_t)RG.total * G.scenes, inner = MR * 23 / (20 * regions);
+        const bool one_wide_pass = regions > kBrNarrowItems && inner > BrNarrow::kPass && inner <= BrWide::kPass;
+        const bool narrow = !cos && C <= kBrNarrowMax && !one_wide_pass;
         const int cc = narrow ? BrNarrow::kCc : BrWide::kCc;
         const int nchunk = (C + cc - 1) / cc;
-        const int64_t items = (int64_t)RG.total * G.scenes * nchunk;
+        const int64_t items = regions * nchunk;
         const int blocks = (int)ceil_div(items, 8) * 8;
         // two-channel staging loads: even C and a grad_feats base aligned to two elements
         const bool pair = (C & 1) == 0 && ((uintptr_t)grad_feats & (fdt == kDtBF16 ? 3 : 7)) == 0;

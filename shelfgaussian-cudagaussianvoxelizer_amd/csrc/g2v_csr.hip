@@ -838,24 +838,24 @@ static bool walk_fits(const Grid& G, int n) {
     return ns > 0 && ns <= (ns <= kDirectN ? direct_max(G) : row_lists_max(G));
 }
 
-// A region's rows are one workgroup's chain, 0.010 (its Gaussians next to each other in memory) to 0.018 us a
-// row and 0.01 us a word over both launches, and workgroups beyond the chip's 256 CUs take turns; the sort spreads
-// its pairs over the chip whatever their regions: about 26 us a pass of digits and 10 us a million pairs.  So
-// the lists are built from the boxes while the mean region's rows and words stay below the sort's cost in rows.
-// us, sorted / listed (count, row lists and fill), density forward: 16 x 16 x 8 voxels (4 regions, one pass), 2,000
-// Gaussians (2,000 rows) 43 / 31, 4,096 41 / 50, 8,000 47 / 100, 40,000 48 / 289; 50 x 50 x 8 (49, two passes), 12,000
-// (2,227 rows) 73 / 60, 30,000 (5,550) 79 / 116, 200,000 (16,428) 106 / 370; 100 x 100 x 16 (169), 60,000 (1,489 and, larger
-// Gaussians, 3,459 rows) 82 / 58 and 128 / 97, 120,000 (2,972) 94 / 99.  Regions in the feature backward: 50 x 50 x 8 (one
-// pass), 8,000 Gaussians (1,485 rows) 57 / 53, 12,000 (2,227) 65 / 70, 20,000 (3,703) 72 / 102.
-// The mean is all that the host knows: where most Gaussians crowd into few regions the lists can lose (four fifths of
-// them in a 25th of 200 x 200 x 16 voxels: 6,000 58 / 36, 18,000 87 / 100, 60,000 141 / 286 us).
-static bool rows_fit(const Grid& G, int n, int64_t M, double rows, int passes) {
-    const int ns = scene_gaussians(G, n);
-    const Regions RG = make_regions(G);
-    const double R = (double)RG.total * G.scenes;
+// A region's rows are one workgroup's chain, 0.010 (its Gaussians next to each other in memory) to 0.020 us a
+// row and 0.01 us a word over the launches, and workgroups beyond the chip's 256 CUs take turns; the sort spreads
+// its pairs over the chip whatever their regions: about 26 us a pass of digits and 10 us a million pairs for the
+// tiles, and for the regions 9 us per 20,000 Gaussians (k_fill_cells) and 15 a million tile pairs
+// (k_region_table) beside its passes.  So the lists are built from the boxes while the mean region's rows and words
+// stay below the sort's cost in rows (sort_rows).
+// us, sorted / listed, the tiles' lists of a density forward: 16 x 16 x 8 voxels (4 regions, one pass), 2,000 Gaussians
+// (2,000 rows) 43 / 31, 4,096 41 / 50, 8,000 47 / 100, 40,000 48 / 289; 50 x 50 x 8 (49, two passes), 12,000 (2,227 rows)
+// 73 / 60, 30,000 (5,550) 79 / 116, 200,000 (16,428) 106 / 370; 100 x 100 x 16 (169), 60,000 (1,489 and, larger
+// Gaussians, 3,459 rows) 82 / 58 and 128 / 97, 120,000 (2,972) 94 / 99.  The regions' of a feature backward: 50 x 50 x 8 (one
+// pass), 8,000 Gaussians (1,485 rows) 57 / 53, 12,000 (2,227) 65 / 70, 20,000 (3,703) 72 / 102; 200 x 200 x 16 (two passes,
+// 625), 80,000 (540) 140 / 96.
+// The mean is all that the host knows: where most Gaussians crowd into few regions the lists can lose (the tiles' with
+// four fifths of the Gaussians in a 25th of 200 x 200 x 16 voxels: 6,000 58 / 36, 18,000 87 / 100, 60,000 141 / 286 us).
+static bool rows_fit(const Grid& G, int n, double rows, double sort_rows) {
+    const double R = (double)make_regions(G).total * G.scenes;
     const double turns = R > 256.0 ? R / 256.0 : 1.0;
-    const double sort_rows = 400.0 + 1300.0 * passes + (double)M / 2000.0 + (ns <= kDirectN ? 700.0 : 0.0);
-    return (rows / R + (double)ceil_div(ns, 64)) * turns <= sort_rows;
+    return (rows / R + (double)ceil_div(scene_gaussians(G, n), 64)) * turns <= sort_rows;
 }
 
 // (region, Gaussian) pairs that M (tile, Gaussian) pairs make: boxes of the mean number of tiles, as close to a
@@ -880,12 +880,17 @@ static double mean_region_rows(const Grid& G, int n, int64_t M) {
     return g * cells;
 }
 
+// The direct walk's launch of row lists less, and its boxes read in order, count as rows too.
 bool tile_lists_fit(const Grid& G, int n, int64_t M) {
-    return walk_fits(G, n) && rows_fit(G, n, M, mean_region_rows(G, n, M), sort_passes(scene_tiles(G) * G.scenes));
+    const double direct = scene_gaussians(G, n) <= kDirectN ? 700.0 : 0.0;
+    return walk_fits(G, n) &&
+           rows_fit(G, n, mean_region_rows(G, n, M), direct + 400.0 + 1300.0 * sort_passes(scene_tiles(G) * G.scenes) + M / 2000.0);
 }
 
 bool region_lists_fit(const Grid& G, int n, int64_t M, int64_t MR) {
-    return walk_fits(G, n) && rows_fit(G, n, M, (double)MR, sort_passes(make_regions(G).total * G.scenes));
+    const double direct = scene_gaussians(G, n) <= kDirectN ? 1100.0 : 0.0;
+    return walk_fits(G, n) &&
+           rows_fit(G, n, (double)MR, direct - 100.0 + 1300.0 * sort_passes(make_regions(G).total * G.scenes) + n / 45.0 + M / 1400.0);
 }
 
 struct ListBufs {

@@ -23,7 +23,7 @@ CASES = {
     "direct_limit": (4096, (33, 30, 7), (0.05, 0.2), True),
     "row_lists": (4097, (33, 30, 7), (0.05, 0.2), False),
     "row_lists_ordered": (5000, (40, 21, 18), (0.05, 0.2), True),
-    "many_rows": (5000, (10, 11, 6), (0.3, 1.0), False),   # sorted: about 3,000 rows in each of four regions
+    "many_rows": (5000, (10, 11, 6), (0.3, 1.0), False),   # sorted: 2,842 to 4,999 rows in each of four regions
 }
 
 

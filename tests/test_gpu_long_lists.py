@@ -60,3 +60,42 @@ def test_long_lists(n, C, dtype):
     print(f"[long] n={n} C={C} {dtype}: " + ", ".join(f"{k} {v:.1e}" for k, (v, _) in err.items()), flush=True)
     for k, (v, t) in err.items():
         assert v < t, (k, v, t)
+
+
+@pytest.mark.parametrize("C,dtype", [(16, torch.float32), (33, torch.float32), (64, torch.bfloat16)])
+def test_many_regions_of_long_rows(C, dtype):
+    """Rows of at most 64 channels in more regions than run at once (23 x 23), whose lists are too long for one pass of
+    phase B's narrow shape and fit one of the wide shape's: the wide shape.  A feature gradient's float32 sums run over at most 1,024 voxels of a region and 49 regions: 3e-5 of
+    the sums of magnitudes, as above."""
+    from CudaGaussianVoxelizer import _C
+    from oracle import g2v_oracle_c as OC
+    from tests import workloads as W
+    from tests.test_gpu_lists import kernels
+    dev = torch.device("cuda")
+    w = W.Workload("long_rows", 5500, C, voxel_range=(0.0, 0.0, 0.0, 73.7, 73.7, 1.7), var_range=(2.0, 12.0))
+    m, o, c, f = W.generate(w, seed=C)
+    f = f.to(dtype)
+    vs, vr = np.array(w.voxel_size, np.float32), np.array(w.voxel_range, np.float32)
+    b = O.gaussian_boxes(m.numpy(), c.numpy(), vs, vr)
+    assert b["dims"] == (184, 184, 4)
+    rows = ((b["ub"][:, :2] // 8 - b["lb"][:, :2] // 8 + 1).prod(1) * (b["nvox"] > 0)).sum()
+    assert 320 < rows * 1.15 / 23 ** 2 < 384
+    print(f"[rows] C={C} {dtype} {rows} rows", flush=True)
+    out = _C.gaussian_voxelizer_forward(m.to(dev), o.to(dev), c.to(dev), w.voxel_size, w.voxel_range, f.to(dev))
+    X, Y, Z = b["dims"]
+    g = torch.Generator().manual_seed(3)
+    gD, gF = torch.zeros(X, Y, Z), torch.randn(X, Y, Z, C, generator=g).to(dtype)
+    res, ran = kernels(lambda: _C.gaussian_voxelizer_backward(
+        gD.to(dev), gF.to(dev), m.to(dev), o.to(dev), out[1], w.voxel_size, w.voxel_range, out[2], out[3], out[4],
+        out[6], out[7], out[0], out[5], f.to(dev)))
+    assert "k_bwd_region" in ran and "BrNarrow" not in ran, ran
+    off, tid, gid, toff, sg = OC.csr(b["tile_lo"], b["tile_hi"], b["tiles"])
+    Ainv = np.linalg.inv(c.numpy().reshape(-1, 3, 3).astype(np.float64)).reshape(-1, 9)
+
+    def grad(up):
+        return OC.backward(m.numpy(), o.numpy(), Ainv, b["lb"], b["ub"], vs, vr, off, tid, f.float().numpy(),
+                           out[0].cpu().numpy(), out[5].float().cpu().numpy(), gD.numpy(), up)[3]
+
+    gF32 = gF.float().numpy()
+    err = np.linalg.norm(res[3].float().cpu().numpy() - grad(gF32)) / np.linalg.norm(grad(np.abs(gF32)))
+    assert err < (3e-5 if dtype == torch.float32 else 2.0 ** -9), err
