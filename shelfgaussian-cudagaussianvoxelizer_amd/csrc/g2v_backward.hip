@@ -252,6 +252,8 @@ constexpr int kBtPass = kBtWaves * kBtNbw * 32;        // 256 Gaussians per pass
 constexpr int kBtStages = 2;                           // F chunks resident in LDS (loaded 1 ahead)
 constexpr int kBtRows = 1024 / kBtRowBytes;            // rows of one 1 KB direct-to-LDS load
 constexpr int kBtDma = kBtPass / kBtRows / kBtWaves;   // such loads per wave per chunk of F
+constexpr int kBtFewTiles = 256;                       // tiles up to which their passes are split
+constexpr int kBtMaxParts = 16;                        // workgroups of a tile
 constexpr int kBtGRows = 64 / kBtWaves;                // voxel rows whose G a wave loads and splits
 constexpr int kWtRow = 128;                            // bf16 per pair: 64 hi then 64 lo
 
@@ -462,15 +464,18 @@ __global__ void __launch_bounds__(kBtThreads, 2) k_bwd_tile(
     const int j0 = uniform(min(max(toff[tb], 0), M));
     const int Ng = uniform(min(max(toff[tb + 1], j0), M)) - j0;
     if (Ng <= skip_le) return;   // empty, or a short list that k_bwd_tile_short takes
+    // gridDim.y workgroups take the tile's passes in turn
+    const int pbase0 = (int)blockIdx.y * kBtPass;
+    if (pbase0 >= Ng) return;
     // the first pass's list entries, requested before the voxel values are staged (raw values at
     // clamped positions; the entries past the pass are selected away where they are used)
-    const int pc0 = min(kBtPass, Ng);
+    const int pc0 = min(kBtPass, Ng - pbase0);
     int gld[kBtNbw], grow[kBtDma];   // the Gaussians of the lane's columns and of its F rows (clamped to the list)
 #pragma unroll
-    for (int j = 0; j < kBtNbw; ++j) gld[j] = sorted_gauss[j0 + min((wave_ + kBtWaves * j) * 32 + (lane_ & 31), pc0 - 1)];
+    for (int j = 0; j < kBtNbw; ++j) gld[j] = sorted_gauss[j0 + pbase0 + min((wave_ + kBtWaves * j) * 32 + (lane_ & 31), pc0 - 1)];
 #pragma unroll
     for (int i = 0; i < kBtDma; ++i)
-        grow[i] = sorted_gauss[j0 + min((wave_ + kBtWaves * i) * kBtRows + lane_ / 8, pc0 - 1)];
+        grow[i] = sorted_gauss[j0 + pbase0 + min((wave_ + kBtWaves * i) * kBtRows + lane_ / 8, pc0 - 1)];
     if (threadIdx.x < 64) {
         const bool ok = vok;
         const int64_t v = vx;
@@ -559,7 +564,7 @@ __global__ void __launch_bounds__(kBtThreads, 2) k_bwd_tile(
     const uint32_t fstride = (uint32_t)nchk * kBtRowBytes;   // bytes of one Gaussian's split row
     const char* fbase = reinterpret_cast<const char*>(fsp);
 
-    for (int pbase = 0; pbase < Ng; pbase += kBtPass) {
+    for (int pbase = pbase0; pbase < Ng; pbase += (int)gridDim.y * kBtPass) {
         const int pcount = min(kBtPass, Ng - pbase);
         // The thread's indices are hidden from the compiler at the start of a pass and again at its epilogues:
         // it would otherwise compute all that depends on them before the pass loop and spill it
@@ -1014,8 +1019,9 @@ __global__ void __launch_bounds__(kBtThreads, 2) k_bwd_tile(
         }
         }
         // the next pass's list entries
-        const int* list = sorted_gauss + j0 + pbase + kBtPass;
-        const int left = Ng - pbase - kBtPass;
+        const int next = pbase + (int)gridDim.y * kBtPass;
+        const int* list = sorted_gauss + j0 + next;
+        const int left = Ng - next;
         if (left > 0) {
 #pragma unroll
             for (int j = 0; j < kBtNbw; ++j) gld[j] = list[min((wave + kBtWaves * j) * 32 + (lane & 31), min(left, kBtPass) - 1)];
@@ -2125,6 +2131,11 @@ hipError_t launch_backward_feats(const Grid& G, int n, int C, const float* grad_
             tlist = b.tl + 1;
         }
         const int lblocks = (int)ceil_div(nlong, 8) * 8;
+        // Fewer tiles than CUs would leave most of the chip idle, and a lone workgroup per CU hides less latency: the
+        // passes of a tile go to several workgroups, two per CU in all, each of which reads t_v's rows for itself (ms,
+        // one workgroup -> several: 4000 Gaussians x 1024 channels in 16 x 16 x 8 voxels 0.623 -> 0.096, in 32 x 32 x 16,
+        // 256 tiles, 0.371 -> 0.293; the eight-wave workgroups of before took 0.531 and 0.318).
+        const int parts = nlong > 0 && nlong <= kBtFewTiles ? min(kBtMaxParts, 2 * kBtFewTiles / nlong) : 1;
         if (!cos) {
             if (fdt == kDtBF16)
                 G2V_LAUNCH(k_bwd_tile_short<true>, dim3(blocks), dim3(kBsThreads), 0, s, G, C, grad_density, grad_feats,
@@ -2136,7 +2147,7 @@ hipError_t launch_backward_feats(const Grid& G, int n, int C, const float* grad_
                            features, b.partials, b.wt, skip_le);
         }
 #define G2V_BT(V, F, FU)                                                                                      \
-    G2V_LAUNCH((k_bwd_tile<V, F, FU>), dim3(lblocks), dim3(kBtThreads), 0, s, G, n, C, nchk, grad_density,         \
+    G2V_LAUNCH((k_bwd_tile<V, F, FU>), dim3(lblocks, parts), dim3(kBtThreads), 0, s, G, n, C, nchk, grad_density,         \
                grad_feats, means, opacity, cov_inv, lb, ub, g2t_offsets, tile_offsets, sorted_gauss, (int)M, density,        \
                grid_feats, fdt, (const __bf16*)b.fsp, b.partials, b.wt, cg, skip_le, tlist, tcount)
         if (nlong == 0) {

@@ -99,3 +99,35 @@ def test_many_regions_of_long_rows(C, dtype):
     gF32 = gF.float().numpy()
     err = np.linalg.norm(res[3].float().cpu().numpy() - grad(gF32)) / np.linalg.norm(grad(np.abs(gF32)))
     assert err < (3e-5 if dtype == torch.float32 else 2.0 ** -9), err
+
+
+@pytest.mark.parametrize("n,dims,C", [(5000, (16, 16, 4), 4), (5000, (16, 16, 4), 5), (1500, (32, 32, 16), 4)])
+def test_few_tiles_of_many_passes(n, dims, C):
+    """Up to 256 tiles, the passes of phase A over a tile's list are split over workgroups: 20 passes over 16, and 6
+    over 2.  The float32 sums of each pair are the same as in one workgroup; features and geometry as above."""
+    from CudaGaussianVoxelizer import _C
+    from oracle import g2v_oracle_c as OC
+    from tests import workloads as W
+    dev = torch.device("cuda")
+    w = W.Workload("few", n, C, voxel_range=(0.0, 0.0, 0.0) + tuple(0.4 * d + 0.1 for d in dims), var_range=(8.0, 20.0))
+    m, o, c, f = W.generate(w, seed=n + C)
+    vs, vr = np.array(w.voxel_size, np.float32), np.array(w.voxel_range, np.float32)
+    b = O.gaussian_boxes(m.numpy(), c.numpy(), vs, vr)
+    assert b["dims"] == dims
+    off, tid, gid, toff, sg = OC.csr(b["tile_lo"], b["tile_hi"], b["tiles"])
+    print(f"[few] n={n} {dims} lists {np.diff(toff).min()} to {np.diff(toff).max()}", flush=True)
+    out = _C.gaussian_voxelizer_forward(m.to(dev), o.to(dev), c.to(dev), w.voxel_size, w.voxel_range, f.to(dev))
+    g = torch.Generator().manual_seed(3)
+    gD, gF = torch.randn(*dims, generator=g), torch.randn(*dims, C, generator=g)
+    res = _C.gaussian_voxelizer_backward(gD.to(dev), gF.to(dev), m.to(dev), o.to(dev), out[1], w.voxel_size,
+                                         w.voxel_range, out[2], out[3], out[4], out[6], out[7], out[0], out[5], f.to(dev))
+    Ainv = np.linalg.inv(c.numpy().reshape(-1, 3, 3).astype(np.float64)).reshape(-1, 9)
+
+    def grad(gd, up):
+        return OC.backward(m.numpy(), o.numpy(), Ainv, b["lb"], b["ub"], vs, vr, off, tid, f.numpy(),
+                           out[0].cpu().numpy(), out[5].cpu().numpy(), gd, up)
+
+    ref, mag = grad(gD.numpy(), gF.numpy()), grad(gD.numpy(), np.abs(gF.numpy()))[3]
+    assert np.linalg.norm(res[3].cpu().numpy() - ref[3]) / np.linalg.norm(mag) < 3e-5
+    for k, what in ((0, "means"), (1, "cov"), (2, "opacity")):
+        assert O.rel_err(res[k].cpu().numpy(), ref[k]) < 3e-4, what
