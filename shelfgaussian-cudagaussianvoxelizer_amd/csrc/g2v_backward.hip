@@ -314,35 +314,12 @@ __device__ __forceinline__ void wait_vm() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-
-
 // Geometry of one lane's 16 epilogue elements against its Gaussian.  The elements of a lane are
 // the 2 x 2 x 4 voxel block x = x0 + a, y = y0 + 2b, z = z0 + c of the tile (a, b < 2, c < 4), so
-// dx = centre - mu and the box test (bit masks) split by axis.
+// dx = centre - mu splits by axis.
 struct LaneGeom {
     float dx[2], dy[2], dz[4];
-    unsigned inx, iny, inz;               // bit a / b / c: the offset lies in the Gaussian's box
 };
-
-__device__ __forceinline__ void lane_geom(const Grid& G, const GaussParams& p, int x0, int y0, int z0,
-                                          LaneGeom& L) {
-#pragma clang fp contract(off)
-    L.inx = L.iny = L.inz = 0;
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-        const int x = x0 + a, y = y0 + 2 * a;
-        L.dx[a] = centre(G, 0, x) - p.mu[0];
-        L.dy[a] = centre(G, 1, y) - p.mu[1];
-        L.inx |= (x >= p.lb[0] && x <= p.ub[0]) ? (1u << a) : 0u;
-        L.iny |= (y >= p.lb[1] && y <= p.ub[1]) ? (1u << a) : 0u;
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const int z = z0 + c;
-        L.dz[c] = centre(G, 2, z) - p.mu[2];
-        L.inz |= (z >= p.lb[2] && z <= p.ub[2]) ? (1u << c) : 0u;
-    }
-}
 
 // The exponent -m/2 of a lane's element (a, b, c), split by axis and scaled by kq so that
 // e = exp2(Fxy[a][b] + Fz[c] + Gxy[a][b] dz[c]) (m = d^T A d summed in this order).
@@ -378,12 +355,6 @@ __device__ __forceinline__ void lane_exp(const SymA& A, const LaneGeom& L, LaneE
         }
 #pragma unroll
     for (int c = 0; c < 4; ++c) E.Fz[c] = kq * (A.zz * L.dz[c] * L.dz[c]);
-}
-
-__device__ __forceinline__ void lane_exp(const GaussParams& p, const LaneGeom& L, LaneExp& E) {
-    SymA A;
-    sym_a(p, A);
-    lane_exp(A, L, E);
 }
 
 __device__ __forceinline__ float lane_e(const LaneExp& E, const LaneGeom& L, int a, int b, int c) {
@@ -1065,8 +1036,8 @@ struct BsSmem {
     float xch[4][kBsMax][kNumGrads];         // moments of each wave's 16 voxels
 };
 
-// e of Gaussian p at voxel (x, y, z) with the operations of lane_geom / lane_exp / lane_e (so the
-// same value); in: the voxel lies in the Gaussian's box.
+// e of Gaussian p at voxel (x, y, z) with the operations of k_bwd_tile's offsets (geom), sym_a, lane_exp and lane_e
+// (so the same value); in: the voxel lies in the Gaussian's box.
 __device__ __forceinline__ float voxel_e(const Grid& G, const GaussParams& p, int x, int y, int z, float& dx,
                                          float& dy, float& dz, bool& in) {
 #pragma clang fp contract(off)

@@ -1292,17 +1292,26 @@ __global__ void __launch_bounds__(kListThreads) k_region_lists(Grid G, Regions R
 // Up to this many tiles of the batch, the list kernels sum the counts before their tiles themselves.
 constexpr int kOwnScanTiles = 16384;
 
-template <ListMode MODE>
-static void run_region_lists(const Grid& G, const Regions& RG, int n, const int* lb, const int* ub, const ListBufs& b,
-                             const ListOut& o, const FillJob& f, hipStream_t s) {
+static void run_region_lists(ListMode mode, const Grid& G, const Regions& RG, int n, const int* lb, const int* ub,
+                             const ListBufs& b, const ListOut& o, const FillJob& f, hipStream_t s) {
     const int ns = scene_gaussians(G, n), nseg = (int)ceil_div(ns, kSegN);
     const dim3 grid((unsigned)(RG.total * G.scenes + ceil_div(f.n, kListThreads / kFillLanes)));
-    if (ns <= kDirectN)
-        G2V_LAUNCH((k_region_lists<MODE, true>), grid, dim3(kListThreads), 0, s, G, RG, ns, nseg, lb, ub, nullptr,
-                   nullptr, o, f);
-    else
-        G2V_LAUNCH((k_region_lists<MODE, false>), grid, dim3(kListThreads), 0, s, G, RG, ns, nseg, lb, ub,
-                   (const int*)b.rowcnt, (const int2*)b.rowlist, o, f);
+    // each mode is launched by its own name (the name of its time)
+#define G2V_RL(MODE)                                                                                                 \
+    do {                                                                                                             \
+        if (ns <= kDirectN)                                                                                          \
+            G2V_LAUNCH((k_region_lists<MODE, true>), grid, dim3(kListThreads), 0, s, G, RG, ns, nseg, lb, ub, nullptr, \
+                       nullptr, o, f);                                                                               \
+        else                                                                                                         \
+            G2V_LAUNCH((k_region_lists<MODE, false>), grid, dim3(kListThreads), 0, s, G, RG, ns, nseg, lb, ub,         \
+                       (const int*)b.rowcnt, (const int2*)b.rowlist, o, f);                                          \
+    } while (0)
+    switch (mode) {
+        case kListCount: G2V_RL(kListCount); break;
+        case kListTiles: G2V_RL(kListTiles); break;
+        case kListTable: G2V_RL(kListTable); break;
+    }
+#undef G2V_RL
 }
 
 // The lengths of all lists (b.tcnt, b.rcnt) and, beyond kOwnScanTiles (own false), their offsets toff (T + 1) and,
@@ -1323,7 +1332,7 @@ static hipError_t list_offsets(const Grid& G, const Regions& RG, int n, const in
     o.first[1] = own ? nullptr : roff;
     o.zero = zero;
     o.nzero = nzero;
-    run_region_lists<kListCount>(G, RG, n, lb, ub, b, o, f, s);
+    run_region_lists(kListCount, G, RG, n, lb, ub, b, o, f, s);
     if (own) return hipGetLastError();
     // inclusive scans behind a leading zero
     return scan_i32_pair(b.tcnt, toff + 1, T, nullptr, b.scan_t, b.rcnt, roff ? roff + 1 : nullptr, roff ? R : 0, nullptr,
@@ -1348,7 +1357,7 @@ hipError_t launch_tile_lists(const Grid& G, int n, const int* lb, const int* ub,
     o.sorted_tiles = sorted_tiles;
     o.sorted_gauss = sorted_gauss;
     o.M = (int)M;
-    run_region_lists<kListTiles>(G, RG, n, lb, ub, b, o, FillJob{}, s);
+    run_region_lists(kListTiles, G, RG, n, lb, ub, b, o, FillJob{}, s);
     return hipGetLastError();
 }
 
@@ -1371,7 +1380,7 @@ hipError_t launch_region_lists(const Grid& G, int n, const int* lb, const int* u
     o.table = table;
     o.M = (int)M;
     o.MR = (int)MR;
-    run_region_lists<kListTable>(G, RG, n, lb, ub, b, o, FillJob{}, s);
+    run_region_lists(kListTable, G, RG, n, lb, ub, b, o, FillJob{}, s);
     return hipGetLastError();
 }
 
