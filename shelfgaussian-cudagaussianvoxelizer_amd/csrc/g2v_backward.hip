@@ -8,7 +8,7 @@
 //
 // With features the work is split in three phases so that every gF row is read from HBM
 // twice instead of once per overlapping Gaussian (the reference re-reads it per pair):
-//   A  k_bwd_tile    one workgroup per 4x4x4 tile: U^T = G_tile (64 x C) . F_list^T on the matrix
+//   A  k_bwd_tile    one workgroup per 4x4x4 tile (several where tiles are few): U^T = G_tile (64 x C) . F_list^T on the matrix
 //                    cores (3-term bf16 split, fp32 accumulate); t_v from U (sum_g [w>0] w u / D is
 //                    sum_c gF F); gw; ten moments of r = gw e over the pair's voxels (sum r d,
 //                    sum r d d^T, sum r with d = centre - mu), stored at the pair's G->T CSR
@@ -28,22 +28,6 @@
 namespace g2v {
 
 constexpr int kNumGrads = 10;  // mu xyz, cov xx yy zz xy xz yz, opacity
-
-__device__ __forceinline__ void accumulate_grads(float (&gr)[kNumGrads], float gw, float e, float o,
-                                                 float qx, float qy, float qz) {
-    const float gwd = gw * o * e;
-    gr[0] += gwd * qx;
-    gr[1] += gwd * qy;
-    gr[2] += gwd * qz;
-    const float h = 0.5f * gwd;
-    gr[3] += h * qx * qx;
-    gr[4] += h * qy * qy;
-    gr[5] += h * qz * qz;
-    gr[6] += h * qx * qy;
-    gr[7] += h * qx * qz;
-    gr[8] += h * qy * qz;
-    gr[9] += gw * e;
-}
 
 __device__ __forceinline__ void write_grads(const float (&gr)[kNumGrads], int g, float* grad_means,
                                             float* grad_cov, float* grad_opacity) {
@@ -1008,7 +992,7 @@ __global__ void __launch_bounds__(kBtThreads, 2) k_bwd_tile(
 // ------------------------------------------------------------------------------------------
 // Phase A for short lists (1 .. smax <= kBsMax Gaussians).  k_bwd_tile holds two tiles per CU (its LDS is
 // sized for 256-Gaussian passes), so a short list leaves those tiles' chains of loads and barriers
-// bare; here a 4-wave workgroup with 17 KB of LDS takes the tile and many run per CU.
+// bare; here a 4-wave workgroup with 15.6 KB of LDS takes the tile and four (117 registers) run per CU.
 //
 // U = G F^T on the float32 matrix cores (16x16x4), straight from the caller's rows: wave w owns the
 // 16 voxels x = x0 + w of the tile (A operand: lane l % 16 = voxel, B operand: lane l % 16 = list entry

@@ -4,6 +4,8 @@
 //                    (reference src/cuda_gaussian_voxelizer.cu:348-536, :201-220)
 //   scan_i32         device-wide scan (replaces cub::DeviceScan, reference .cu:1605-1615, :1758-1772)
 //   k_fill_g2t       row-major G->T rows (reference .cu:228-286)
+//   k_region_lists   the tiles' and regions' lists straight from the boxes (with k_row_lists beyond 4,096 Gaussians a
+//                    scene), where that is cheaper than sorting the pairs; else:
 //   radix_sort_pairs stable LSD radix sort over only ceil(log2 T) key bits
 //                    (replaces cub::DeviceRadixSort::SortPairs over 32 bits, reference .cu:1673-1691)
 //   k_tile_offsets   run boundaries of the sorted tile ids for every tile, empty ones included
@@ -784,9 +786,9 @@ hipError_t launch_tile_offsets(const int* sorted_keys, int64_t M, int T, int* ti
 // Lists from the boxes.  A tile's list is the ascending sequence of the Gaussians whose box meets it, so
 // it need not be sorted out of the G->T pairs: one workgroup per region (2 x 2 x up to 4 tiles) walks the
 // Gaussians in order, keeps those that reach the region, and one wave per tile picks its own from them by
-// ballot.  The sort moved every pair through memory twice per pass in three dependent launches per pass
-// (eight launches from the fill to the tile offsets, and as many again for the regions, whose row table
-// then searched each pair); here a count, a scan and a fill remain.
+// ballot.  The sort moves every pair through memory twice per pass in three dependent launches per pass
+// (eight launches from the fill to the tile offsets with two passes, and ten for the regions, whose row table
+// then searches each pair); here a count and a fill remain, and a scan beyond kOwnScanTiles.
 //
 // The Gaussians are walked 64 at a time, a word of hit bits each.  With more than kDirectN per scene a
 // first kernel keeps, for every x row of regions and segment of kSegN Gaussians, those whose box reaches the

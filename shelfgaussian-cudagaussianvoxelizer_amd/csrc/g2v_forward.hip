@@ -435,7 +435,7 @@ __device__ __forceinline__ void fwd_zero_tile(const Grid& G, int tile, int C, fl
 // ------------------------------------------------------------------------------------------
 // Tiles whose list holds at most smax <= kFsMax Gaussians, empty ones included.  k_fwd_feats keeps two
 // tiles per CU (its LDS holds a 256-Gaussian K chunk), so a short list leaves that tile's chain of
-// loads and barriers bare; here a 4-wave workgroup with 17 KB of LDS takes the tile and several
+// loads and barriers bare; here a 4-wave workgroup with 17 KB of LDS takes the tile and seven
 // run per CU.
 // S = W F on the float32 matrix cores (16x16x4): wave w owns the 16 voxels x = x0 + w, lane l % 16 = voxel,
 // and the lane group q = l / 16 evaluates the weights of the list entries 4 s + q, which are then the A
